@@ -553,6 +553,74 @@ bool ensure_fp4_image(fiu_dataset *d, hipStream_t s)
     return true;
 }
 
+// Room for `bytes` more of a dataset's derived tables.
+static bool room_for(fiu_dataset *d, uint64_t bytes, bool quarter)
+{
+    if (d->arena) return bytes <= d->arena->largest_free();
+    size_t free_b = 0, total_b = 0;
+    check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+    return bytes + (64ull << 20) <= (quarter ? free_b / 4 : free_b);
+}
+
+bool ensure_tuple_image(fiu_dataset *d, hipStream_t s)
+{
+    std::lock_guard<std::mutex> lk(d->prep_mu);
+    if (d->fp4x_ready) return true;
+    const uint64_t units = 12ull * (d->dev.quads[0] + d->dev.quads[1]) * d->dev.n_pad;
+    if (!room_for(d, units * 16, false)) return false;
+    d->fp4x.alloc(units);
+    check(launch_tuple_image(d->dev, d->fp4x.p, s), "fp4 image launch");
+    check(hipStreamSynchronize(s), "fp4 image sync");
+    d->fp4x_ready = true;
+    return true;
+}
+
+Fp4Image tuple_image(const fiu_dataset *d, bool all_cells)
+{
+    Fp4Image F;
+    F.base = all_cells ? d->fp4x.p : d->fp4.p;
+    F.class_off[0] = 0;
+    F.class_off[1] = (all_cells ? 12ull : 8ull) * d->dev.quads[0] * d->dev.n_pad;
+    return F;
+}
+
+bool ensure_tuple_tables(fiu_dataset *d, int m, hipStream_t s)
+{
+    if (!ensure_fp4_image(d, s)) return false;
+    const uint64_t *binom = ensure_binom(d, std::max(m, 2), s);
+    std::lock_guard<std::mutex> lk(d->prep_mu);
+    const uint64_t n = d->snps;
+    uint64_t bytes = 0;
+    for (int j = d->tup_ready + 1; j <= m; ++j) {
+        const uint64_t c = binom_sat(n, (uint64_t)j);
+        if (c >= (1ull << 40)) return false;
+        bytes += (c << j) * 4;
+    }
+    if (bytes == 0) return true;
+    if (!room_for(d, bytes, true)) return false;
+    TupleArgs A{};
+    A.F = tuple_image(d, false);
+    A.stride = 1;
+    A.fill = kTupleFill;
+    ScanParams P{};
+    P.step = 1;
+    P.binom = binom;
+    for (int j = d->tup_ready + 1; j <= m; ++j) {
+        d->tup[j].alloc(binom_sat(n, (uint64_t)j) << j);
+        if (j == 1) {
+            check(launch_tuple_singles(d->dev, d->tup[1].p, s), "singles table launch");
+        } else {
+            A.out = d->tup[j].p;
+            P.j0 = 0;
+            P.j1 = j == 2 ? ((int64_t)n + tuple_b_block(2, false) - 1) / tuple_b_block(2, false) : (int64_t)n;
+            check(launch_tuples(j, false, d->dev, P, nullptr, A, s), "count table launch");
+        }
+    }
+    check(hipStreamSynchronize(s), "count table sync");
+    d->tup_ready = m;
+    return true;
+}
+
 // The prefixes that share their first m-1 indices form a run of consecutive
 // ranks whose last index increases by one; each run is summed in closed form.
 // The (m-1)-combinations heading the runs are walked in lexicographic order
@@ -713,6 +781,9 @@ struct ChunkPlan {
 class Workspace {
   public:
     virtual ~Workspace() = default;
+    // tables of fewer SNPs' counts up to m (marginal), or the three-row fp4
+    // image (all cells), for the scans around a head; false without them
+    virtual bool tuples(fiu_dataset *, int, bool, hipStream_t) { return false; }
     // binomial table C(x, j), x <= snps, j <= m
     virtual const uint64_t *binom(fiu_dataset *d, int m, hipStream_t s) = 0;
     // the dataset's pair table / fp4 image, built when missing if allowed
@@ -755,6 +826,10 @@ class DatasetWorkspace final : public Workspace {
     const uint64_t *binom(fiu_dataset *d, int m, hipStream_t s) override { return ensure_binom(d, m, s); }
     bool pair_table(fiu_dataset *d, hipStream_t s) override { return ensure_pair_table(d, s); }
     bool fp4_image(fiu_dataset *d, hipStream_t s) override { return ensure_fp4_image(d, s); }
+    bool tuples(fiu_dataset *d, int m, bool all_cells, hipStream_t s) override
+    {
+        return all_cells ? ensure_tuple_image(d, s) : ensure_tuple_tables(d, m, s);
+    }
     uint32_t max_candidates() const override { return UINT32_MAX; }
     uint64_t max_chunks() const override { return UINT64_MAX; }
     void buffers(fiu_dataset *d, uint32_t cap, uint64_t chunks, uint32_t outputs, Cand *&cand, Cand *&top,
@@ -825,6 +900,17 @@ class DatasetWorkspace final : public Workspace {
     const Cand *listed_ = nullptr;
 };
 
+// Whether the matrix-core scan around a head beats the popcount scan.  Its
+// tables, launches and half-empty tiles cost a few tenths of a millisecond:
+// measured at order 4 on 60 SNPs x 4,000 samples (2.0e9 combinations x
+// samples) 0.88 ms against 1.28, on 40 x 4,000 (3.7e8) 0.73 against 0.49; an
+// order-3 share on 300 x 4,000 (4.5e9) 0.51 against 0.53, on 150 x 4,000
+// (5.5e8) 0.39 against 0.38.
+bool tuple_scan_pays(int order, int n, double combos, uint64_t samples)
+{
+    return combos * (double)samples >= 2e9 && n >= 48;
+}
+
 // Exhaustive search of `d` in workspace `ws` (fiu_search, fiu_search_static).
 void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offset, uint32_t outputs,
             const fiu_config *cfg, int32_t *out_combos, float *out_mi, uint32_t *out_count, fiu_search_stats *stats)
@@ -892,11 +978,25 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     const uint64_t *binom = ws.binom(d, order, s);   // rows up to k: prefix ranks and combination keys
     int algo = FIU_ALGO_DIRECT;
     const bool small_classes = d->cases < (1u << 24) && d->ctrls < (1u << 24);   // fp32-exact counts
+    const double per_avg = (double)(n - M) / (double)(M + 1);
+    const double combos_est = (double)n_pref * per_avg;
+    const uint64_t samples = (uint64_t)d->cases + d->ctrls;
+    // matrix cores around a head of order - 2 SNPs: order 4, shares of orders
+    // 2 and 3 (the whole-scan kernels would compute the other shares' tiles
+    // too) and, every cell counted, order 3 on datasets with uncalled
+    // genotypes.  Measured against the popcount scans: order 4, 240 x 16,000,
+    // 33 ms against 478; share (8, 3) of order 3, 2,500 x 16,000, 40 ms
+    // against 110; order 3, 601 x 6,007 with 1 % uncalled, 6.5 ms against 17.7
+    const bool tup_all = !d->dev.uniform;
+    const bool tup_fits = tup_all ? order == 3 : order == 4 || (order <= 3 && step > 1);
+    const bool tup = tup_fits && (algo_req == FIU_ALGO_AUTO || (from_table && order >= 4)) &&
+                     d->cases < (1u << 16) && d->ctrls < (1u << 16) && tuple_scan_pays(order, n, combos_est, samples) &&
+                     ws.tuples(d, order - 1, tup_all, s);
     if (algo_req != FIU_ALGO_DIRECT && d->dev.uniform && order >= 4 && order <= kMaxKmOrder)
         algo = FIU_ALGO_MARGINAL;
     if (algo_req != FIU_ALGO_DIRECT && d->dev.uniform && (order == 2 || order == 3)) {
         algo = FIU_ALGO_MARGINAL;
-        if (order == 3 && !ws.pair_table(d, s)) algo = FIU_ALGO_DIRECT;  // table does not fit
+        if (order == 3 && !tup && !ws.pair_table(d, s)) algo = FIU_ALGO_DIRECT;  // table does not fit
         // order 2: the matrix-core scan is the faster exact path (4.4x on
         // 50,000 SNPs x 32,000 samples, also ahead on small inputs)
         if (order == 2 && algo_req != FIU_ALGO_MARGINAL) algo = FIU_ALGO_MFMA;
@@ -918,7 +1018,6 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     // 6 from 2,048 SNPs and 8,192 samples on (measured: the larger tile is
     // 7 % faster on 10,000 x 16,000, slower on 2,000 x 4,000 and below, where
     // its fewer workgroups and longer epilogue do not pay), else 4
-    const uint64_t samples = (uint64_t)d->cases + d->ctrls;
     int ring = algo == FIU_ALGO_MFMA && order == 3 && variant ? variant
                                                               : (n >= 2048 && samples >= 8192 ? 6 : 4);
     if (ring >= 5 && (d->cases >= (1u << 16) || d->ctrls >= (1u << 16) || !ws.private_memory())) ring = 4;
@@ -928,7 +1027,7 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     const int T = d->dev.n_pad / 64;
     const int64_t n_super = mfma2_superblocks(T);
     const bool int8 = (cfg && (cfg->flags & FIU_FLAG_MFMA_INT8)) || (order == 2 && variant == 1);
-    const bool mfma_fp4 = algo == FIU_ALGO_MFMA && !int8 && small_classes && ws.fp4_image(d, s);
+    const bool mfma_fp4 = algo == FIU_ALGO_MFMA && !tup && !int8 && small_classes && ws.fp4_image(d, s);
     // order-2 matrix-core variants: 1 int8 operands, 2 fp4 with the 64 x 64
     // tile, 3 fp4 with the 64 x 128 tile, 4 fp4 with the 128 x 128 tile (the
     // last two: 16-bit counts between the classes, so classes below 2^16
@@ -945,11 +1044,20 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     // prefixes of the distribution (about 2^24 combinations, spread over many
     // short wavefronts) histograms the screening MI and sets a starting
     // threshold, so that the first chunks push few candidates
-    const double per_avg = (double)(n - M) / (double)(M + 1);
     const uint64_t target = cfg && cfg->chunk_combos ? cfg->chunk_combos : (1ull << 28);
     const uint64_t max_chunks = ws.max_chunks();
     ChunkPlan plan;
-    if (algo == FIU_ALGO_MFMA && order == 2) {
+    // units of a scan around a head: the heads, or (order 2) blocks of b's
+    const int64_t tup_units =
+        !tup ? 0
+             : order == 2 ? ((int64_t)n_pref + tuple_b_block(2, tup_all) - 1) / tuple_b_block(2, tup_all)
+                          : (int64_t)binom_sat((uint64_t)n, (uint64_t)order - 2);
+    if (tup) {
+        const double per_unit = combos_est / (double)std::max<int64_t>(tup_units, 1);
+        int64_t len = (int64_t)std::max<double>(1.0, (double)target / std::max(per_unit, 1.0));
+        len = std::max<int64_t>(len, (int64_t)(((uint64_t)tup_units + max_chunks - 1) / max_chunks));
+        plan.set_uniform(tup_units, len);
+    } else if (algo == FIU_ALGO_MFMA && order == 2) {
         // chunks of super-blocks (262,144 pairs each) instead of prefixes
         int64_t len = std::max<int64_t>(1, (int64_t)(target / (64 * 4096)));
         // the 64 x 128 tile: launches of at most 64 super-blocks (2,048
@@ -985,11 +1093,10 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     // combinations at least (on 1,000 SNPs x 4,000 samples, top-10: 4,096
     // lets 3x more candidates through the scan and the merge, 65,536 makes
     // the sampling pass cost as much as the scan).
-    const double combos_est = (double)n_pref * per_avg;
     const uint64_t sample_floor = (uint64_t)std::max(16384.0, 2.0 * (double)outputs * combos_est / (double)cap);
     const uint64_t sample_cap = std::max<uint64_t>(sample_floor, (uint64_t)(combos_est * sample_frac));
     const int64_t sample_prefixes =
-        plan.count == 0 || !sample
+        plan.count == 0 || !sample || tup
             ? 0
             : tail_prefixes(n, M, (uint64_t)step, (uint64_t)offset, total_prefixes, (int64_t)n_pref,
                             std::min<uint64_t>({1ull << 24, target, sample_cap}));
@@ -1006,7 +1113,8 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     };
     Cand *mwork = big_merge ? ws.merge_work(d, pow2_at_least((uint64_t)outputs + cap)) : nullptr;
     // state reset and (when sampling) histogram cleared in one launch
-    check(launch_search_begin(state, sample_prefixes > 0 ? hist : nullptr, s), "search start launch");
+    const bool sampled = sample_prefixes > 0 || (tup && sample && plan.count > 0);
+    check(launch_search_begin(state, sampled ? hist : nullptr, s), "search start launch");
 
     ScanParams P{};
     P.step = step;
@@ -1020,6 +1128,13 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     P.pair = d->pair_ready ? d->pair.p : nullptr;
     P.cells = order >= kMinBigOrder ? ws.big_cells(d, order) : nullptr;
     mi_constants(d->cases, d->ctrls, d->complete(), P);
+    TupleArgs TA{};
+    if (tup) {
+        TA.F = tuple_image(d, tup_all);
+        for (int j = 1; j < order && !tup_all; ++j) TA.T.t[j] = d->tup[j].p;
+        TA.stride = 1;
+        TA.fill = kTupleFill;
+    }
 
     size_t ev = 0;
     bool timed = true;
@@ -1035,7 +1150,9 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
             timed = e0 && e1;
         }
         if (e0 && e1) check(hipEventRecord(e0, s), "event");
-        if (algo == FIU_ALGO_MFMA && order == 2) {
+        if (tup) {
+            check(launch_tuples(order, tup_all, d->dev, P, state, TA, s), "scan launch");
+        } else if (algo == FIU_ALGO_MFMA && order == 2) {
             check(launch_mfma2(d->dev, P, state, c.j0, c.j1, T, mfma_fp4 ? d->fp4.p : nullptr, m2_tile, s),
                   "scan launch");
         } else if (algo == FIU_ALGO_MFMA) {
@@ -1075,6 +1192,20 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
             check(launch_scan_marginal(order, d->dev, H, state, s), "sample launch");
         else
             check(launch_scan_direct(order, d->dev, H, state, s), "sample launch");
+        check(launch_tau_from_hist(hist, outputs, P.delta, state, s), "threshold launch");
+    } else if (sampled) {
+        // the same kernel over evenly spaced units: about 1/128 of the
+        // combinations (they cost what the scan's do), at least the floor
+        const double want = std::min(std::max((double)sample_floor, combos_est / 128.0), (double)target);
+        const double frac = std::min(1.0, want / std::max(combos_est, 1.0));
+        const int64_t count = std::max<int64_t>(1, (int64_t)std::ceil((double)tup_units * frac));
+        ScanParams H = P;
+        TupleArgs B = TA;
+        B.stride = std::max<int64_t>(1, tup_units / count);
+        H.j0 = B.stride / 2;
+        H.j1 = tup_units;
+        H.hist = hist;
+        check(launch_tuples(order, tup_all, d->dev, H, state, B, s), "sample launch");
         check(launch_tau_from_hist(hist, outputs, P.delta, state, s), "threshold launch");
     }
     for (uint64_t ci = 0; ci < plan.count; ++ci) run_chunk(ci, true);

@@ -181,6 +181,10 @@ struct fiu_dataset {
     fiu::DBuf<uint4> fp4;            // fp4 image of genotype rows 0/1 (matrix-core scans)
     fiu::DBuf<uint32_t> big;         // orders 10-12: count slots (big_cells_bytes)
     fiu::DBuf<fiu::Cand> mwork;      // outputs above kMaxOutputs: the merge's sort buffer
+    fiu::DBuf<uint4> fp4x;           // fp4 image of all three rows (all-cells matrix-core scans)
+    fiu::DBuf<uint32_t> tup[4];      // tables of m = 1 .. 3 SNPs' counts (TupleTables)
+    int tup_ready = 0;               // tables 1 .. tup_ready are built
+    bool fp4x_ready = false;
     bool fp4_ready = false;
     bool pair_ready = false;
     std::vector<hipEvent_t> events;
@@ -198,7 +202,8 @@ struct fiu_dataset {
     {
         arena = a;
         bits.arena = singles.arena = flags.arena = binom.arena = redo.arena = pair.arena = hist.arena = a;
-        fp4.arena = big.arena = mwork.arena = a;
+        fp4.arena = big.arena = mwork.arena = fp4x.arena = a;
+        for (auto &t : tup) t.arena = a;
         cand.arena = top.arena = a;
         state.arena = a;
     }
@@ -268,6 +273,17 @@ inline size_t pair_table_bytes(size_t snps) { return snps < 2 ? 0 : snps * (snps
 // fp4 image of genotype rows 0 and 1 (4 bits per sample and row); false when
 // it does not fit.
 bool ensure_fp4_image(fiu_dataset *d, hipStream_t s);
+// fp4 image of all three genotype rows; false when it does not fit.
+bool ensure_tuple_image(fiu_dataset *d, hipStream_t s);
+// Tables of 1 .. m SNPs' counts (TupleTables, m <= 3; classes below 2^16
+// samples, every SNP covering the same ones) and the fp4 image they are
+// counted from; false when they do not fit, or would take more than a quarter
+// of the free device memory.
+bool ensure_tuple_tables(fiu_dataset *d, int m, hipStream_t s);
+// The image a scan around a head reads.
+Fp4Image tuple_image(const fiu_dataset *d, bool all_cells);
+// Workgroups of such a scan that keep the device busy through its tail.
+constexpr int32_t kTupleFill = 16384;
 // The dataset admits the matrix-core scans: every SNP covers the same samples
 // (the counts of the other cells follow by inclusion-exclusion) and both
 // classes are below 2^24 samples (FP32 counts are exact).

@@ -70,6 +70,33 @@ hipError_t launch_contingency_batch(const DevData &D, const int32_t *combos, int
 hipError_t launch_mi_batch(const uint32_t *tables, uint64_t n, uint64_t ct_size, double n64, double hy64, float *out,
                            hipStream_t s);
 
+// Combinations around a head of order - 2 SNPs on the matrix cores
+// (fiu_tuples.hip).  Counts of m SNPs in table t[m]: per m-combination, in
+// lexicographic rank order, 2^m words (genotypes 0 and 1, first SNP most
+// significant), cases | controls << 16; every class below 2^16 samples.
+struct TupleTables {
+    const uint32_t *t[4];
+};
+struct TupleArgs {
+    Fp4Image F;              // genotype rows 0, 1 (marginal) or 0, 1, 2 (all cells)
+    TupleTables T;           // marginal scans: tables of fewer SNPs than the order
+    uint32_t *out;           // set: write the order's table (orders 2, 3) instead of scoring
+    int64_t stride;          // units j0, j0 + stride, .. of [j0, j1) (a sample), else 1
+    int64_t units;           // set by the launcher
+    int32_t rounds;          // set by the launcher
+    int32_t fill;            // workgroups that fill the device
+};
+// Scores (or samples, P.hist) units [P.j0, P.j1): heads (order >= 3) or blocks
+// of tuple_b_block b's (order 2) of the share (P.step, P.offset).  all_cells:
+// orders 2 and 3, any dataset; else orders 2 to 4, uniform datasets.
+int tuple_b_block(int order, bool all_cells);
+hipError_t launch_tuples(int order, bool all_cells, const DevData &D, const ScanParams &P, TopState *st,
+                         const TupleArgs &A, hipStream_t s);
+// t[1] of the tables (2 n words), and the fp4 image of all three rows
+// (12 (quads[0] + quads[1]) n_pad uint4, controls after cases).
+hipError_t launch_tuple_singles(const DevData &D, uint32_t *out, hipStream_t s);
+hipError_t launch_tuple_image(const DevData &D, uint4 *out, hipStream_t s);
+
 // Batched scans: resident workgroups of the persistent scan kernel of launch
 // 0 (popcount orders 2-3), 1 (direct order 4), 2 (matrix-core kinds, a
 // multiple of 8) or 3 (marginal orders 4-5) on the current device, and the

@@ -1,0 +1,585 @@
+// gfx950 kernels that count k-combinations on the matrix cores around a fixed
+// head of k - 2 SNPs: the scans of order 4, of round-robin shares and of
+// datasets with uncalled genotypes, and the tables of lower-order counts that
+// the marginal form needs.
+//
+// For a head h = (s_1 < .. < s_{k-2}) the counts of the combinations
+// (h, b, c) are dot products over the samples: row (b, y) times row (c, z)
+// masked by the head's genotype rows.  Marginal form (complete coverage):
+// genotypes 0 and 1 only, 2^k products per combination; the other cells
+// follow by inclusion-exclusion from the counts of fewer SNPs.  All-cells
+// form (any dataset): genotypes 0, 1 and 2, 3^k products and no tables.
+//
+// Counts of a combination travel as one 32-bit word per cell, cases in the
+// low half and controls in the high half (every class below 2^16 samples):
+// the inclusion-exclusion then runs on both classes with one subtraction,
+// since every intermediate value is itself a pair of counts and no half
+// borrows from the other.
+#include "fiu_kernels.h"
+
+#include <algorithm>
+
+#include "fiu_matrix.h"
+#include "fiu_score.h"
+
+namespace fiu {
+
+namespace {
+
+constexpr int ipow(int b, int e) { return e == 0 ? 1 : b * ipow(b, e - 1); }
+
+enum TupleMode { kScore = 0, kSample = 1, kTable = 2 };
+
+// Shape of one kernel: NB blocks of 16 b rows per workgroup against 64 c
+// columns, wave w taking c0 + 16 w ..; NB is the most whose accumulators
+// (4 registers per product and block) stay at 128 or below, so that two
+// waves per SIMD fit.
+template <int K, bool ALL> struct Tup {
+    static constexpr int G = ALL ? 3 : 2;            // genotype rows per SNP
+    static constexpr int H = K - 2;                  // head SNPs
+    static constexpr int M = ipow(G, H);             // head cells
+    static constexpr int dots = ipow(G, K);
+    static constexpr int NB = dots <= 8 ? 4 : dots == 9 ? 2 : dots == 16 ? 2 : 1;
+    static constexpr int BT = 16 * NB;               // b rows per workgroup
+    static constexpr int b_rows = G * BT;            // LDS rows (64 bytes) per stage
+    static constexpr int c_rows = G * 64;
+    static constexpr int a_rows = G * H;             // per wave: every wave has its own copy
+    static constexpr int stage = (b_rows + c_rows + 4 * a_rows) * 64;
+    static constexpr int ring = 4;                   // stages in LDS, ring - 1 in flight
+    static constexpr int b_loads = (b_rows + 63) / 64;   // 16-byte units / 4 waves / 64 lanes
+    static constexpr int loads = b_loads + G + (H > 0 ? 1 : 0);   // per wave and stage
+    static constexpr int inst = 4 * NB;              // combinations per lane
+    static constexpr int cells = ipow(3, K);
+    static_assert(loads * (ring - 2) < 16, "vmcnt immediate");
+};
+
+__device__ __forceinline__ int swz16(int r) { return (r >> 1) & 3; }
+
+// A workgroup's head and its b progression: SNPs b_first, b_first + step, ..
+// (the share's prefixes (head, b)), below n - 1.
+template <int H> struct Head {
+    int s[H > 0 ? H : 1];
+    int last;        // largest head SNP (-1 without a head)
+    int b_first;     // n - 1 or above: no prefix of the share
+};
+
+template <int K>
+__device__ __forceinline__ Head<K - 2> head_at(const ScanParams &P, int n, uint64_t h)
+{
+    constexpr int H = K - 2;
+    Head<H> r;
+    r.last = -1;
+    if constexpr (H > 0) {
+        unrank(h, n, H, P.binom, r.s);
+        r.last = r.s[H - 1];
+    }
+    r.b_first = r.last + 1;
+    if (P.step != 1 || P.offset != 0) {
+        // rank of the prefix (head, b) = r0 + b
+        const uint64_t stride = (uint64_t)n + 1;
+        int64_t r0 = (int64_t)P.binom[(uint64_t)(K - 1) * stride + n] - n;
+#pragma unroll
+        for (int i = 0; i < H; ++i) r0 -= (int64_t)P.binom[(uint64_t)(K - 1 - i) * stride + (n - 1 - r.s[i])];
+        const int64_t at = r0 + r.b_first, rel = at - P.offset;
+        const int64_t skip = rel < 0 ? -rel : (P.step - rel % P.step) % P.step;
+        r.b_first = skip >= n ? n : r.b_first + (int)skip;
+    }
+    return r;
+}
+
+// Positions of a combination: 0 .. K - 3 the head, K - 2 b, K - 1 c.  For
+// every proper subset of them (bit i = position i) the address of its counts
+// in the table of its size, split into the part that depends on the head and
+// c (`p`) and the part that depends on b.  Entry of the m-combination
+// t_0 < .. < t_{m-1}: its lexicographic rank C(n, m) - 1 - sum_i C(n-1-t_i,
+// m-i), 2^m words each.
+template <int K> struct Subsets {
+    const uint32_t *p[1 << K];
+};
+
+template <int K>
+__device__ __forceinline__ void subsets_at(Subsets<K> &S, const TupleTables &T, const ScanParams &P, int n,
+                                           const Head<K - 2> &h, int c)
+{
+    constexpr int H = K - 2;
+    const uint64_t stride = (uint64_t)n + 1;
+    static_for<(1 << K) - 1>([&](auto I) __attribute__((always_inline)) {
+        constexpr int s = decltype(I)::value;
+        if constexpr (s != 0) {
+            constexpr int m = __builtin_popcount(s);
+            int64_t r = (int64_t)P.binom[(uint64_t)m * stride + n] - 1;
+            int at = 0;
+#pragma unroll
+            for (int i = 0; i < H; ++i)
+                if (s >> i & 1) {
+                    r -= (int64_t)P.binom[(uint64_t)(m - at) * stride + (n - 1 - h.s[i])];
+                    ++at;
+                }
+            if constexpr ((s >> (K - 1) & 1) != 0) r -= n - 1 - c;
+            S.p[s] = T.t[m] + (r << m);
+        }
+    });
+}
+
+// Words of the counts of subset s for the instance's b.
+template <int K, int s>
+__device__ __forceinline__ const uint32_t *subset_words(const Subsets<K> &S, int n, int b)
+{
+    constexpr int m = __builtin_popcount(s);
+    constexpr bool has_b = (s >> (K - 2) & 1) != 0, has_c = (s >> (K - 1) & 1) != 0;
+    if constexpr (!has_b) return S.p[s];
+    const int64_t v = n - 1 - b;
+    return S.p[s] - ((has_c ? v * (v - 1) / 2 : v) << m);
+}
+
+// The 3^K cells (word: cases | controls << 16, first SNP most significant)
+// of the combination whose 2^K corner counts (genotypes 0 and 1) are corner(i).
+template <int K, class C>
+__device__ __forceinline__ void marginal_cells(const Subsets<K> &S, int n, int b, uint32_t total, C &&corner,
+                                               uint32_t (&m)[ipow(3, K)])
+{
+    // entry with "any genotype" (digit 2) outside subset s: the counts of s
+    static_for<(1 << K)>([&](auto I) __attribute__((always_inline)) {
+        constexpr int s = decltype(I)::value;
+        constexpr int sz = __builtin_popcount(s);
+        // cell index of entry e of the subset: the digits of its positions
+        auto cell_of = [](int e) constexpr {
+            int idx = 0, at = 0;
+            for (int i = 0; i < K; ++i) {
+                int d = 2;
+                if (s >> i & 1) {
+                    d = e >> (sz - 1 - at) & 1;
+                    ++at;
+                }
+                idx = idx * 3 + d;
+            }
+            return idx;
+        };
+        if constexpr (s == 0) {
+            m[ipow(3, K) - 1] = total;
+        } else if constexpr (s == (1 << K) - 1) {
+            static_for<(1 << K)>([&](auto E) __attribute__((always_inline)) {
+                constexpr int e = decltype(E)::value;
+                constexpr int at = cell_of(e);
+                m[at] = corner(std::integral_constant<int, e>{});
+            });
+        } else {
+            const uint32_t *p = subset_words<K, s>(S, n, b);
+            if constexpr (sz == 1) {
+                const uint2 v = *(const uint2 *)p;
+                constexpr int a0 = cell_of(0), a1 = cell_of(1);
+                m[a0] = v.x;
+                m[a1] = v.y;
+            } else {
+                static_for<(1 << sz) / 4>([&](auto Q) __attribute__((always_inline)) {
+                    constexpr int q = decltype(Q)::value;
+                    const uint4 v = ((const uint4 *)p)[q];
+                    constexpr int a0 = cell_of(4 * q), a1 = cell_of(4 * q + 1), a2 = cell_of(4 * q + 2),
+                                  a3 = cell_of(4 * q + 3);
+                    m[a0] = v.x;
+                    m[a1] = v.y;
+                    m[a2] = v.z;
+                    m[a3] = v.w;
+                });
+            }
+        }
+    });
+    // "any" -> genotype 2, last SNP first
+#pragma unroll
+    for (int d = 1; d < ipow(3, K); d *= 3)
+#pragma unroll
+        for (int hi = 0; hi < ipow(3, K); hi += 3 * d)
+#pragma unroll
+            for (int lo = 0; lo < d; ++lo) m[hi + 2 * d + lo] -= m[hi + lo] + m[hi + d + lo];
+}
+
+// What bounds it: the 2^K (3^K) products per combination, 16 passes of a SIMD
+// each for 256 combinations x 128 samples; the operands come from L2 through
+// a ring of 64-byte LDS rows filled by direct-to-LDS loads.  Why this split:
+// the head's masks go on the c operand, of which a wave holds one 16-row
+// block, so that a masked fragment (1 three-operand AND per word and head
+// cell) feeds NB x G products; each wave loads its own c and head rows and a
+// quarter of the shared b rows.
+template <int K, bool ALL, int MODE>
+__device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P, TopState *st, const TupleArgs &A,
+                                           const Head<K - 2> &hd, int bmin, int c0,
+                                           int8_t (*lds)[Tup<K, ALL>::stage], uint32_t *lds_hist)
+{
+    using Z = Tup<K, ALL>;
+    constexpr int G = Z::G, H = Z::H, NB = Z::NB, R = Z::ring;
+    const int n = D.n, np = D.n_pad;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // staging offsets within a quad of the image.  b rows: 16-byte units
+    // U = b_rows w + 64 i + lane of the stage's b part, row U / 4 = (genotype,
+    // progression index), stored segment U % 4; rows past the last SNP read
+    // the last one and are dropped in the epilogue
+    uint32_t vb[Z::b_loads];
+#pragma unroll
+    for (int i = 0; i < Z::b_loads; ++i) {
+        const int u = Z::b_rows * w + 64 * i + lane, row = u >> 2;
+        const int g = row / Z::BT, j = row % Z::BT;
+        const int64_t snp = std::min<int64_t>((int64_t)bmin + (int64_t)P.step * j, n - 1);
+        vb[i] = 16u * (uint32_t)(4 * (g * np + (int)snp) + ((u & 3) ^ swz16(row & 15)));
+    }
+    const int lr = lane >> 2, ls = (lane & 3) ^ swz16(lr);
+    const uint32_t vc = 16u * (uint32_t)(4 * std::min(c0 + 16 * w + lr, n - 1) + ls);
+    uint32_t va = 0;
+    if constexpr (H > 0) {
+        int s = hd.s[0];
+#pragma unroll
+        for (int i = 1; i < H; ++i)
+            if (lr >= G * i) s = hd.s[i];
+        va = 16u * (uint32_t)(4 * ((lr % G) * np + s) + (lane & 3));
+    }
+    const bool a_lane = lane < 4 * Z::a_rows;
+    const int rr = lane & 15, kc = lane >> 4;
+    const int fo = rr * 64 + ((kc ^ swz16(rr)) << 4), ao = kc << 4;
+    // a wave whose 16 columns all lie past the last SNP or at or below the
+    // tile's first b has no combination: it stages and waits with the others
+    const bool active = c0 + 16 * w < n;
+    v4f acc[Z::dots][NB];
+    // per lane: the counts of its combinations, [instance][product]; the
+    // pointer passes through an empty asm so that it stays in memory
+    uint32_t counts_mem[Z::inst * Z::dots];
+    __attribute__((address_space(5))) uint32_t *counts = (__attribute__((address_space(5))) uint32_t *)counts_mem;
+    asm volatile("" : "+v"(counts));
+#pragma unroll 1
+    for (int cls = 0; cls < 2; ++cls) {
+#pragma unroll
+        for (int e = 0; e < Z::dots; ++e)
+#pragma unroll
+            for (int bb = 0; bb < NB; ++bb) acc[e][bb] = (v4f){0.f, 0.f, 0.f, 0.f};
+        const int iters = D.quads[cls];
+        const uint4 *img = A.F.base + A.F.class_off[cls];
+        auto issue = [&](int q) __attribute__((always_inline)) {
+            const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
+                (void *)(img + (int64_t)q * 4 * G * np), (short)0, 64 * G * np, 0x00020000);
+            int8_t *s = lds[q % R];
+#pragma unroll
+            for (int i = 0; i < Z::b_loads; ++i) {
+                int8_t *to = s + (Z::b_rows * w + 64 * i) * 16;
+                if (64 * (i + 1) <= Z::b_rows) dma16(rq, vb[i], to);
+                else if (lane < Z::b_rows - 64 * i) dma16(rq, vb[i], to);
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+                dma16(rq, vc + 64u * (uint32_t)(g * np), s + (Z::b_rows + 64 * g + 16 * w) * 64);
+            if constexpr (H > 0)
+                if (a_lane) dma16(rq, va, s + (Z::b_rows + Z::c_rows + Z::a_rows * w) * 64);
+        };
+#pragma unroll
+        for (int q = 0; q < R - 1; ++q)
+            if (q < iters) issue(q);
+        auto stage = [&](int it, bool steady) __attribute__((always_inline)) {
+            // this wave's loads of stage it are complete once at most those
+            // of the stages issued after it are pending; the barrier then
+            // publishes every wave's part, and tells that the slot of stage
+            // it - 1 is read no more
+            if (steady) wait_vmcnt<Z::loads * (R - 2)>();
+            else wait_stages<R - 2, Z::loads>(iters - 1 - it);
+            stage_barrier();
+            const bool more = steady || it + R - 1 < iters;
+            if (active) {
+                __builtin_amdgcn_s_setprio(1);
+                const int8_t *sb = lds[it % R];
+                v4i fa[H > 0 ? Z::a_rows : 1], fc[G], fb[G][NB];
+                if constexpr (H > 0) {
+#pragma unroll
+                    for (int r = 0; r < Z::a_rows; ++r)
+                        fa[r] = *(const v4i *)(sb + (Z::b_rows + Z::c_rows + Z::a_rows * w + r) * 64 + ao);
+                }
+#pragma unroll
+                for (int g = 0; g < G; ++g) fc[g] = *(const v4i *)(sb + (Z::b_rows + 64 * g + 16 * w) * 64 + fo);
+#pragma unroll
+                for (int g = 0; g < G; ++g)
+#pragma unroll
+                    for (int bb = 0; bb < NB; ++bb) fb[g][bb] = *(const v4i *)(sb + (g * Z::BT + 16 * bb) * 64 + fo);
+                if (more) issue(it + R - 1);
+                static_for<Z::M>([&](auto MI) __attribute__((always_inline)) {
+                    constexpr int mi = decltype(MI)::value;
+#pragma unroll
+                    for (int z = 0; z < G; ++z) {
+                        v4i mc = fc[z];   // nibble 0x2 & 0x2 = 1.0, else 0
+#pragma unroll
+                        for (int i = 0; i < H; ++i) mc &= fa[i * G + mi / ipow(G, H - 1 - i) % G];
+                        const v8i c8 = {mc[0], mc[1], mc[2], mc[3], 0, 0, 0, 0};
+#pragma unroll
+                        for (int y = 0; y < G; ++y)
+#pragma unroll
+                            for (int bb = 0; bb < NB; ++bb) {
+                                const v8i b8 = {fb[y][bb][0], fb[y][bb][1], fb[y][bb][2], fb[y][bb][3], 0, 0, 0, 0};
+                                v4f &d = acc[(mi * G + y) * G + z][bb];
+                                d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b8, c8, d, 4, 4, 0, 0, 0, 0);
+                            }
+                    }
+                });
+                __builtin_amdgcn_s_setprio(0);
+            } else if (more) {
+                issue(it + R - 1);
+            }
+        };
+        int it = 0;
+        for (; it + R - 1 < iters; ++it) stage(it, true);
+        for (; it < iters; ++it) stage(it, false);
+        // the ring is filled again by the next class (or tile)
+        stage_barrier();
+        if (active) {
+#pragma unroll
+            for (int bb = 0; bb < NB; ++bb)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int e = 0; e < Z::dots; ++e) {
+                        const int at = (bb * 4 + j) * Z::dots + e;
+                        const uint32_t v = (uint32_t)acc[e][bb][j];
+                        if (cls == 0) counts[at] = v;
+                        else counts[at] |= v << 16;
+                    }
+        }
+    }
+    if (!active) return;
+    // epilogue: lane holds column c = c0 + 16 w + lane % 16 and rows
+    // b = bmin + step (16 bb + 4 (lane / 16) + j)
+    const int c = std::min(c0 + 16 * w + rr, n - 1);
+    const bool c_ok = c0 + 16 * w + rr < n;
+    const float tau = MODE == kScore ? st->tau : 0.0f;
+    const uint64_t tau_combo = MODE == kScore ? st->tau_combo : 0;
+    auto b_at = [&](int i) { return (int64_t)bmin + (int64_t)P.step * (16 * (i >> 2) + 4 * kc + (i & 3)); };
+    Subsets<K> S;
+    if constexpr (!ALL && MODE != kTable) subsets_at<K>(S, A.T, P, n, hd, c);
+    auto cells_of = [&](int i, int b, uint32_t (&m)[Z::cells]) __attribute__((always_inline)) {
+        const __attribute__((address_space(5))) uint32_t *w0 = counts + i * Z::dots;
+        if constexpr (ALL) {
+#pragma unroll
+            for (int e = 0; e < Z::cells; ++e) m[e] = w0[e];
+        } else {
+            marginal_cells<K>(S, n, b, D.total[0] | D.total[1] << 16,
+                              [&](auto E) __attribute__((always_inline)) { return w0[decltype(E)::value]; }, m);
+        }
+    };
+    uint32_t pend = 0;
+#pragma unroll 1
+    for (int i = 0; i < Z::inst; ++i) {
+        const int64_t bi = b_at(i);
+        const bool valid = c_ok && bi < c;
+        if constexpr (MODE == kTable) {
+            if (valid) {
+                const uint64_t stride = (uint64_t)n + 1;
+                int64_t r = (int64_t)P.binom[(uint64_t)K * stride + n] - 1;
+#pragma unroll
+                for (int q = 0; q < H; ++q) r -= (int64_t)P.binom[(uint64_t)(K - q) * stride + (n - 1 - hd.s[q])];
+                const int64_t v = n - 1 - bi;
+                r -= v * (v - 1) / 2 + (n - 1 - c);
+                uint4 *to = (uint4 *)(A.out + (r << K));
+                const __attribute__((address_space(5))) uint32_t *w0 = counts + i * Z::dots;
+#pragma unroll
+                for (int e = 0; e < Z::dots; e += 4) to[e / 4] = make_uint4(w0[e], w0[e + 1], w0[e + 2], w0[e + 3]);
+            }
+        } else {
+            // a combination outside the scan reads a valid one's tables
+            const int b = valid ? (int)bi : hd.last + 1;
+            uint32_t m[Z::cells];
+            cells_of(i, b, m);
+            if constexpr (MODE == kSample) {
+                const float ms = fmaf(screen_sum_fn<Z::cells>([&](int x, float &fc, float &ft) __attribute__((always_inline)) {
+                                          fc = (float)(m[x] & 0xffffu);
+                                          ft = (float)(m[x] >> 16);
+                                      }),
+                                      P.inv_n * 0.69314718f, P.hy);
+                if (valid) atomicAdd(&lds_hist[hist_bin(ms)], 1u);
+            } else {
+                bool pass = valid;
+                if (P.bounded) {
+                    const float bd = mi_bound_fn<Z::cells>(
+                        [&](int x, float &fc, float &fx) __attribute__((always_inline)) {
+                            fc = (float)(m[x] & 0xffffu);
+                            fx = fc + (float)(m[x] >> 16);
+                        },
+                        P.frac_c, P.chi_scale);
+                    pass = pass && bound_passes(bd, tau, P.delta);
+                }
+                if (pass) pend |= 1u << i;
+            }
+        }
+    }
+    if constexpr (MODE == kScore) {
+        // one marked combination per lane and round: screen, exact MI, push
+        while (__ballot(pend != 0)) {
+            bool want = false;
+            float mf = 0.0f;
+            uint64_t combo = ~0ull;
+            if (pend) {
+                const int i = __builtin_ctz(pend);
+                pend &= pend - 1;
+                const int b = (int)b_at(i);
+                uint32_t m[Z::cells];
+                cells_of(i, b, m);
+                auto cell = [&](int x, float &fc, float &ft) __attribute__((always_inline)) {
+                    fc = (float)(m[x] & 0xffffu);
+                    ft = (float)(m[x] >> 16);
+                };
+                const float ms = fmaf(screen_sum_fn<Z::cells>(cell), P.inv_n * 0.69314718f, P.hy);
+                if (ms >= tau - P.delta) {
+#pragma clang fp contract(off)
+                    double hx = 0.0, hall = 0.0;
+                    mi_exact_part_fn<Z::cells>(
+                        [&](int x, uint32_t &n0, uint32_t &n1) __attribute__((always_inline)) {
+                            n0 = m[x] & 0xffffu;
+                            n1 = m[x] >> 16;
+                        },
+                        P.n64, hx, hall);
+                    mf = (float)(hx + P.hy64 - hall);
+                    int pre[K - 1];
+#pragma unroll
+                    for (int q = 0; q < H; ++q) pre[q] = hd.s[q];
+                    pre[H] = b;
+                    combo = prefix_key(P.binom, n, pre, K - 1) + (uint64_t)c;
+                    want = better(mf, combo, tau, tau_combo);
+                }
+            }
+            push_candidates(want, mf, combo, P, st);
+        }
+    }
+}
+
+// Work: unit u of [j0, j1), u = j0 + i * stride, is a head (K >= 3) or a block
+// of BT b's (K = 2, no head).  A head's tiles (b blocks of BT, and for each
+// the 64-column tiles past the block's first b) are dealt to 8 * `rounds`
+// workgroups.  Workgroup L runs on XCD L % 8: for 64 units in a row it takes
+// the same tile number, so that units resident on one XCD share their b and
+// c rows in its L2, then the next, so that the XCDs' shares of units with
+// few tiles even out.
+template <int K, bool ALL, int MODE>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_tuples(const DevData D, const ScanParams P, TopState *st, const TupleArgs A)
+{
+    using Z = Tup<K, ALL>;
+    __shared__ __attribute__((aligned(1024))) int8_t lds[Z::ring][Z::stage];
+    __shared__ uint32_t lds_hist[MODE == kSample ? kHistBins : 1];
+    const int64_t L = blockIdx.x, s = L >> 3;
+    const int64_t i = s % A.units, first = s / A.units * 8 + ((L + (i >> 6)) & 7);
+    const int64_t u = P.j0 + i * A.stride;
+    const Head<Z::H> hd = head_at<K>(P, D.n, K == 2 ? 0 : (uint64_t)u);
+    hist_begin<MODE == kSample>(lds_hist);
+    int64_t tile = first;
+    int64_t bmin = hd.b_first;
+    if constexpr (K == 2) bmin += u * Z::BT * P.step;
+    while (bmin < D.n - 1) {
+        const int ct = (int)(D.n - 1 - bmin + 63) >> 6;   // 64-column tiles past bmin
+        if (tile < ct) {
+            tuple_tile<K, ALL, MODE>(D, P, st, A, hd, (int)bmin, (int)bmin + 1 + 64 * (int)tile, lds, lds_hist);
+            tile += 8 * (int64_t)A.rounds;
+        } else {
+            if constexpr (K == 2) break;
+            tile -= ct;
+            bmin += (int64_t)Z::BT * P.step;
+        }
+    }
+    hist_end<MODE == kSample>(lds_hist, P.hist);
+}
+
+// fp4 image of genotype rows 0 .. G - 1, as the two-row image of the pair
+// and triple scans: quad q, genotype g, SNP s of a class at 4 ((G q + g)
+// n_pad + s) past the class's offset.
+__global__ void k_tuple_image(const uint4 *__restrict__ bits, DevData D, uint4 *__restrict__ out, uint64_t off1)
+{
+    const uint64_t id = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t per0 = 3ull * D.quads[0] * D.n_pad, total = per0 + 3ull * D.quads[1] * D.n_pad;
+    if (id >= total) return;
+    const int cls = id < per0 ? 0 : 1;
+    const uint64_t v = cls ? id - per0 : id;
+    const uint4 w = bits[D.class_off[cls] + v];
+    uint4 *dst = out + (cls ? off1 : 0) + 4 * v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t x = comp(w, e);
+        dst[e] = make_uint4(byte_fp4(x & 255u), byte_fp4(x >> 8 & 255u), byte_fp4(x >> 16 & 255u), byte_fp4(x >> 24));
+    }
+}
+
+// Table of one SNP: words (genotype 0, genotype 1), cases | controls << 16.
+__global__ void k_tuple_singles(DevData D, uint32_t *out)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= 2 * D.n) return;
+    const uint32_t *sp = D.singles + (size_t)(i >> 1) * 6 + (i & 1);
+    out[i] = sp[0] | sp[3] << 16;
+}
+
+constexpr int64_t kMaxBlocks = (int64_t)(0xffffffffu / (uint32_t)kBlock);
+
+template <int K, bool ALL, int MODE>
+hipError_t launch_tuples_as(const DevData &D, ScanParams P, TopState *st, TupleArgs A, hipStream_t s)
+{
+    using Z = Tup<K, ALL>;
+    int64_t units = (P.j1 - P.j0 + A.stride - 1) / A.stride;
+    if (units <= 0) return hipSuccess;
+    // tiles of the head with the most (the first), dealt in rounds of 8: one
+    // round per 8 tiles unless the units alone fill the device
+    const int64_t nb = std::max<int64_t>(1, (D.n + Z::BT * P.step - 1) / (Z::BT * P.step)), nc = (D.n + 63) / 64;
+    const int64_t most = K == 2 ? nc : nb * nc;
+    const int64_t want = std::max<int64_t>(1, (int64_t)A.fill / std::max<int64_t>(1, 8 * units));
+    A.rounds = (int32_t)std::min<int64_t>((most + 7) / 8, want);
+    const int64_t per_launch = std::max<int64_t>(1, kMaxBlocks / (8 * A.rounds));
+    for (int64_t i = 0; i < units; i += per_launch) {
+        ScanParams Q = P;
+        TupleArgs B = A;
+        Q.j0 = P.j0 + i * A.stride;
+        B.units = std::min(per_launch, units - i);
+        hipLaunchKernelGGL((k_tuples<K, ALL, MODE>), dim3((unsigned)(B.units * 8 * B.rounds)), dim3(kBlock), 0, s, D, Q,
+                           st, B);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+template <int K, bool ALL>
+hipError_t launch_tuples_k(const DevData &D, const ScanParams &P, TopState *st, const TupleArgs &A, hipStream_t s)
+{
+    if constexpr (!ALL && K <= 3)
+        if (A.out) return launch_tuples_as<K, ALL, kTable>(D, P, st, A, s);
+    if (P.hist) return launch_tuples_as<K, ALL, kSample>(D, P, st, A, s);
+    return launch_tuples_as<K, ALL, kScore>(D, P, st, A, s);
+}
+
+}  // namespace
+
+int tuple_b_block(int order, bool all_cells)
+{
+    if (all_cells) return order == 2 ? Tup<2, true>::BT : Tup<3, true>::BT;
+    return order == 2 ? Tup<2, false>::BT : order == 3 ? Tup<3, false>::BT : Tup<4, false>::BT;
+}
+
+hipError_t launch_tuples(int order, bool all_cells, const DevData &D, const ScanParams &P, TopState *st,
+                         const TupleArgs &A, hipStream_t s)
+{
+    if (all_cells) {
+        if (order == 2) return launch_tuples_k<2, true>(D, P, st, A, s);
+        if (order == 3) return launch_tuples_k<3, true>(D, P, st, A, s);
+        return hipErrorInvalidValue;
+    }
+    if (order == 2) return launch_tuples_k<2, false>(D, P, st, A, s);
+    if (order == 3) return launch_tuples_k<3, false>(D, P, st, A, s);
+    if (order == 4) return launch_tuples_k<4, false>(D, P, st, A, s);
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_tuple_singles(const DevData &D, uint32_t *out, hipStream_t s)
+{
+    if (D.n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_tuple_singles, dim3((unsigned)((2 * D.n + 255) / 256)), dim3(256), 0, s, D, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_tuple_image(const DevData &D, uint4 *out, hipStream_t s)
+{
+    const uint64_t total = 3ull * (D.quads[0] + D.quads[1]) * D.n_pad;
+    if (!total) return hipSuccess;
+    hipLaunchKernelGGL(k_tuple_image, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, D.bits, D, out,
+                       12ull * D.quads[0] * D.n_pad);
+    return hipGetLastError();
+}
+
+}  // namespace fiu
