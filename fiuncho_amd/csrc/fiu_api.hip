@@ -601,6 +601,7 @@ bool ensure_tuple_tables(fiu_dataset *d, int m, hipStream_t s)
     TupleArgs A{};
     A.F = tuple_image(d, false);
     A.stride = 1;
+    A.tile_stride = 1;
     A.fill = kTupleFill;
     ScanParams P{};
     P.step = 1;
@@ -983,12 +984,13 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     const uint64_t samples = (uint64_t)d->cases + d->ctrls;
     // matrix cores around a head of order - 2 SNPs: order 4, shares of orders
     // 2 and 3 (the whole-scan kernels would compute the other shares' tiles
-    // too) and, every cell counted, order 3 on datasets with uncalled
+    // too) and, every cell counted, orders 2 and 3 on datasets with uncalled
     // genotypes.  Measured against the popcount scans: order 4, 240 x 16,000,
     // 33 ms against 478; share (8, 3) of order 3, 2,500 x 16,000, 40 ms
-    // against 110; order 3, 601 x 6,007 with 1 % uncalled, 6.5 ms against 17.7
+    // against 110; with 1 % uncalled, order 3 on 601 x 6,007 5.9 ms against
+    // 16.9 and order 2 on 4,001 x 8,999 0.95 ms against 3.1
     const bool tup_all = !d->dev.uniform;
-    const bool tup_fits = tup_all ? order == 3 : order == 4 || (order <= 3 && step > 1);
+    const bool tup_fits = tup_all ? order <= 3 : order == 4 || (order <= 3 && step > 1);
     const bool tup = tup_fits && (algo_req == FIU_ALGO_AUTO || (from_table && order >= 4)) &&
                      d->cases < (1u << 16) && d->ctrls < (1u << 16) && tuple_scan_pays(order, n, combos_est, samples) &&
                      ws.tuples(d, order - 1, tup_all, s);
@@ -1040,10 +1042,9 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
                             ? m2_pick : 0;
 
     // chunk plan: even chunks of about `target` combinations (at most
-    // max_chunks of them); before the first, a sampling pass over the last
-    // prefixes of the distribution (about 2^24 combinations, spread over many
-    // short wavefronts) histograms the screening MI and sets a starting
-    // threshold, so that the first chunks push few candidates
+    // max_chunks of them); before the first, a sampling pass histograms the
+    // screening MI and sets a starting threshold, so that the first chunks
+    // push few candidates
     const uint64_t target = cfg && cfg->chunk_combos ? cfg->chunk_combos : (1ull << 28);
     const uint64_t max_chunks = ws.max_chunks();
     ChunkPlan plan;
@@ -1082,24 +1083,32 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
         plan.set_uniform((int64_t)n_pref, len);
     }
     if (plan.count > max_chunks) fail(FIU_ERR_UNSUPPORTED, "too many launches for this entry point");
-    const bool sample = !(cfg && (cfg->flags & FIU_FLAG_NO_THRESHOLD_SAMPLE));
-    // at most about 1/16 of the scan's combinations (the pass screens every
-    // combination it samples with a popcount kernel), 1/256 ahead of a
-    // matrix-core scan, which costs 5-12x less per combination
-    const double sample_frac = algo == FIU_ALGO_MFMA ? 1.0 / 256.0 : 1.0 / 16.0;
-    // The floor: the scan pushes about outputs x combinations / sample
-    // candidates above the starting threshold (twice that with the bins'
-    // width), kept near the size of one chunk's candidate buffer; 16,384
-    // combinations at least (on 1,000 SNPs x 4,000 samples, top-10: 4,096
-    // lets 3x more candidates through the scan and the merge, 65,536 makes
-    // the sampling pass cost as much as the scan).
-    const uint64_t sample_floor = (uint64_t)std::max(16384.0, 2.0 * (double)outputs * combos_est / (double)cap);
-    const uint64_t sample_cap = std::max<uint64_t>(sample_floor, (uint64_t)(combos_est * sample_frac));
+    const bool sample = plan.count > 0 && !(cfg && (cfg->flags & FIU_FLAG_NO_THRESHOLD_SAMPLE));
+    // A sample of one combination in S lets about S x outputs of them past
+    // the starting threshold, each an FP64 MI and a merge entry, whatever the
+    // data -- if it is spread evenly: a pass over the distribution's last
+    // prefixes misses SNPs with an effect in the middle, and then every
+    // combination with one of them passes (triples of 1,201 x 7,013, top-50:
+    // 24 to 28 ms per search with such a pass, 11 with an even one).  S = 128, with at least
+    // 32,768 combinations and at most 2^23, but as many as keep the expected
+    // candidates within an eighth of their buffer.
+    const bool tup_sample = sample && (tup || (algo == FIU_ALGO_MFMA && d->cases < (1u << 16) &&
+                                               d->ctrls < (1u << 16) && mfma_fp4 && ws.tuples(d, order - 1, false, s)));
+    const double sample_want =
+        std::min(std::max({combos_est / 128.0, 32768.0, 8.0 * (double)outputs * combos_est / (double)cap}),
+                 std::max(8388608.0, 2.0 * (double)outputs * combos_est / (double)cap));
+    int64_t sample_step = std::max<int64_t>(1, (int64_t)(combos_est / std::max(std::min(sample_want, (double)target), 1.0)));
+    // Without the tuple kernels the popcount scan samples the share (step x
+    // sample_step) of the prefixes, at 5-12x the matrix cores' cost per
+    // combination; where that leaves too few prefixes to fill the device, the
+    // distribution's last ones, which have the fewest last SNPs.
+    if (!tup_sample && algo == FIU_ALGO_MFMA) sample_step = std::max<int64_t>(sample_step, 256);
+    const bool layered = sample && !tup_sample && (int64_t)n_pref / sample_step >= 1024;
     const int64_t sample_prefixes =
-        plan.count == 0 || !sample || tup
+        !sample || tup_sample || layered
             ? 0
             : tail_prefixes(n, M, (uint64_t)step, (uint64_t)offset, total_prefixes, (int64_t)n_pref,
-                            std::min<uint64_t>({1ull << 24, target, sample_cap}));
+                            std::min<uint64_t>(target, (uint64_t)std::max(16384.0, combos_est / (double)sample_step)));
     Cand *cand = nullptr, *top = nullptr;
     TopState *state = nullptr;
     uint32_t *redo = nullptr, *hist = nullptr;
@@ -1113,7 +1122,7 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     };
     Cand *mwork = big_merge ? ws.merge_work(d, pow2_at_least((uint64_t)outputs + cap)) : nullptr;
     // state reset and (when sampling) histogram cleared in one launch
-    const bool sampled = sample_prefixes > 0 || (tup && sample && plan.count > 0);
+    const bool sampled = tup_sample || layered || sample_prefixes > 0;
     check(launch_search_begin(state, sampled ? hist : nullptr, s), "search start launch");
 
     ScanParams P{};
@@ -1129,10 +1138,11 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     P.cells = order >= kMinBigOrder ? ws.big_cells(d, order) : nullptr;
     mi_constants(d->cases, d->ctrls, d->complete(), P);
     TupleArgs TA{};
-    if (tup) {
+    if (tup || tup_sample) {
         TA.F = tuple_image(d, tup_all);
         for (int j = 1; j < order && !tup_all; ++j) TA.T.t[j] = d->tup[j].p;
         TA.stride = 1;
+        TA.tile_stride = 1;
         TA.fill = kTupleFill;
     }
 
@@ -1181,31 +1191,41 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
         }
         ++st.launches;
     };
-    if (sample_prefixes > 0) {
+    if (sampled) {
         ScanParams H = P;
-        H.j0 = (int64_t)n_pref - sample_prefixes;
-        H.j1 = (int64_t)n_pref;
         H.hist = hist;
-        if (algo == FIU_ALGO_MARGINAL && order >= 4)
-            check(launch_scan_km(order, d->dev, H, state, s), "sample launch");
-        else if (algo == FIU_ALGO_MARGINAL || algo == FIU_ALGO_MFMA)
-            check(launch_scan_marginal(order, d->dev, H, state, s), "sample launch");
-        else
-            check(launch_scan_direct(order, d->dev, H, state, s), "sample launch");
-        check(launch_tau_from_hist(hist, outputs, P.delta, state, s), "threshold launch");
-    } else if (sampled) {
-        // the same kernel over evenly spaced units: about 1/128 of the
-        // combinations (they cost what the scan's do), at least the floor
-        const double want = std::min(std::max((double)sample_floor, combos_est / 128.0), (double)target);
-        const double frac = std::min(1.0, want / std::max(combos_est, 1.0));
-        const int64_t count = std::max<int64_t>(1, (int64_t)std::ceil((double)tup_units * frac));
-        ScanParams H = P;
-        TupleArgs B = TA;
-        B.stride = std::max<int64_t>(1, tup_units / count);
-        H.j0 = B.stride / 2;
-        H.j1 = tup_units;
-        H.hist = hist;
-        check(launch_tuples(order, tup_all, d->dev, H, state, B, s), "sample launch");
+        if (tup_sample) {
+            // one unit in `stride`, and of its tiles one in `tile_stride`
+            TupleArgs B = TA;
+            const int64_t units = order == 2 ? ((int64_t)n_pref + tuple_b_block(2, tup_all) - 1) / tuple_b_block(2, tup_all)
+                                             : (int64_t)binom_sat((uint64_t)n, (uint64_t)order - 2);
+            // (about 32 tiles of an order-3 head, so that many heads are seen)
+            const int64_t head_tiles = (int64_t)((n + 63) / 64) * ((n + 63) / 64) / 2;
+            const int64_t tiles = order == 2   ? sample_step
+                                  : order == 3 ? std::min(sample_step, std::max<int64_t>(2, head_tiles / 32))
+                                               : 1;
+            B.tile_stride = (int32_t)std::min<int64_t>(tiles, 1 << 20);
+            B.stride = std::max<int64_t>(1, std::min(sample_step / tiles, units));
+            H.j0 = B.stride / 2;
+            H.j1 = units;
+            check(launch_tuples(order, tup_all, d->dev, H, state, B, s), "sample launch");
+        } else {
+            if (layered) {
+                H.step = (int64_t)step * sample_step;
+                H.offset = (int64_t)offset + (int64_t)step * (sample_step / 2);
+                H.j0 = 0;
+                H.j1 = ((int64_t)n_pref - sample_step / 2 + sample_step - 1) / sample_step;
+            } else {
+                H.j0 = (int64_t)n_pref - sample_prefixes;
+                H.j1 = (int64_t)n_pref;
+            }
+            if (algo == FIU_ALGO_MARGINAL && order >= 4)
+                check(launch_scan_km(order, d->dev, H, state, s), "sample launch");
+            else if (algo == FIU_ALGO_MARGINAL || algo == FIU_ALGO_MFMA)
+                check(launch_scan_marginal(order, d->dev, H, state, s), "sample launch");
+            else
+                check(launch_scan_direct(order, d->dev, H, state, s), "sample launch");
+        }
         check(launch_tau_from_hist(hist, outputs, P.delta, state, s), "threshold launch");
     }
     for (uint64_t ci = 0; ci < plan.count; ++ci) run_chunk(ci, true);

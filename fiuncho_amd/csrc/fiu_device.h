@@ -93,10 +93,12 @@ __host__ __device__ inline uint64_t big_cells_bytes(int order)
     return (uint64_t)big_slots(order) * 2 * c * sizeof(uint32_t);
 }
 
-// Histogram of screening MI values by the top 12 bits of their float image
-// (sign, exponent, 3 mantissa bits): monotone for non-negative values, so the
-// N-th best bin bounds the N-th best value from below.
+// Histogram of MI values by the exponent and the top 7 mantissa bits of their
+// float image, from 2^-24 up (bins 0.8 % wide; bin 0 also holds everything
+// below): monotone, so the N-th best bin bounds the N-th best value from
+// below.
 constexpr int kHistBins = 4096;
+constexpr uint32_t kHistBase = (127u - 24u) << 7;
 __host__ __device__ inline uint32_t hist_bin(float v)
 {
     union {
@@ -104,7 +106,18 @@ __host__ __device__ inline uint32_t hist_bin(float v)
         uint32_t u;
     } x;
     x.f = v > 0.0f ? v : 0.0f;
-    return x.u >> 20;
+    const uint32_t b = x.u >> 16;
+    return b <= kHistBase ? 0 : b - kHistBase < kHistBins ? b - kHistBase : kHistBins - 1;
+}
+// Lower edge of a bin.
+__host__ __device__ inline float hist_edge(uint32_t bin)
+{
+    union {
+        float f;
+        uint32_t u;
+    } x;
+    x.u = bin == 0 ? 0u : (bin + kHistBase) << 16;
+    return x.f;
 }
 
 // ---------------------------------------------------------------------------

@@ -82,6 +82,7 @@ struct TupleArgs {
     TupleTables T;           // marginal scans: tables of fewer SNPs than the order
     uint32_t *out;           // set: write the order's table (orders 2, 3) instead of scoring
     int64_t stride;          // units j0, j0 + stride, .. of [j0, j1) (a sample), else 1
+    int32_t tile_stride;     // sampling: every tile_stride-th tile of a unit (>= 1)
     int64_t units;           // set by the launcher
     int32_t rounds;          // set by the launcher
     int32_t fill;            // workgroups that fill the device

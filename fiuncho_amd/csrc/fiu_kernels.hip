@@ -62,12 +62,7 @@ __global__ void __launch_bounds__(kTauThreads) k_tau_from_hist(const uint32_t *h
     for (int i = kTauPer - 1; i >= 0; --i) {
         cum += h[i];
         if (cum >= N) {
-            union {
-                uint32_t u;
-                float f;
-            } x;
-            x.u = (uint32_t)(t * kTauPer + i) << 20;
-            st->tau = x.f - delta;
+            st->tau = hist_edge((uint32_t)(t * kTauPer + i)) - delta;
             st->tau_combo = ~0ull;
             return;
         }
@@ -1622,15 +1617,14 @@ __device__ __forceinline__ void mfma2w_tile(const DevData &D, const ScanParams &
     });
     int taken = 0;
     while (__ballot(pend != 0)) {
-        bool want = false;
-        float mf = 0.0f;
-        uint64_t combo = ~0ull;
+        bool need = false;
+        int a = 0;
+        float m0[9], m1[9];
         if (pend) {
             const int i = __builtin_ctz(pend), ab = i >> 4, r = (i >> 2) & 3, q = i & 3;
             pend &= pend - 1;
-            const int a = a0 + 64 * wa + 32 * ab + 8 * r + 4 * (lane >> 5) + q;
+            a = a0 + 64 * wa + 32 * ab + 8 * r + 4 * (lane >> 5) + q;
             const v4i wd = marked[taken++];
-            float m0[9], m1[9];
             cells(
                 a,
                 [&](int cls, int g, int h) __attribute__((always_inline)) {
@@ -1638,10 +1632,10 @@ __device__ __forceinline__ void mfma2w_tile(const DevData &D, const ScanParams &
                     return (float)(cls ? v >> 16 : v & 0xffffu);
                 },
                 m0, m1);
-            screen_exact<9>(m0, m1, [&] { return prefix_key(P.binom, D.n, &a, 1) + (uint64_t)b; }, tau, tau_combo, P,
-                            want, mf, combo);
+            need = mi_screen<9>(m0, m1, P.hy, P.inv_n) >= tau - P.delta;
         }
-        push_candidates(want, mf, combo, P, st);
+        exact_push_arrays<9>(need, m0, m1, [&] { return prefix_key(P.binom, D.n, &a, 1) + (uint64_t)b; }, tau,
+                             tau_combo, P, st);
     }
 }
 
@@ -2274,16 +2268,15 @@ __device__ __forceinline__ void mfma3w_tile(const DevData &D, const ScanParams &
     });
     int taken = 0;
     while (__ballot(pend != 0)) {
-        bool want = false;
-        float mf = 0.0f;
-        uint64_t combo = ~0ull;
+        bool need = false;
+        int b = 0;
+        float m0[27], m1[27];
         if (pend) {
             const int i = __builtin_ctz(pend), bb = i >> 2, j = i & 3;
             pend &= pend - 1;
-            const int b = b0 + 16 * bb + 4 * (lane >> 4) + j;
+            b = b0 + 16 * bb + 4 * (lane >> 4) + j;
             const v4i w0 = marked[2 * taken], w1 = marked[2 * taken + 1];
             ++taken;
-            float m0[27], m1[27];
             m3_cells(
                 D, P, L, a, b,
                 [&](int cls, int x, int y, int z) __attribute__((always_inline)) {
@@ -2292,9 +2285,9 @@ __device__ __forceinline__ void mfma3w_tile(const DevData &D, const ScanParams &
                     return (float)(cls ? v >> 16 : v & 0xffffu);
                 },
                 m0, m1);
-            screen_exact<27>(m0, m1, [&] { return m3_key(P, D.n, a, b, L.c); }, tau, tau_combo, P, want, mf, combo);
+            need = mi_screen<27>(m0, m1, P.hy, P.inv_n) >= tau - P.delta;
         }
-        push_candidates(want, mf, combo, P, st);
+        exact_push_arrays<27>(need, m0, m1, [&] { return m3_key(P, D.n, a, b, L.c); }, tau, tau_combo, P, st);
     }
 }
 
@@ -2369,53 +2362,103 @@ __global__ void k_unpack_top(const Cand *top, uint32_t count, int order, int n, 
 // ---------------------------------------------------------------------------
 // Top-N merge (one workgroup): current list + candidates -> best N, unique.
 // ---------------------------------------------------------------------------
-// Sorts buf[0, L) (L a power of two, padded with empty entries) by key,
-// then writes the first N unique non-empty entries to top; returns how many
-// unique entries there were (all threads).
-__device__ __forceinline__ uint32_t sort_unique(Cand *buf, uint32_t L, Cand *top, uint32_t N, uint32_t *psum)
+// Inclusive prefix sum over the workgroup's 1024 threads (16 waves): a shuffle
+// scan per wave, then the sums of the waves before it (`part`: 16 words).
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t *part, uint32_t &total)
 {
-    const int tid = threadIdx.x;
-    for (uint32_t k = 2; k <= L; k <<= 1) {
-        for (uint32_t jj = k >> 1; jj > 0; jj >>= 1) {
-            for (uint32_t i = tid; i < L; i += 1024) {
-                const uint32_t ixj = i ^ jj;
-                if (ixj > i) {
-                    const Cand a = buf[i], b = buf[ixj];
-                    const bool desc = (i & k) == 0;
-                    const bool sw = desc ? better(b.mi, b.combo, a.mi, a.combo) : better(a.mi, a.combo, b.mi, b.combo);
-                    if (sw) { buf[i] = b; buf[ixj] = a; }
-                }
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t o = __shfl_up(v, off);
+        if (lane >= off) v += o;
+    }
+    __syncthreads();   // `part` may still be read from an earlier scan
+    if (lane == 63) part[w] = v;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const uint32_t s = part[i];
+        before += i < w ? s : 0;
+        all += s;
+    }
+    total = all;
+    return v + before;
+}
+
+// Sorts buf[0, m) by key, then writes the first N unique non-empty entries to
+// top; returns how many unique entries there were (all threads).  Up to 1,024
+// entries: every thread counts the entries ahead of its own (buf read in
+// order by all lanes at once, a broadcast) and places it in the buffer's
+// second half, two barriers in all; above: bitonic, a barrier per step.  The
+// merge of a pair search on 1,000 x 4,000 takes 14 us; sorting every
+// candidate in bitonic steps it took 119.
+constexpr uint32_t kRankSlots = 1024;
+static_assert(2 * kRankSlots <= (uint32_t)kMergeSlots, "two halves of the merge buffer");
+__device__ __forceinline__ uint32_t sort_unique(Cand *buf, uint32_t m, Cand *top, uint32_t N, uint32_t *psum)
+{
+    const uint32_t tid = threadIdx.x;
+    const Cand *sorted = buf;
+    if (m <= kRankSlots) {
+        if (tid < m) {
+            const Cand e = buf[tid];
+            uint32_t rank = 0;
+#pragma unroll 4
+            for (uint32_t j = 0; j < m; ++j) {
+                const Cand o = buf[j];
+                rank += better(o.mi, o.combo, e.mi, e.combo) || (o.mi == e.mi && o.combo == e.combo && j < tid);
             }
-            __syncthreads();
+            buf[kRankSlots + rank] = e;
+        }
+        sorted = buf + kRankSlots;
+        __syncthreads();
+    } else {
+        uint32_t L = 2;
+        while (L < m) L <<= 1;
+        for (uint32_t i = m + tid; i < L; i += 1024) {
+            Cand e;
+            e.mi = -INFINITY;
+            e.tag = 0;
+            e.combo = ~0ull;
+            buf[i] = e;
+        }
+        __syncthreads();
+        for (uint32_t k = 2; k <= L; k <<= 1) {
+            for (uint32_t jj = k >> 1; jj > 0; jj >>= 1) {
+                for (uint32_t i = tid; i < L; i += 1024) {
+                    const uint32_t ixj = i ^ jj;
+                    if (ixj > i) {
+                        const Cand a = buf[i], b = buf[ixj];
+                        const bool desc = (i & k) == 0;
+                        const bool sw =
+                            desc ? better(b.mi, b.combo, a.mi, a.combo) : better(a.mi, a.combo, b.mi, b.combo);
+                        if (sw) { buf[i] = b; buf[ixj] = a; }
+                    }
+                }
+                __syncthreads();
+            }
         }
     }
     // unique, non-empty entries in order; contiguous segments per thread
-    const uint32_t seg = (L + 1023) / 1024;
-    const uint32_t s0 = min(L, tid * seg), s1 = min(L, s0 + seg);
+    const uint32_t seg = (m + 1023) / 1024;
+    const uint32_t s0 = min(m, tid * seg), s1 = min(m, s0 + seg);
     auto keep = [&](uint32_t i) {
-        const bool empty = buf[i].combo == ~0ull && buf[i].mi == -INFINITY;
-        const bool dup = i > 0 && buf[i].combo == buf[i - 1].combo && buf[i].mi == buf[i - 1].mi &&
-                         buf[i].tag == buf[i - 1].tag;
+        const Cand c = sorted[i];
+        const bool empty = c.combo == ~0ull && c.mi == -INFINITY;
+        const bool dup = i > 0 && c.combo == sorted[i - 1].combo && c.mi == sorted[i - 1].mi &&
+                         c.tag == sorted[i - 1].tag;
         return !empty && !dup;
     };
     uint32_t local = 0;
     for (uint32_t i = s0; i < s1; ++i) local += keep(i);
-    psum[tid] = local;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        const uint32_t v = tid >= off ? psum[tid - off] : 0;
-        __syncthreads();
-        psum[tid] += v;
-        __syncthreads();
-    }
-    uint32_t pos = psum[tid] - local;
+    uint32_t unique;
+    uint32_t pos = block_scan(local, psum, unique) - local;
     for (uint32_t i = s0; i < s1; ++i) {
         if (keep(i)) {
-            if (pos < N) top[pos] = buf[i];
+            if (pos < N) top[pos] = sorted[i];
             ++pos;
         }
     }
-    const uint32_t unique = psum[1023];
     __syncthreads();
     return unique;
 }
@@ -2435,7 +2478,7 @@ __device__ __forceinline__ void merge_topn(TopState *st, Cand *top, const Cand *
     const uint32_t count = min(st->cand_count, cap);
     uint32_t n_top = st->n_top;
     bool merged = false;
-    if (count > (uint32_t)kMergeSlots / 2 && N > 0) {
+    if (n_top + count > kRankSlots && N > 0 && n_top + count > 2 * N) {
         static_assert(kHistBins * sizeof(uint32_t) <= kMergeSlots * sizeof(Cand), "histogram in the merge buffer");
         static_assert(kHistBins == 4 * 1024, "four bins per thread");
         uint32_t *hist = (uint32_t *)buf;
@@ -2444,67 +2487,39 @@ __device__ __forceinline__ void merge_topn(TopState *st, Cand *top, const Cand *
         for (uint32_t i = tid; i < count; i += 1024) atomicAdd(&hist[hist_bin(cand[i].mi)], 1u);
         for (uint32_t i = tid; i < n_top; i += 1024) atomicAdd(&hist[hist_bin(top[i].mi)], 1u);
         __syncthreads();
-        // suffix sums over the threads' four-bin groups (thread t: bins 4t .. 4t + 3)
-        uint32_t grp[4], local = 0;
+        // thread t: bins 4t .. 4t + 3; entries in the bins above them
+        uint32_t grp[4], local = 0, all;
 #pragma unroll
         for (int q = 0; q < 4; ++q) local += grp[q] = hist[4 * tid + q];
-        psum[tid] = local;
+        const uint32_t through = block_scan(local, psum, all);
+        const uint32_t need = 2 * N, above = all - through;
+        if (tid == 0) psum[16] = 0;   // no pick: keep every bin
         __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            const uint32_t v = tid + off < 1024 ? psum[tid + off] : 0;
-            __syncthreads();
-            psum[tid] += v;
-            __syncthreads();
-        }
-        const uint32_t need = 2 * N;
-        const uint32_t above = tid + 1 < 1024 ? psum[tid + 1] : 0;   // entries in the bins of higher threads
-        int sel = -1;                                                   // this thread's pick, if it holds b
-        if (psum[tid] >= need && above < need) {
+        if (above < need && above + local >= need) {
             uint32_t acc = above;
+            int sel = -1;
             for (int q = 3; q >= 0 && sel < 0; --q) {
                 acc += grp[q];
                 if (acc >= need) sel = 4 * tid + q;
             }
+            psum[16] = (uint32_t)sel;
         }
         __syncthreads();
-        if (tid == 0) psum[0] = 0;   // no pick: keep every bin
-        __syncthreads();
-        if (sel >= 0) psum[0] = (uint32_t)sel;
-        __syncthreads();
-        const uint32_t bmin = psum[0];
-        __syncthreads();
+        const uint32_t bmin = psum[16];
         // compact the entries in bins >= bmin into buf (order is irrelevant:
         // they are sorted next); counts first, so that the total is known
         uint32_t mine = 0;
         for (uint32_t i = tid; i < count; i += 1024) mine += hist_bin(cand[i].mi) >= bmin;
         for (uint32_t i = tid; i < n_top; i += 1024) mine += hist_bin(top[i].mi) >= bmin;
-        psum[tid] = mine;
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            const uint32_t v = tid >= off ? psum[tid - off] : 0;
-            __syncthreads();
-            psum[tid] += v;
-            __syncthreads();
-        }
-        const uint32_t total = psum[1023];
-        if (total <= (uint32_t)kMergeSlots) {
-            uint32_t pos = psum[tid] - mine;
-            __syncthreads();   // the histogram (the start of buf) is read no more
+        uint32_t total;
+        uint32_t pos = block_scan(mine, psum, total) - mine;
+        if (total <= (uint32_t)kMergeSlots) {   // the histogram (the start of buf) is read no more
             for (uint32_t i = tid; i < n_top; i += 1024)
                 if (hist_bin(top[i].mi) >= bmin) buf[pos++] = top[i];
             for (uint32_t i = tid; i < count; i += 1024)
                 if (hist_bin(cand[i].mi) >= bmin) buf[pos++] = cand[i];
-            uint32_t L = 2;
-            while (L < total) L <<= 1;
-            for (uint32_t i = total + tid; i < L; i += 1024) {
-                Cand e;
-                e.mi = -INFINITY;
-                e.tag = 0;
-                e.combo = ~0ull;
-                buf[i] = e;
-            }
             __syncthreads();
-            n_top = min(N, sort_unique(buf, L, top, N, psum));
+            n_top = min(N, sort_unique(buf, total, top, N, psum));
             merged = true;
         }
         __syncthreads();
@@ -2512,17 +2527,9 @@ __device__ __forceinline__ void merge_topn(TopState *st, Cand *top, const Cand *
     for (uint32_t done = 0; !merged && done < count;) {
         const uint32_t take = min(count - done, (uint32_t)kMergeSlots - n_top);
         const uint32_t total = n_top + take;
-        uint32_t L = 2;
-        while (L < total) L <<= 1;
-        for (uint32_t i = tid; i < L; i += 1024) {
-            Cand e;
-            if (i < n_top) e = top[i];
-            else if (i < total) e = cand[done + (i - n_top)];
-            else { e.mi = -INFINITY; e.tag = 0; e.combo = ~0ull; }
-            buf[i] = e;
-        }
+        for (uint32_t i = tid; i < total; i += 1024) buf[i] = i < n_top ? top[i] : cand[done + (i - n_top)];
         __syncthreads();
-        n_top = min(N, sort_unique(buf, L, top, N, psum));
+        n_top = min(N, sort_unique(buf, total, top, N, psum));
         done += take;
     }
     __syncthreads();

@@ -236,27 +236,6 @@ __device__ __forceinline__ void mi_exact_part_fn(F &&cell, double n, double &hx,
     }
 }
 
-template <int CELLS>
-__device__ __forceinline__ void mi_exact_part(const uint32_t *a0, const uint32_t *a1, double n, double &hx,
-                                              double &hall)
-{
-    mi_exact_part_fn<CELLS>(
-        [&](int x, uint32_t &n0, uint32_t &n1) __attribute__((always_inline)) {
-            n0 = a0[x];
-            n1 = a1[x];
-        },
-        n, hx, hall);
-}
-
-template <int CELLS>
-__device__ __forceinline__ double mi_exact(const uint32_t *a0, const uint32_t *a1, double n, double hy)
-{
-#pragma clang fp contract(off)
-    double hx = 0.0, hall = 0.0;
-    mi_exact_part<CELLS>(a0, a1, n, hx, hall);
-    return hx + hy - hall;
-}
-
 __device__ __forceinline__ bool better(float ma, uint64_t ca, float mb, uint64_t cb)
 {
     return ma > mb || (ma == mb && ca < cb);
@@ -287,25 +266,95 @@ __device__ __forceinline__ void push_candidates(bool want, float mi, uint64_t co
     }
 }
 
-// Screening MI, then exact MI and the key test for the survivors (one lane's
-// combination; the push is separate).
-template <int CELLS, class T, class K>
-__device__ __forceinline__ void screen_exact(const T *a0, const T *a1, K &&key, float tau, uint64_t tau_combo,
-                                             const ScanParams &P, bool &want, float &mf, uint64_t &combo)
+__device__ __forceinline__ double readlane64(double v, int lane)
 {
-    const float ms = mi_screen<CELLS>(a0, a1, P.hy, P.inv_n);
-    if (ms >= tau - P.delta) {
-        if constexpr (std::is_same<T, uint32_t>::value) {
-            mf = (float)mi_exact<CELLS>(a0, a1, P.n64, P.hy64);
-        } else {
-            uint32_t u0[CELLS], u1[CELLS];
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(u >> 32), lane);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+// The exact MI of lane src's table by the whole wave: lane x computes the
+// three terms of cell x (64 cells at a time), then every lane runs the same
+// chain over them in cell order, so the value is mi_exact_part_fn's bit for bit.
+// cell(x, n0, n1) gives the calling lane's own counts.
+template <int CELLS, class F>
+__device__ __forceinline__ double mi_exact_wave(F &&cell, int src, double n, double hy)
+{
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & 63;
+    double hx = 0.0, hall = 0.0;
 #pragma unroll
-            for (int x = 0; x < CELLS; ++x) u0[x] = (uint32_t)a0[x], u1[x] = (uint32_t)a1[x];
-            mf = (float)mi_exact<CELLS>(u0, u1, P.n64, P.hy64);
+    for (int base = 0; base < CELLS; base += 64) {
+        const int m = CELLS - base < 64 ? CELLS - base : 64;
+        uint32_t c = 0, t = 0;
+#pragma unroll
+        for (int x = 0; x < m; ++x) {
+            uint32_t n0, n1;
+            cell(base + x, n0, n1);
+            n0 = (uint32_t)__builtin_amdgcn_readlane((int)n0, src);
+            n1 = (uint32_t)__builtin_amdgcn_readlane((int)n1, src);
+            if (lane == x) c = n0, t = n1;
         }
+        const double pc = (double)c / n, pt = (double)t / n, pa = pc + pt;
+        const double lc = plogp(pc), lt = plogp(pt), la = plogp(pa);
+#pragma unroll 1
+        for (int x = 0; x < m; ++x) {
+            hall -= readlane64(lc, x);
+            hall -= readlane64(lt, x);
+            hx -= readlane64(la, x);
+        }
+    }
+    return hx + hy - hall;
+}
+
+// Exact MI and the key test of the lanes that `need` them, and the push (all
+// 64 lanes call).  A lane alone takes 3 CELLS FP64 logarithms one after the
+// other, the wave three per table: up to kExactWave lanes are taken one by one
+// by the wave, more of them side by side.  What a small search waits for:
+// pairs of 1,000 x 4,000, scan 106 -> 47 us; triples of 151 x 1,203, 145 -> 73.
+constexpr int kExactWave = 12;
+template <int CELLS, class F, class K>
+__device__ __forceinline__ void exact_push(bool need, F &&cell, K &&key, float tau, uint64_t tau_combo,
+                                           const ScanParams &P, TopState *st)
+{
+    const uint64_t mask = __ballot(need);
+    if (mask == 0) return;
+    const int lane = threadIdx.x & 63;
+    float mf = 0.0f;
+    if (__popcll(mask) <= kExactWave) {
+        for (uint64_t m = mask; m; m &= m - 1) {
+            const int src = __builtin_ctzll(m);
+            const float v = (float)mi_exact_wave<CELLS>(cell, src, P.n64, P.hy64);
+            if (lane == src) mf = v;
+        }
+    } else if (need) {
+#pragma clang fp contract(off)
+        double hx = 0.0, hall = 0.0;
+        mi_exact_part_fn<CELLS>(cell, P.n64, hx, hall);
+        mf = (float)(hx + P.hy64 - hall);
+    }
+    uint64_t combo = ~0ull;
+    bool want = false;
+    if (need) {
         combo = key();
         want = better(mf, combo, tau, tau_combo);
     }
+    push_candidates(want, mf, combo, P, st);
+}
+
+// exact_push on tables held as two arrays (integers, or FP32 integers).
+template <int CELLS, class T, class K>
+__device__ __forceinline__ void exact_push_arrays(bool need, const T *a0, const T *a1, K &&key, float tau,
+                                                  uint64_t tau_combo, const ScanParams &P, TopState *st)
+{
+    exact_push<CELLS>(
+        need,
+        [&](int x, uint32_t &n0, uint32_t &n1) __attribute__((always_inline)) {
+            n0 = (uint32_t)a0[x];
+            n1 = (uint32_t)a1[x];
+        },
+        key, tau, tau_combo, P, st);
 }
 
 // Whether a valid combination passes the bound (always, without it).
@@ -323,11 +372,9 @@ template <int CELLS, class T, class K>
 __device__ __forceinline__ void score_and_push(bool valid, const T *a0, const T *a1, K &&key, float tau,
                                                uint64_t tau_combo, const ScanParams &P, TopState *st)
 {
-    bool want = false;
-    float mf = 0.0f;
-    uint64_t combo = ~0ull;
-    if (valid && bound_ok<CELLS>(a0, a1, tau, P)) screen_exact<CELLS>(a0, a1, key, tau, tau_combo, P, want, mf, combo);
-    push_candidates(want, mf, combo, P, st);
+    const bool need = valid && bound_ok<CELLS>(a0, a1, tau, P) &&
+                      mi_screen<CELLS>(a0, a1, P.hy, P.inv_n) >= tau - P.delta;
+    exact_push_arrays<CELLS>(need, a0, a1, key, tau, tau_combo, P, st);
 }
 
 // Uniform lookup of prefix j < j1: rank -> SNP indices, or an empty marker.

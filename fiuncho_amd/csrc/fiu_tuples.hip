@@ -406,39 +406,31 @@ __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P
     if constexpr (MODE == kScore) {
         // one marked combination per lane and round: screen, exact MI, push
         while (__ballot(pend != 0)) {
-            bool want = false;
-            float mf = 0.0f;
-            uint64_t combo = ~0ull;
+            bool need = false;
+            int pre[K - 1] = {};
+            uint32_t m[Z::cells];
             if (pend) {
                 const int i = __builtin_ctz(pend);
                 pend &= pend - 1;
                 const int b = (int)b_at(i);
-                uint32_t m[Z::cells];
                 cells_of(i, b, m);
-                auto cell = [&](int x, float &fc, float &ft) __attribute__((always_inline)) {
-                    fc = (float)(m[x] & 0xffffu);
-                    ft = (float)(m[x] >> 16);
-                };
-                const float ms = fmaf(screen_sum_fn<Z::cells>(cell), P.inv_n * 0.69314718f, P.hy);
-                if (ms >= tau - P.delta) {
-#pragma clang fp contract(off)
-                    double hx = 0.0, hall = 0.0;
-                    mi_exact_part_fn<Z::cells>(
-                        [&](int x, uint32_t &n0, uint32_t &n1) __attribute__((always_inline)) {
-                            n0 = m[x] & 0xffffu;
-                            n1 = m[x] >> 16;
-                        },
-                        P.n64, hx, hall);
-                    mf = (float)(hx + P.hy64 - hall);
-                    int pre[K - 1];
 #pragma unroll
-                    for (int q = 0; q < H; ++q) pre[q] = hd.s[q];
-                    pre[H] = b;
-                    combo = prefix_key(P.binom, n, pre, K - 1) + (uint64_t)c;
-                    want = better(mf, combo, tau, tau_combo);
-                }
+                for (int q = 0; q < H; ++q) pre[q] = hd.s[q];
+                pre[H] = b;
+                const float ms = fmaf(screen_sum_fn<Z::cells>([&](int x, float &fc, float &ft) __attribute__((always_inline)) {
+                                          fc = (float)(m[x] & 0xffffu);
+                                          ft = (float)(m[x] >> 16);
+                                      }),
+                                      P.inv_n * 0.69314718f, P.hy);
+                need = ms >= tau - P.delta;
             }
-            push_candidates(want, mf, combo, P, st);
+            exact_push<Z::cells>(
+                need,
+                [&](int x, uint32_t &n0, uint32_t &n1) __attribute__((always_inline)) {
+                    n0 = m[x] & 0xffffu;
+                    n1 = m[x] >> 16;
+                },
+                [&] { return prefix_key(P.binom, n, pre, K - 1) + (uint64_t)c; }, tau, tau_combo, P, st);
         }
     }
 }
@@ -449,7 +441,8 @@ __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P
 // workgroups.  Workgroup L runs on XCD L % 8: for 64 units in a row it takes
 // the same tile number, so that units resident on one XCD share their b and
 // c rows in its L2, then the next, so that the XCDs' shares of units with
-// few tiles even out.
+// few tiles even out.  Sampling takes every tile_stride-th tile of a unit,
+// starting elsewhere in each.
 template <int K, bool ALL, int MODE>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_tuples(const DevData D, const ScanParams P, TopState *st, const TupleArgs A)
@@ -463,13 +456,16 @@ k_tuples(const DevData D, const ScanParams P, TopState *st, const TupleArgs A)
     const Head<Z::H> hd = head_at<K>(P, D.n, K == 2 ? 0 : (uint64_t)u);
     hist_begin<MODE == kSample>(lds_hist);
     int64_t tile = first;
+    uint32_t pick = MODE == kSample ? (uint32_t)(u % A.tile_stride) * 5u + (uint32_t)first : 0;
     int64_t bmin = hd.b_first;
     if constexpr (K == 2) bmin += u * Z::BT * P.step;
     while (bmin < D.n - 1) {
         const int ct = (int)(D.n - 1 - bmin + 63) >> 6;   // 64-column tiles past bmin
         if (tile < ct) {
-            tuple_tile<K, ALL, MODE>(D, P, st, A, hd, (int)bmin, (int)bmin + 1 + 64 * (int)tile, lds, lds_hist);
+            if (MODE != kSample || pick % (uint32_t)A.tile_stride == 0)
+                tuple_tile<K, ALL, MODE>(D, P, st, A, hd, (int)bmin, (int)bmin + 1 + 64 * (int)tile, lds, lds_hist);
             tile += 8 * (int64_t)A.rounds;
+            pick += 8 * (uint32_t)A.rounds;
         } else {
             if constexpr (K == 2) break;
             tile -= ct;
