@@ -590,6 +590,8 @@ bool ensure_tuple_tables(fiu_dataset *d, int m, hipStream_t s)
     const uint64_t *binom = ensure_binom(d, std::max(m, 2), s);
     std::lock_guard<std::mutex> lk(d->prep_mu);
     const uint64_t n = d->snps;
+    // the kernels address an entry's (b, c) part with 32-bit byte offsets
+    if (m >= 2 && (binom_sat(n, 2) << (m + 2)) >> 32) return false;
     uint64_t bytes = 0;
     for (int j = d->tup_ready + 1; j <= m; ++j) {
         const uint64_t c = binom_sat(n, (uint64_t)j);
@@ -986,9 +988,9 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     // 2 and 3 (the whole-scan kernels would compute the other shares' tiles
     // too) and, every cell counted, orders 2 and 3 on datasets with uncalled
     // genotypes.  Measured against the popcount scans: order 4, 240 x 16,000,
-    // 33 ms against 478; share (8, 3) of order 3, 2,500 x 16,000, 40 ms
-    // against 110; with 1 % uncalled, order 3 on 601 x 6,007 5.9 ms against
-    // 16.9 and order 2 on 4,001 x 8,999 0.95 ms against 3.1
+    // 22 ms against 478; share (8, 3) of order 3, 2,500 x 16,000, 26 ms
+    // against 110; with 1 % uncalled, order 3 on 601 x 6,007 3.9 ms against
+    // 17.5 and order 2 on 4,001 x 8,999 0.87 ms against 3.2
     const bool tup_all = !d->dev.uniform;
     const bool tup_fits = tup_all ? order <= 3 : order == 4 || (order <= 3 && step > 1);
     const bool tup = tup_fits && (algo_req == FIU_ALGO_AUTO || (from_table && order >= 4)) &&

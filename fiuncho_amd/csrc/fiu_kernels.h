@@ -84,7 +84,7 @@ struct TupleArgs {
     int64_t stride;          // units j0, j0 + stride, .. of [j0, j1) (a sample), else 1
     int32_t tile_stride;     // sampling: every tile_stride-th tile of a unit (>= 1)
     int64_t units;           // set by the launcher
-    int32_t rounds;          // set by the launcher
+    int32_t rounds, nb, nc, aligned;   // set by the launcher
     int32_t fill;            // workgroups that fill the device
 };
 // Scores (or samples, P.hist) units [P.j0, P.j1): heads (order >= 3) or blocks

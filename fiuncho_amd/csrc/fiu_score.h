@@ -166,6 +166,10 @@ __device__ __forceinline__ float mi_screen(const T *a0, const T *a1, float hy, f
     return fmaf(screen_sum<CELLS>(a0, a1), inv_n * 0.69314718f, hy);
 }
 
+// v_mul_legacy_f32: the product, with 0 times anything 0 (the compiler's own
+// intrinsic, which has no builtin name).
+__device__ float fmul_legacy(float a, float b) __asm("llvm.amdgcn.fmul.legacy");
+
 // Upper bound on the MI in nats, one reciprocal per cell and no logarithm:
 // MI = KL(P_XY || P_X P_Y) <= ln(1 + chi2/N) <= chi2/N (Jensen's inequality
 // on E_P[P_XY / (P_X P_Y)]), and with two classes
@@ -181,8 +185,10 @@ __device__ __forceinline__ float mi_bound_fn(F &&cell, float frac_c, float chi_s
     for (int x = 0; x < CELLS; ++x) {
         float fc, fx;
         cell(x, fc, fx);
+        // an empty cell has d = 0, and 0 times its infinite reciprocal is 0 in
+        // the legacy product: no clamp of fx
         const float d = fmaf(-fx, frac_c, fc);
-        s = fmaf(d * d, __builtin_amdgcn_rcpf(fmaxf(fx, 1.0f)), s);
+        s = fmaf(fmul_legacy(d, __builtin_amdgcn_rcpf(fx)), d, s);
     }
     return s * chi_scale;
 }
