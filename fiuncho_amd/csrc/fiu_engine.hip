@@ -1008,7 +1008,7 @@ void Server::ingest_main()
             } else {
                 if (!j->ds) {
                     j->owned.reset(create_dataset(j->words.data(), j->snps, j->cw, j->tw, j->cases, j->ctrls,
-                                                  arena_.get(), ingest_stream_, false));
+                                                  arena_.get(), ingest_stream_));
                     j->ds = j->owned.get();
                     std::vector<uint64_t>().swap(j->words);
                 }

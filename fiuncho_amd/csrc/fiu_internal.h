@@ -165,7 +165,6 @@ struct fiu_dataset {
     fiu::Arena *arena = nullptr;   // set: every device buffer comes from it
     size_t snps = 0, cw = 0, tw = 0;
     uint32_t cases = 0, ctrls = 0;
-    std::vector<uint64_t> host_words;
     fiu::DBuf<uint4> bits;
     fiu::DBuf<uint32_t> singles;
     fiu::DBuf<uint32_t> flags;
@@ -216,8 +215,7 @@ namespace fiu {
 // SNP-minor layout, row popcounts, coverage flags).  `stream` null: the
 // dataset gets a stream of its own.  Memory from `arena` when given.
 fiu_dataset *create_dataset(const uint64_t *words, size_t snps, size_t cw, size_t tw, uint32_t cases,
-                            uint32_t ctrls, Arena *arena = nullptr, hipStream_t stream = nullptr,
-                            bool keep_host_words = true);
+                            uint32_t ctrls, Arena *arena = nullptr, hipStream_t stream = nullptr);
 
 // Pack a SNP-major genotype matrix on the device into the reference layout
 // (as RawFile::fill does; `reader_flush`: with the readers' re-flushed words

@@ -62,6 +62,9 @@ hipError_t launch_pack_words(const int8_t *geno, uint64_t snps, uint64_t samples
                              const uint8_t *zero, uint64_t *words, hipStream_t s);
 hipError_t launch_transpose(const uint64_t *src, uint4 *dst, int n, int n_pad, int cls, uint64_t cw, uint64_t tw,
                             int quads, uint64_t class_off, hipStream_t s);
+// Reference-layout words of SNPs [s0, s0 + count) from the device image.
+hipError_t launch_words(const DevData &D, uint64_t s0, uint64_t count, uint64_t cw, uint64_t tw, uint64_t *out,
+                        hipStream_t s);
 hipError_t launch_singles(const uint4 *bits, const DevData &D, uint32_t *singles, uint32_t *flags, hipStream_t s);
 hipError_t launch_combine_batch(const DevData &D, const int32_t *combos, int k, uint64_t n, uint64_t cw, uint64_t tw,
                                 uint64_t *out, hipStream_t s);

@@ -2938,6 +2938,16 @@ __device__ __forceinline__ uint64_t load_word(const uint4 *bits, const DevData &
     return (w & 1) ? ((uint64_t)v.z | ((uint64_t)v.w << 32)) : ((uint64_t)v.x | ((uint64_t)v.y << 32));
 }
 
+__global__ void k_words(DevData D, uint64_t s0, uint64_t count, uint64_t cw, uint64_t tw, uint64_t *out)
+{
+    const uint64_t id = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, per = 3 * (cw + tw);
+    if (id >= count * per) return;
+    const uint64_t r = id % per;
+    const int cls = r >= 3 * cw;
+    const uint64_t v = cls ? r - 3 * cw : r, W = cls ? tw : cw;
+    out[id] = load_word(D.bits, D, cls, (int)(v / W), (int)(s0 + id / per), v % W);
+}
+
 __global__ void k_combine_batch(const uint4 *__restrict__ bits, DevData D, const int32_t *combos, int k,
                                 uint64_t n, uint64_t cw, uint64_t tw, uint64_t *out)
 {
@@ -3304,6 +3314,15 @@ hipError_t launch_transpose(const uint64_t *src, uint4 *dst, int n, int n_pad, i
     if (!total) return hipSuccess;
     hipLaunchKernelGGL(k_transpose, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, src, dst, n, n_pad, cls,
                        cw, tw, quads, class_off);
+    return hipGetLastError();
+}
+
+hipError_t launch_words(const DevData &D, uint64_t s0, uint64_t count, uint64_t cw, uint64_t tw, uint64_t *out,
+                        hipStream_t s)
+{
+    const uint64_t total = count * 3 * (cw + tw);
+    if (!total) return hipSuccess;
+    hipLaunchKernelGGL(k_words, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, D, s0, count, cw, tw, out);
     return hipGetLastError();
 }
 
