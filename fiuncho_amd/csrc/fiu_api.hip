@@ -742,6 +742,117 @@ int64_t tail_prefixes(int n, int M, uint64_t step, uint64_t offset, uint64_t tot
     return m;
 }
 
+}  // namespace
+
+namespace fiu {
+
+ThresholdSample plan_sample(int order, int n, int64_t step, int64_t offset, uint64_t total_prefixes, int64_t n_pref,
+                            uint32_t outputs, uint32_t cap, uint64_t target, bool tup, bool matrix)
+{
+    // A sample of one combination in S lets about S x outputs of them past
+    // the starting threshold, each an FP64 MI and a merge entry, whatever the
+    // data -- if it is spread evenly: a pass over the distribution's last
+    // prefixes misses SNPs with an effect in the middle, and then every
+    // combination with one of them passes (triples of 1,201 x 7,013, top-50:
+    // 24 to 28 ms per search with such a pass, 11 with an even one).  S = 128,
+    // with at least 32,768 combinations and at most 2^23, but as many as keep
+    // the expected candidates within an eighth of their buffer.
+    ThresholdSample S;
+    const double combos = (double)n_pref * (double)(n - order + 1) / (double)order;
+    const double expect = (double)outputs * combos / (double)cap;
+    const double want = std::min(std::min(std::max({combos / 128.0, 32768.0, 8.0 * expect}),
+                                          std::max(8388608.0, 2.0 * expect)),
+                                 (double)target);
+    S.step = std::max<int64_t>(1, (int64_t)(combos / std::max(want, 1.0)));
+    S.tup = tup;
+    S.on = tup;
+    if (tup) return S;
+    // Without the tuple kernels the popcount scan samples the share (step x
+    // S.step) of the prefixes, at 5-12x the matrix cores' cost per
+    // combination; where that leaves too few prefixes to fill the device, the
+    // distribution's last ones, which have the fewest last SNPs.
+    if (matrix) S.step = std::max<int64_t>(S.step, 256);
+    S.layered = n_pref / S.step >= 1024;
+    if (!S.layered)
+        S.prefixes = tail_prefixes(n, order - 1, (uint64_t)step, (uint64_t)offset, total_prefixes, n_pref,
+                                   std::min<uint64_t>(target, (uint64_t)std::max(16384.0, combos / (double)S.step)));
+    S.on = S.layered || S.prefixes > 0;
+    return S;
+}
+
+void launch_sample(const ThresholdSample &S, const fiu_dataset *d, const ScanParams &P, int order, int algo,
+                   bool all_cells, int64_t n_pref, uint32_t *hist, uint32_t outputs, TopState *st, hipStream_t s)
+{
+    ScanParams H = P;
+    H.hist = hist;
+    if (S.tup) {
+        // one unit in `stride`, and of its tiles one in `tile_stride` (about
+        // 32 tiles of an order-3 head, so that many heads are seen)
+        TupleArgs B = tuple_args(d, order, all_cells);
+        const int64_t n = (int64_t)d->snps, units = tuple_units(order, all_cells, (uint64_t)n, n_pref);
+        const int64_t head_tiles = (n + 63) / 64 * ((n + 63) / 64) / 2;
+        const int64_t tiles = order == 2   ? S.step
+                              : order == 3 ? std::min(S.step, std::max<int64_t>(2, head_tiles / 32))
+                                           : 1;
+        B.tile_stride = (int32_t)std::min<int64_t>(tiles, 1 << 20);
+        B.stride = std::max<int64_t>(1, std::min(S.step / tiles, units));
+        H.j0 = B.stride / 2;
+        H.j1 = units;
+        check(launch_tuples(order, all_cells, d->dev, H, st, B, s), "sample launch");
+    } else {
+        if (S.layered) {
+            H.step = P.step * S.step;
+            H.offset = P.offset + P.step * (S.step / 2);
+            H.j0 = 0;
+            H.j1 = (n_pref - S.step / 2 + S.step - 1) / S.step;
+        } else {
+            H.j0 = n_pref - S.prefixes;
+            H.j1 = n_pref;
+        }
+        if (algo == FIU_ALGO_MARGINAL && order >= 4)
+            check(launch_scan_km(order, d->dev, H, st, s), "sample launch");
+        else if (algo == FIU_ALGO_MARGINAL || algo == FIU_ALGO_MFMA)
+            check(launch_scan_marginal(order, d->dev, H, st, s), "sample launch");
+        else
+            check(launch_scan_direct(order, d->dev, H, st, s), "sample launch");
+    }
+    check(launch_tau_from_hist(hist, outputs, P.delta, st, s), "threshold launch");
+}
+
+int64_t tuple_units(int order, bool all_cells, uint64_t n, int64_t n_pref)
+{
+    const int bt = tuple_b_block(2, all_cells);
+    return order == 2 ? (n_pref + bt - 1) / bt : (int64_t)binom_sat(n, (uint64_t)order - 2);
+}
+
+TupleArgs tuple_args(const fiu_dataset *d, int order, bool all_cells)
+{
+    TupleArgs A{};
+    A.F = tuple_image(d, all_cells);
+    for (int j = 1; j < order && !all_cells; ++j) A.T.t[j] = d->tup[j].p;
+    A.stride = 1;
+    A.tile_stride = 1;
+    A.fill = kTupleFill;
+    return A;
+}
+
+// Its tables, launches and half-empty tiles cost a few tenths of a
+// millisecond: measured at order 4 on 60 SNPs x 4,000 samples (2.0e9
+// combinations x samples) 0.88 ms against 1.28, on 40 x 4,000 (3.7e8) 0.73
+// against 0.49; an order-3 share on 300 x 4,000 (4.5e9) 0.51 against 0.53, on
+// 150 x 4,000 (5.5e8) 0.39 against 0.38.
+bool tuple_scan(const fiu_dataset *d, int order, int64_t step, int64_t n_pref)
+{
+    const double n = (double)d->snps, combos = (double)n_pref * (n - order + 1) / order;
+    const bool fits = !d->dev.uniform ? order <= 3 : order == 4 || (order <= 3 && step > 1);
+    return fits && d->cases < (1u << 16) && d->ctrls < (1u << 16) && n >= 48 &&
+           combos * ((double)d->cases + (double)d->ctrls) >= 2e9;
+}
+
+}  // namespace fiu
+
+namespace {
+
 hipStream_t stream_of(const fiu_dataset *d, const fiu_config *cfg)
 {
     return cfg && cfg->stream ? (hipStream_t)cfg->stream : d->stream;
@@ -924,17 +1035,6 @@ class DatasetWorkspace final : public Workspace {
     const Cand *listed_ = nullptr;
 };
 
-// Whether the matrix-core scan around a head beats the popcount scan.  Its
-// tables, launches and half-empty tiles cost a few tenths of a millisecond:
-// measured at order 4 on 60 SNPs x 4,000 samples (2.0e9 combinations x
-// samples) 0.88 ms against 1.28, on 40 x 4,000 (3.7e8) 0.73 against 0.49; an
-// order-3 share on 300 x 4,000 (4.5e9) 0.51 against 0.53, on 150 x 4,000
-// (5.5e8) 0.39 against 0.38.
-bool tuple_scan_pays(int order, int n, double combos, uint64_t samples)
-{
-    return combos * (double)samples >= 2e9 && n >= 48;
-}
-
 // Exhaustive search of `d` in workspace `ws` (fiu_search, fiu_search_static).
 void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offset, uint32_t outputs,
             const fiu_config *cfg, int32_t *out_combos, float *out_mi, uint32_t *out_count, fiu_search_stats *stats)
@@ -1003,7 +1103,6 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     int algo = FIU_ALGO_DIRECT;
     const bool small_classes = d->cases < (1u << 24) && d->ctrls < (1u << 24);   // fp32-exact counts
     const double per_avg = (double)(n - M) / (double)(M + 1);
-    const double combos_est = (double)n_pref * per_avg;
     const uint64_t samples = (uint64_t)d->cases + d->ctrls;
     // matrix cores around a head of order - 2 SNPs: order 4, shares of orders
     // 2 and 3 (the whole-scan kernels would compute the other shares' tiles
@@ -1013,10 +1112,8 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     // against 110; with 1 % uncalled, order 3 on 601 x 6,007 3.9 ms against
     // 17.5 and order 2 on 4,001 x 8,999 0.87 ms against 3.2
     const bool tup_all = !d->dev.uniform;
-    const bool tup_fits = tup_all ? order <= 3 : order == 4 || (order <= 3 && step > 1);
-    const bool tup = tup_fits && (algo_req == FIU_ALGO_AUTO || (from_table && order >= 4)) &&
-                     d->cases < (1u << 16) && d->ctrls < (1u << 16) && tuple_scan_pays(order, n, combos_est, samples) &&
-                     ws.tuples(d, order - 1, tup_all, s);
+    const bool tup = (algo_req == FIU_ALGO_AUTO || (from_table && order >= 4)) &&
+                     tuple_scan(d, order, step, (int64_t)n_pref) && ws.tuples(d, order - 1, tup_all, s);
     if (algo_req != FIU_ALGO_DIRECT && d->dev.uniform && order >= 4 && order <= kMaxKmOrder)
         algo = FIU_ALGO_MARGINAL;
     if (algo_req != FIU_ALGO_DIRECT && d->dev.uniform && (order == 2 || order == 3)) {
@@ -1040,11 +1137,12 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     // order-3 matrix-core variants: 3 and 4 the 64 x 32 tile with rings of 3
     // and 4 stages, 5 and 6 the 64 x 64 tile (its counts wait as 16-bit
     // pairs: classes below 2^16 samples, else the 64 x 32 tile).  Default:
-    // 6 from 2,048 SNPs and 8,192 samples on (measured: the larger tile is
-    // 7 % faster on 10,000 x 16,000, slower on 2,000 x 4,000 and below, where
-    // its fewer workgroups and longer epilogue do not pay), else 4
+    // 6 from 768 SNPs on, else 4, whose finer tiles fill the device on fewer
+    // SNPs (scan ms, 4 / 6: 400 x 4,000 0.72 / 0.95, 800 x 3,000 2.15 / 2.08,
+    // 800 x 16,000 5.60 / 4.98, 1,201 x 7,013 11.45 / 11.47, 2,000 x 3,000
+    // 26.3 / 25.4, 2,000 x 8,000 44.3 / 38.4)
     int ring = algo == FIU_ALGO_MFMA && order == 3 && variant ? variant
-                                                              : (n >= 2048 && samples >= 8192 ? 6 : 4);
+                                                              : (n >= 768 ? 6 : 4);
     if (ring >= 5 && (d->cases >= (1u << 16) || d->ctrls >= (1u << 16) || !ws.private_memory())) ring = 4;
     // matrix-core scans walk super-blocks of 8 x 8 tiles of 64 x 64 pairs;
     // fp4 operands accumulate in fp32, exact while every count is below 2^24;
@@ -1056,11 +1154,13 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     // order-2 matrix-core variants: 1 int8 operands, 2 fp4 with the 64 x 64
     // tile, 3 fp4 with the 64 x 128 tile, 4 fp4 with the 128 x 128 tile (the
     // last two: 16-bit counts between the classes, so classes below 2^16
-    // samples, else 64 x 64).  Default: 4 from 16,384 SNPs and 8,192 samples
-    // on (measured on 50,000 x 32,000: 59.4 ms per scan, 61.2 with 3, 83.6
-    // with 2; slower below), else 2
-    const bool m2_big = variant == 0 && n >= 16384 && samples >= 8192;
-    const int m2_pick = variant == 4 || m2_big ? 2 : variant == 3 ? 1 : 0;
+    // samples, else 64 x 64).  Default from 8,192 samples on: 4 from 16,384
+    // SNPs, 3 from 8,192; else 2 (scan ms, 2 / 3 / 4: 50,000 x 32,000
+    // 83.6 / 61.2 / 59.4, 14,000 x 30,000 7.0 / 4.5 / 4.5, 10,000 x 16,000
+    // 1.59 / 1.45 / 1.65, 5,003 x 9,001 0.33 / 0.35 / 0.41, 20,000 x 2,000
+    // 1.44 / 1.67 / 1.94)
+    const bool m2_auto = variant == 0 && samples >= 8192;
+    const int m2_pick = variant == 4 || (m2_auto && n >= 16384) ? 2 : variant == 3 || (m2_auto && n >= 8192) ? 1 : 0;
     const int m2_tile = order == 2 && d->cases < (1u << 16) && d->ctrls < (1u << 16) && ws.private_memory()
                             ? m2_pick : 0;
 
@@ -1071,16 +1171,13 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     const uint64_t target = cfg && cfg->chunk_combos ? cfg->chunk_combos : (1ull << 28);
     const uint64_t max_chunks = ws.max_chunks();
     ChunkPlan plan;
-    // units of a scan around a head: the heads, or (order 2) blocks of b's
-    const int64_t tup_units =
-        !tup ? 0
-             : order == 2 ? ((int64_t)n_pref + tuple_b_block(2, tup_all) - 1) / tuple_b_block(2, tup_all)
-                          : (int64_t)binom_sat((uint64_t)n, (uint64_t)order - 2);
     if (tup) {
-        const double per_unit = combos_est / (double)std::max<int64_t>(tup_units, 1);
+        // heads, or (order 2) blocks of b's
+        const int64_t units = tuple_units(order, tup_all, (uint64_t)n, (int64_t)n_pref);
+        const double per_unit = (double)n_pref * per_avg / (double)std::max<int64_t>(units, 1);
         int64_t len = (int64_t)std::max<double>(1.0, (double)target / std::max(per_unit, 1.0));
-        len = std::max<int64_t>(len, (int64_t)(((uint64_t)tup_units + max_chunks - 1) / max_chunks));
-        plan.set_uniform(tup_units, len);
+        len = std::max<int64_t>(len, (int64_t)(((uint64_t)units + max_chunks - 1) / max_chunks));
+        plan.set_uniform(units, len);
     } else if (algo == FIU_ALGO_MFMA && order == 2) {
         // chunks of super-blocks (262,144 pairs each) instead of prefixes
         int64_t len = std::max<int64_t>(1, (int64_t)(target / (64 * 4096)));
@@ -1107,31 +1204,12 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     }
     if (plan.count > max_chunks) fail(FIU_ERR_UNSUPPORTED, "too many launches for this entry point");
     const bool sample = plan.count > 0 && !(cfg && (cfg->flags & FIU_FLAG_NO_THRESHOLD_SAMPLE));
-    // A sample of one combination in S lets about S x outputs of them past
-    // the starting threshold, each an FP64 MI and a merge entry, whatever the
-    // data -- if it is spread evenly: a pass over the distribution's last
-    // prefixes misses SNPs with an effect in the middle, and then every
-    // combination with one of them passes (triples of 1,201 x 7,013, top-50:
-    // 24 to 28 ms per search with such a pass, 11 with an even one).  S = 128, with at least
-    // 32,768 combinations and at most 2^23, but as many as keep the expected
-    // candidates within an eighth of their buffer.
     const bool tup_sample = sample && (tup || (algo == FIU_ALGO_MFMA && d->cases < (1u << 16) &&
                                                d->ctrls < (1u << 16) && mfma_fp4 && ws.tuples(d, order - 1, false, s)));
-    const double sample_want =
-        std::min(std::max({combos_est / 128.0, 32768.0, 8.0 * (double)outputs * combos_est / (double)cap}),
-                 std::max(8388608.0, 2.0 * (double)outputs * combos_est / (double)cap));
-    int64_t sample_step = std::max<int64_t>(1, (int64_t)(combos_est / std::max(std::min(sample_want, (double)target), 1.0)));
-    // Without the tuple kernels the popcount scan samples the share (step x
-    // sample_step) of the prefixes, at 5-12x the matrix cores' cost per
-    // combination; where that leaves too few prefixes to fill the device, the
-    // distribution's last ones, which have the fewest last SNPs.
-    if (!tup_sample && algo == FIU_ALGO_MFMA) sample_step = std::max<int64_t>(sample_step, 256);
-    const bool layered = sample && !tup_sample && (int64_t)n_pref / sample_step >= 1024;
-    const int64_t sample_prefixes =
-        !sample || tup_sample || layered
-            ? 0
-            : tail_prefixes(n, M, (uint64_t)step, (uint64_t)offset, total_prefixes, (int64_t)n_pref,
-                            std::min<uint64_t>(target, (uint64_t)std::max(16384.0, combos_est / (double)sample_step)));
+    const ThresholdSample TS =
+        sample ? plan_sample(order, n, step, offset, total_prefixes, (int64_t)n_pref, outputs, cap, target, tup_sample,
+                             algo == FIU_ALGO_MFMA)
+               : ThresholdSample{};
     Cand *cand = nullptr, *top = nullptr;
     TopState *state = nullptr;
     uint32_t *redo = nullptr, *hist = nullptr;
@@ -1145,8 +1223,7 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     };
     Cand *mwork = big_merge ? ws.merge_work(d, pow2_at_least((uint64_t)outputs + cap)) : nullptr;
     // state reset and (when sampling) histogram cleared in one launch
-    const bool sampled = tup_sample || layered || sample_prefixes > 0;
-    check(launch_search_begin(state, sampled ? hist : nullptr, s), "search start launch");
+    check(launch_search_begin(state, TS.on ? hist : nullptr, s), "search start launch");
 
     ScanParams P{};
     P.step = step;
@@ -1160,14 +1237,7 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     P.pair = d->pair_ready ? d->pair.p : nullptr;
     P.cells = order >= kMinBigOrder ? ws.big_cells(d, order) : nullptr;
     mi_constants(d->cases, d->ctrls, d->complete(), P);
-    TupleArgs TA{};
-    if (tup || tup_sample) {
-        TA.F = tuple_image(d, tup_all);
-        for (int j = 1; j < order && !tup_all; ++j) TA.T.t[j] = d->tup[j].p;
-        TA.stride = 1;
-        TA.tile_stride = 1;
-        TA.fill = kTupleFill;
-    }
+    const TupleArgs TA = tup ? tuple_args(d, order, tup_all) : TupleArgs{};
 
     size_t ev = 0;
     bool timed = true;
@@ -1214,43 +1284,7 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
         }
         ++st.launches;
     };
-    if (sampled) {
-        ScanParams H = P;
-        H.hist = hist;
-        if (tup_sample) {
-            // one unit in `stride`, and of its tiles one in `tile_stride`
-            TupleArgs B = TA;
-            const int64_t units = order == 2 ? ((int64_t)n_pref + tuple_b_block(2, tup_all) - 1) / tuple_b_block(2, tup_all)
-                                             : (int64_t)binom_sat((uint64_t)n, (uint64_t)order - 2);
-            // (about 32 tiles of an order-3 head, so that many heads are seen)
-            const int64_t head_tiles = (int64_t)((n + 63) / 64) * ((n + 63) / 64) / 2;
-            const int64_t tiles = order == 2   ? sample_step
-                                  : order == 3 ? std::min(sample_step, std::max<int64_t>(2, head_tiles / 32))
-                                               : 1;
-            B.tile_stride = (int32_t)std::min<int64_t>(tiles, 1 << 20);
-            B.stride = std::max<int64_t>(1, std::min(sample_step / tiles, units));
-            H.j0 = B.stride / 2;
-            H.j1 = units;
-            check(launch_tuples(order, tup_all, d->dev, H, state, B, s), "sample launch");
-        } else {
-            if (layered) {
-                H.step = (int64_t)step * sample_step;
-                H.offset = (int64_t)offset + (int64_t)step * (sample_step / 2);
-                H.j0 = 0;
-                H.j1 = ((int64_t)n_pref - sample_step / 2 + sample_step - 1) / sample_step;
-            } else {
-                H.j0 = (int64_t)n_pref - sample_prefixes;
-                H.j1 = (int64_t)n_pref;
-            }
-            if (algo == FIU_ALGO_MARGINAL && order >= 4)
-                check(launch_scan_km(order, d->dev, H, state, s), "sample launch");
-            else if (algo == FIU_ALGO_MARGINAL || algo == FIU_ALGO_MFMA)
-                check(launch_scan_marginal(order, d->dev, H, state, s), "sample launch");
-            else
-                check(launch_scan_direct(order, d->dev, H, state, s), "sample launch");
-        }
-        check(launch_tau_from_hist(hist, outputs, P.delta, state, s), "threshold launch");
-    }
+    if (TS.on) launch_sample(TS, d, P, order, algo, tup_all, (int64_t)n_pref, hist, outputs, state, s);
     for (uint64_t ci = 0; ci < plan.count; ++ci) run_chunk(ci, true);
     // chunks whose candidates overflowed the buffer are scanned again with
     // the (higher) final threshold until none overflows

@@ -137,6 +137,7 @@ enum BatchKind : int32_t {
     kKindKm4 = 7,      // order 4, marginal in the last SNP (launch 3)
     kKindKm5 = 8,      // order 5, marginal in the last SNP (launch 3)
     kKindKm5All = 9,   // order 5, every cell counted (any dataset; launch 3)
+    kKindTuples = 10,  // scans around a head (k_tuples, a launch of its own per range)
 };
 
 // fp4 image of a dataset's genotype rows 0 and 1 (operands of the matrix-core

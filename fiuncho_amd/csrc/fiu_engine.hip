@@ -151,6 +151,9 @@ struct Job {
     int64_t n_pref = 0, next = 0, given = 0, seed = 1;
     double instr_per_prefix = 1.0;    // popcount kinds: cost of one prefix
     double instr_per_combo = 0.0;     // matrix-core kinds: cost of one combination
+    bool all_cells = false;           // kKindTuples: every cell counted
+    int64_t prefixes = 0;             // prefixes of the distribution (n_pref counts the kind's units)
+    ThresholdSample sample;           // pass that seeds the threshold before the first slice
     std::deque<std::pair<int64_t, int64_t>> redo;
     int inflight = 0;
     int slot = -1;
@@ -228,6 +231,7 @@ class Engine {
     DBuf<TopState> states_d_;
     DBuf<Cand> cand_d_, top_d_;
     DBuf<char> desc_d_;
+    DBuf<uint32_t> hist_d_;   // histogram of the sampling passes (one at a time on stream_)
     BatchJob *jobs_h_ = nullptr;
     TopState *init_h_ = nullptr;
     char *desc_h_[2] = {nullptr, nullptr};
@@ -279,6 +283,7 @@ Engine::Engine(int device, const EngineConfig &cfg, Clock::time_point epoch) : d
     cand_d_.alloc((size_t)A * cfg_.cand_cap);
     top_d_.alloc((size_t)A * kMaxOutputs);
     desc_d_.alloc(desc_bytes_);
+    hist_d_.alloc(kHistBins);
     jobs_h_ = pinned<BatchJob>(A);
     top_h_ = pinned<Cand>(kMaxOutputs);
     init_h_ = pinned<TopState>(1);
@@ -354,6 +359,7 @@ void Engine::plan_job(Job *j)
     j->rs.combinations = (j->step == 1 && j->offset == 0)
                              ? binom_sat((uint64_t)n, (uint64_t)order)
                              : count_combinations((uint64_t)n, M, (uint64_t)j->step, (uint64_t)j->offset);
+    j->prefixes = j->n_pref;
     // the matrix cores take order 2 (any distribution: the tiles mask other
     // shares) and whole order-3 scans, as the single search does by default
     const int T = d->dev.n_pad / 64;
@@ -363,6 +369,36 @@ void Engine::plan_job(Job *j)
     const bool has_te = tuned(order, d->snps, (uint64_t)d->cases + d->ctrls, te);
     const int tuned_algo = has_te ? te.algorithm : FIU_ALGO_AUTO;
     const double unit_instr = has_te && te.batch_unit ? 40000.0 * std::ldexp(1.0, (int)te.batch_unit - 3) : 40000.0;
+    // a scan around a head where the single search takes one and prepare_scan
+    // found room for its tables: launches of its own, a whole range each
+    // (order 4 on 160 SNPs x 5,000 samples: the popcount kind's persistent
+    // launches took 3.5 ms of a 17 ms batch)
+    const double quads = (double)d->dev.quads[0] + (double)d->dev.quads[1];
+    j->all_cells = !d->dev.uniform;
+    const bool tables = j->all_cells ? d->fp4x_ready : d->fp4_ready && d->tup_ready >= order - 1;
+    // the threshold is seeded as the single search's when the sampling kernel's
+    // tables are there and the scan is large enough to gain by it: its first
+    // slice is then the whole scan, not the doubling slices that raise the
+    // threshold from nothing
+    const double combos = (double)j->prefixes * (double)(n - M) / (double)(M + 1);
+    const bool sampled = tables && combos >= (double)(1 << 18) && d->cases < (1u << 16) && d->ctrls < (1u << 16);
+    auto sample = [&](bool matrix) {
+        if (!sampled) return;
+        j->sample = plan_sample(order, n, j->step, j->offset, total_prefixes, j->prefixes, j->outputs, 1u << 16,
+                                UINT64_MAX, true, matrix);
+        j->seed = j->n_pref;
+    };
+    if ((tuned_algo == FIU_ALGO_AUTO || order >= 4) && tables && tuple_scan(d, order, j->step, j->prefixes)) {
+        j->kind = kKindTuples;
+        j->pw = 1;
+        j->n_pref = tuple_units(order, j->all_cells, (uint64_t)n, j->prefixes);
+        const double per = combos / (double)std::max<int64_t>(j->n_pref, 1);
+        j->instr_per_prefix = per * (j->all_cells || order == 4 ? 0.4 * quads + 12.0 : 0.2 * quads + 4.0);
+        j->seed = 1;
+        sample(true);
+        j->rs.algorithm = j->all_cells ? FIU_ALGO_DIRECT : order == 2 ? FIU_ALGO_MFMA : FIU_ALGO_MARGINAL;
+        return;
+    }
     if ((tuned_algo == FIU_ALGO_AUTO || tuned_algo == FIU_ALGO_MFMA) && mfma_dataset(d) && d->fp4_ready &&
         (order == 2 || (order == 3 && d->pair_ready && j->step == 1))) {
         j->kind = order == 2 ? kKindMfma2 : kKindMfma3;
@@ -384,6 +420,7 @@ void Engine::plan_job(Job *j)
         // popcount kinds (measured: about 6x the popcount throughput)
         j->instr_per_combo = 0.15 * ((double)d->dev.quads[0] + (double)d->dev.quads[1]) + 3.0;
         j->seed = 1;
+        sample(true);
         j->rs.algorithm = FIU_ALGO_MFMA;
         return;
     }
@@ -401,7 +438,6 @@ void Engine::plan_job(Job *j)
     int cells = 1;
     for (int i = 0; i < order; ++i) cells *= marginal && order <= 3 ? 2 : 3;
     if (marginal && order >= 4) cells = cells / 3 * 2;
-    const double quads = (double)d->dev.quads[0] + (double)d->dev.quads[1];
     const double epi = marginal ? (order == 3 ? 600.0 : order >= 4 ? 400.0 : 200.0) : 300.0;
     const double per_tile = (double)cells * 8.0 * quads + epi;   // wave instructions per prefix and tile
     const int n_tiles = std::max(1, d->dev.n_pad / 64);
@@ -422,6 +458,25 @@ void Engine::plan_job(Job *j)
 // Scans the matrix cores would take (order 2, whole order-3 scans): their
 // datasets get the fp4 image when it fits.
 bool wants_fp4(const Job *j) { return j->order == 2 || (j->order == 3 && j->step == 1); }
+
+// Tables of the scans around a head and of the sampling pass (also run by
+// that kernel), for datasets outside an arena.
+void prepare_tuples(Job *j, hipStream_t s)
+{
+    fiu_dataset *d = j->ds;
+    const uint64_t n = d->snps;
+    if (d->arena || j->order > 4 || j->step < 1 || j->offset < 0 || n < (uint64_t)j->order || d->cases >= (1u << 16) ||
+        d->ctrls >= (1u << 16))
+        return;
+    const uint64_t all = binom_sat(n, (uint64_t)j->order - 1);
+    const uint64_t pref = all > (uint64_t)j->offset ? (all - (uint64_t)j->offset + (uint64_t)j->step - 1) / (uint64_t)j->step : 0;
+    if (pref > (uint64_t)INT64_MAX / 2) return;
+    if (!d->dev.uniform) {
+        if (tuple_scan(d, j->order, j->step, (int64_t)pref)) (void)ensure_tuple_image(d, s);
+    } else if (j->order <= 3 || tuple_scan(d, j->order, j->step, (int64_t)pref)) {
+        (void)ensure_tuple_tables(d, j->order - 1, s);
+    }
+}
 
 void prepare_fp4(Job *j, hipStream_t s)
 {
@@ -521,7 +576,14 @@ void Engine::activate(Job *j, int slot)
     check_range(jobs_d_.p + slot, sizeof(B), jobs_d_.p, jobs_d_.n * sizeof(BatchJob), "job upload");
     check_range(states_d_.p + slot, sizeof(TopState), states_d_.p, states_d_.n * sizeof(TopState), "state init");
     check(hipMemcpyAsync(jobs_d_.p + slot, &B, sizeof(B), hipMemcpyHostToDevice, stream_), "job upload");
-    check(hipMemcpyAsync(states_d_.p + slot, init_h_, sizeof(TopState), hipMemcpyHostToDevice, stream_), "state init");
+    if (j->sample.on) {
+        check(launch_search_begin(B.st, hist_d_.p, stream_), "state init");
+        launch_sample(j->sample, d, P, j->order, j->rs.algorithm, j->all_cells, j->prefixes, hist_d_.p, j->outputs, B.st,
+                      stream_);
+    } else {
+        check(hipMemcpyAsync(states_d_.p + slot, init_h_, sizeof(TopState), hipMemcpyHostToDevice, stream_),
+              "state init");
+    }
 }
 
 bool Engine::launch_step()
@@ -615,8 +677,15 @@ bool Engine::launch_step()
         R.est_instr += range_cost(j, a, b);
         return true;
     };
+    std::vector<std::tuple<Job *, int64_t, int64_t>> tuples;
     auto add_seg = [&](Job *j, int64_t a, int64_t b) {
         if (batch_mfma(j->kind)) return add_mseg(j, a, b);
+        if (j->kind == kKindTuples) {
+            tuples.emplace_back(j, a, b);
+            R.ranges.emplace_back(j, a, b);
+            R.est_instr += range_cost(j, a, b);
+            return true;
+        }
         const int L = j->kind == kKindDirect4 ? 1
                       : (j->kind == kKindKm4 || j->kind == kKindKm5 || j->kind == kKindKm5All) ? 2
                                                                                                  : 0;
@@ -697,6 +766,17 @@ bool Engine::launch_step()
                              hipMemcpyHostToDevice, stream_),
               "step descriptor");
     check(hipEventRecord(ev_start_[parity], stream_), "event");
+    uint64_t heads = 0;
+    for (auto &t : tuples) {
+        const Job *j = std::get<0>(t);
+        ScanParams P = jobs_h_[j->slot].P;
+        P.j0 = std::get<1>(t);
+        P.j1 = std::get<2>(t);
+        heads += (uint64_t)(P.j1 - P.j0);
+        check(launch_tuples(j->order, j->all_cells, j->ds->dev, P, jobs_h_[j->slot].st,
+                            tuple_args(j->ds, j->order, j->all_cells), stream_),
+              "scan launch");
+    }
     check(hipGraphLaunch(exec_, stream_), "step graph launch");
     check(hipEventRecord(ev_end_[parity], stream_), "event");
     check(hipMemcpyAsync(states_h_[parity], states_d_.p, (size_t)cfg_.max_active * sizeof(TopState),
@@ -706,7 +786,7 @@ bool Engine::launch_step()
     R.valid = true;
     ++step_no_;
     ++stats_.steps;
-    stats_.units += units[0] + units[1] + units[2] + 8 * munits;
+    stats_.units += units[0] + units[1] + units[2] + 8 * munits + heads;
     return true;
 }
 
@@ -1015,6 +1095,7 @@ void Server::ingest_main()
                 j->binom = ensure_binom(j->ds, j->order, ingest_stream_);
                 if (j->order == 3 && j->ds->dev.uniform) (void)ensure_pair_table(j->ds, ingest_stream_);
                 prepare_fp4(j, ingest_stream_);
+                prepare_tuples(j, ingest_stream_);
                 Engine::plan_job(j);
             }
         } catch (const Failure &e) {
@@ -1180,7 +1261,8 @@ fiu_status fiu_search_batch(fiu_scan *scans, size_t n, const fiu_batch_config *c
     return guard([&] {
         if (!scans && n) fail(FIU_ERR_INVALID, "scans is NULL");
         const auto t0 = Clock::now();
-        const EngineConfig ec = engine_config(cfg, 24.0);
+        EngineConfig ec = engine_config(cfg, 24.0);
+        ec.max_active = (int)std::min<size_t>((size_t)ec.max_active, std::max<size_t>(n, 1));
         std::vector<std::unique_ptr<Job>> jobs;
         int device = -1;
         for (size_t i = 0; i < n; ++i) {
@@ -1226,6 +1308,7 @@ fiu_status fiu_search_batch(fiu_scan *scans, size_t n, const fiu_batch_config *c
                 j->binom = ensure_binom(j->ds, j->order, eng.prep_stream());
                 if (j->order == 3 && j->ds->dev.uniform) (void)ensure_pair_table(j->ds, eng.prep_stream());
                 prepare_fp4(j, eng.prep_stream());
+                prepare_tuples(j, eng.prep_stream());
                 Engine::plan_job(j);
             } catch (const Failure &e) {
                 j->scan->status = e.status;

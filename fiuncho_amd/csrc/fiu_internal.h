@@ -282,6 +282,24 @@ bool ensure_tuple_tables(fiu_dataset *d, int m, hipStream_t s);
 Fp4Image tuple_image(const fiu_dataset *d, bool all_cells);
 // Workgroups of such a scan that keep the device busy through its tail.
 constexpr int32_t kTupleFill = 16384;
+// Whether a scan around a head is the faster one for an AUTO search of these
+// n_pref prefixes; its units (heads, or at order 2 blocks of b's); its
+// arguments once ensure_tuple_tables / ensure_tuple_image succeeded.
+bool tuple_scan(const fiu_dataset *d, int order, int64_t step, int64_t n_pref);
+int64_t tuple_units(int order, bool all_cells, uint64_t n, int64_t n_pref);
+TupleArgs tuple_args(const fiu_dataset *d, int order, bool all_cells);
+
+// The pass that seeds a search's threshold: which combinations it screens,
+// and its launches (histogram, then the threshold in st).  `tup`: by a scan
+// around a head (tables or image ready), else by the popcount kernels.
+struct ThresholdSample {
+    bool on = false, tup = false, layered = false;
+    int64_t step = 1, prefixes = 0;
+};
+ThresholdSample plan_sample(int order, int n, int64_t step, int64_t offset, uint64_t total_prefixes, int64_t n_pref,
+                            uint32_t outputs, uint32_t cap, uint64_t target, bool tup, bool matrix);
+void launch_sample(const ThresholdSample &S, const fiu_dataset *d, const ScanParams &P, int order, int algo,
+                   bool all_cells, int64_t n_pref, uint32_t *hist, uint32_t outputs, TopState *st, hipStream_t s);
 // The dataset admits the matrix-core scans: every SNP covers the same samples
 // (the counts of the other cells follow by inclusion-exclusion) and both
 // classes are below 2^24 samples (FP32 counts are exact).

@@ -2663,6 +2663,7 @@ k_batch_scan(const BatchJob *__restrict__ jobs, const BatchSeg *__restrict__ seg
 {
     const int lane = threadIdx.x & 63;
     const uint32_t nseg = hdr->nseg[LAUNCH], units = hdr->units[LAUNCH];
+    if (units == 0) return;   // no counter traffic from a launch without work
     for (;;) {
         uint32_t u = 0;
         if (lane == 0) u = atomicAdd(&hdr->head[LAUNCH], 1u);
@@ -2731,6 +2732,7 @@ k_batch_mfma(const BatchJob *__restrict__ jobs, const BatchSeg *__restrict__ seg
     __shared__ uint32_t unit_sh;
     const int x = blockIdx.x & 7;
     const uint32_t nseg = hdr->mseg, units = hdr->munits;
+    if (units == 0) return;
     for (;;) {
         if (threadIdx.x == 0) unit_sh = atomicAdd(&hdr->mhead[x], 1u);
         __syncthreads();
