@@ -13,7 +13,6 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -153,34 +152,6 @@ void finish_upload(fiu_dataset *d, const uint64_t *words)
     D.total[1] = fl[2];
 }
 
-// Copy of caller memory to a new device buffer.  The runtime pins pageable
-// memory piece by piece as it copies; a second thread with the second half
-// overlaps that with the first half's transfer (160 MB: 5.5 ms by one thread,
-// 3.7 by two, 3.9 by four; pinned memory would take 2.9).
-void host_to_device(void *dst, const void *src, size_t bytes, fiu_dataset *d)
-{
-    if (!bytes) return;
-    constexpr size_t kSplit = 32u << 20;
-    const size_t half = bytes >= kSplit && !d->arena ? bytes / 2 / 4096 * 4096 : 0;
-    hipError_t other = hipSuccess;
-    std::thread helper;
-    if (half) {
-        try {
-            helper = std::thread([&] {
-                other = hipSetDevice(d->device);
-                if (other == hipSuccess) other = hipMemcpy(dst, src, half, hipMemcpyHostToDevice);
-            });
-        } catch (const std::system_error &) {   // no thread to be had: one copy
-        }
-    }
-    const size_t from = helper.joinable() ? half : 0;
-    const hipError_t e = hipMemcpyAsync((char *)dst + from, (const char *)src + from, bytes - from,
-                                        hipMemcpyHostToDevice, d->stream);
-    if (helper.joinable()) helper.join();
-    check(other, "upload");
-    check(e, "upload");
-}
-
 void upload(fiu_dataset *d, const uint64_t *words, hipStream_t stream)
 {
     bind_stream(d, stream);
@@ -188,7 +159,7 @@ void upload(fiu_dataset *d, const uint64_t *words, hipStream_t stream)
     DBuf<uint64_t> staging;
     staging.arena = d->arena;
     staging.alloc(nwords);
-    host_to_device(staging.p, words, nwords * 8, d);
+    if (nwords) check(hipMemcpyAsync(staging.p, words, nwords * 8, hipMemcpyHostToDevice, d->stream), "upload");
     finish_upload(d, staging.p);
 }
 
@@ -277,7 +248,9 @@ fiu_dataset *dataset_from_genotypes(const int8_t *geno, size_t snps, size_t samp
         DBuf<uint8_t> dz;
         g.arena = di.arena = dz.arena = d->arena;
         g.alloc((snps * samples + 15) / 16 * 16);   // the kernel reads whole 16-byte blocks
-        host_to_device(g.p, geno, snps * samples, d.get());
+        // (one copy: two threads with half each took 3.7 ms for 160 MB against
+        // 5.5 alone, but on some calls 11)
+        check(hipMemcpyAsync(g.p, geno, snps * samples, hipMemcpyHostToDevice, d->stream), "genotype upload");
         if (!runs) {
             di.alloc(samples);
             check(hipMemcpyAsync(di.p, idx.data(), samples * 4, hipMemcpyHostToDevice, d->stream), "sample lists");
@@ -412,7 +385,7 @@ fiu_dataset *stage_dataset(const uint64_t *words, size_t snps, size_t cw, size_t
         d->pair.arena = arena;
         if (pair_table_bytes(snps) <= arena->largest_free()) {
             try {
-                d->pair.alloc(snps * (snps - 1) / 2 * 8);
+                d->pair.alloc(pair_words(snps));
                 up.pair = true;
                 d->pair_ready = true;   // in stream order, before any scan of it
             } catch (const Failure &) {
@@ -420,7 +393,7 @@ fiu_dataset *stage_dataset(const uint64_t *words, size_t snps, size_t cw, size_t
             }
         }
     }
-    if (want_fp4 && mfma_dataset(d.get()) && (order == 2 || (order == 3 && up.pair))) {
+    if (want_fp4 && mfma_dataset(d.get()) && (order == 2 || (order == 3 && up.pair && mfma3_dataset(d.get())))) {
         const size_t units = fp4_image_units(D, 0) + fp4_image_units(D, 1);
         if (units * 16 <= arena->largest_free()) {
             try {
@@ -460,7 +433,7 @@ void enqueue_upload(fiu_dataset *d, StagedUpload &up, hipStream_t s)
         P.offset = 0;
         P.total_prefixes = d->snps;
         P.binom = d->binom.p;
-        check(launch_pair_table(d->dev, P, d->pair.p, s), "pair table launch");
+        check(launch_pair_table(d->dev, P, pair_table(d), s), "pair table launch");
     }
     if (up.fp4) check(launch_fp4_image(d->dev, d->fp4.p, s), "fp4 image launch");
 }
@@ -533,15 +506,15 @@ bool ensure_pair_table(fiu_dataset *d, hipStream_t s)
     const uint64_t *binom = ensure_binom(d, 1, s);
     std::lock_guard<std::mutex> lk(d->prep_mu);
     if (d->pair_ready) return true;
-    const uint64_t n = d->snps, pairs = n * (n - 1) / 2;
+    const uint64_t n = d->snps, bytes = pair_words(n) * 4;
     if (d->arena) {
-        if (pairs * 32 > d->arena->largest_free()) return false;
+        if (bytes > d->arena->largest_free()) return false;
     } else {
         size_t free_b = 0, total_b = 0;
         check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-        if (pairs * 32 + (64ull << 20) > free_b) return false;
+        if (bytes + (64ull << 20) > free_b) return false;
     }
-    d->pair.alloc(pairs * 8);
+    d->pair.alloc(pair_words(n));
     ScanParams P{};
     P.j0 = 0;
     P.j1 = (int64_t)n;
@@ -549,7 +522,7 @@ bool ensure_pair_table(fiu_dataset *d, hipStream_t s)
     P.offset = 0;
     P.total_prefixes = n;
     P.binom = binom;
-    check(launch_pair_table(d->dev, P, d->pair.p, s), "pair table launch");
+    check(launch_pair_table(d->dev, P, pair_table(d), s), "pair table launch");
     check(hipStreamSynchronize(s), "pair table sync");
     d->pair_ready = true;
     return true;
@@ -1125,7 +1098,7 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
         // order 3: the matrix-core scan walks every (b, c) of its first SNPs,
         // so by default it takes whole scans (a round-robin share of the
         // prefixes is masked, which wastes the other shares' work)
-        if (order == 3 && algo == FIU_ALGO_MARGINAL && small_classes &&
+        if (order == 3 && algo == FIU_ALGO_MARGINAL && mfma3_dataset(d) &&
             (algo_req == FIU_ALGO_MFMA || (algo_req == FIU_ALGO_AUTO && step == 1)) && ws.fp4_image(d, s))
             algo = FIU_ALGO_MFMA;
     }
@@ -1234,7 +1207,7 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     P.cand_cap = cap;
     P.order = order;
     P.tag = 0;
-    P.pair = d->pair_ready ? d->pair.p : nullptr;
+    P.pair = d->pair_ready ? pair_table(d) : nullptr;
     P.cells = order >= kMinBigOrder ? ws.big_cells(d, order) : nullptr;
     mi_constants(d->cases, d->ctrls, d->complete(), P);
     const TupleArgs TA = tup ? tuple_args(d, order, tup_all) : TupleArgs{};

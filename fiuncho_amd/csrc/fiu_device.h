@@ -76,7 +76,7 @@ struct ScanParams {
     uint32_t bounded;        // 1: complete genotype tables, the MI upper bound applies
     uint32_t tag;
     double hy64, n64;        // H(Y) and cases+ctrls in FP64
-    const uint32_t *pair;    // marginal pair table (order 3), or null
+    const uint32_t *pair;    // marginal pair table (order 3; pair_words), or null
     uint32_t *hist;          // threshold sampling pass: histogram of the
                              // screening MI (kHistBins bins), else null
     uint32_t *cells;         // orders 10-12: big_slots(order) slots of
@@ -187,6 +187,16 @@ struct BatchHeader {
     uint32_t munits;         // units of each XCD's queue in it
     uint32_t mhead[8];       // its per-XCD work counters (cleared by the graph)
 };
+
+// Marginal pair table: per pair 8 words, for (x, y) in {0, 1}^2 the case counts
+// f(x, y), then the case + control counts, as FP32 (exact below 2^24 samples;
+// the matrix-core epilogue reads them without a conversion); on datasets with
+// 2^24 samples or more integers, case counts then control counts.  kPairSlack
+// entries of padding on both sides: a tile's lanes past the last SNP, or with b
+// above c, read there and are dropped, with no select per address.
+__host__ __device__ inline bool pair_float(const DevData &D) { return (uint64_t)D.cases + D.ctrls < (1u << 24); }
+constexpr uint64_t kPairSlack = 4096;
+__host__ __device__ inline uint64_t pair_words(uint64_t n) { return ((n < 2 ? 0 : n * (n - 1) / 2) + 2 * kPairSlack) * 8; }
 
 __host__ __device__ inline uint64_t pair_index(int64_t b, int64_t c, int64_t n)
 {

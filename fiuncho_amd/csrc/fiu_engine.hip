@@ -400,7 +400,7 @@ void Engine::plan_job(Job *j)
         return;
     }
     if ((tuned_algo == FIU_ALGO_AUTO || tuned_algo == FIU_ALGO_MFMA) && mfma_dataset(d) && d->fp4_ready &&
-        (order == 2 || (order == 3 && d->pair_ready && j->step == 1))) {
+        (order == 2 || (order == 3 && d->pair_ready && j->step == 1 && mfma3_dataset(d)))) {
         j->kind = order == 2 ? kKindMfma2 : kKindMfma3;
         // the tile: a tuning entry's batch tile (batch_unit 1 = the 64 x 32 /
         // 64 x 64 tiles, 2 = the wide ones), else the sizes where the single
@@ -481,7 +481,7 @@ void prepare_tuples(Job *j, hipStream_t s)
 void prepare_fp4(Job *j, hipStream_t s)
 {
     fiu_dataset *d = j->ds;
-    if (wants_fp4(j) && mfma_dataset(d) && (j->order == 2 || d->pair_ready)) (void)ensure_fp4_image(d, s);
+    if (wants_fp4(j) && mfma_dataset(d) && (j->order == 2 || (d->pair_ready && mfma3_dataset(d)))) (void)ensure_fp4_image(d, s);
 }
 
 // Estimated cost of units [a, b) of a job.  Order 3 on the matrix cores: first
@@ -556,7 +556,7 @@ void Engine::activate(Job *j, int slot)
     P.cand_cap = cfg_.cand_cap;
     P.order = j->order;
     P.tag = (uint32_t)slot;
-    P.pair = (j->kind == kKindScan3m || j->kind == kKindMfma3) ? d->pair.p : nullptr;
+    P.pair = (j->kind == kKindScan3m || j->kind == kKindMfma3) ? pair_table(d) : nullptr;
     P.hist = nullptr;
     mi_constants(d->cases, d->ctrls, d->complete(), P);
     B.st = states_d_.p + slot;

@@ -267,7 +267,9 @@ const uint64_t *ensure_binom(fiu_dataset *d, int m, hipStream_t s);
 // pair).  Returns false when the table does not fit in free device memory
 // (hipMalloc datasets) or in the arena.
 bool ensure_pair_table(fiu_dataset *d, hipStream_t s);
-inline size_t pair_table_bytes(size_t snps) { return snps < 2 ? 0 : snps * (snps - 1) / 2 * 32; }
+inline size_t pair_table_bytes(size_t snps) { return snps < 2 ? 0 : pair_words(snps) * 4; }
+// The table's first pair.
+inline uint32_t *pair_table(const fiu_dataset *d) { return d->pair.p + kPairSlack * 8; }
 // fp4 image of genotype rows 0 and 1 (4 bits per sample and row); false when
 // it does not fit.
 bool ensure_fp4_image(fiu_dataset *d, hipStream_t s);
@@ -307,6 +309,8 @@ inline bool mfma_dataset(const fiu_dataset *d)
 {
     return d->dev.uniform && d->cases < (1u << 24) && d->ctrls < (1u << 24);
 }
+// Order 3 also reads the pair table as FP32 sums of both classes.
+inline bool mfma3_dataset(const fiu_dataset *d) { return mfma_dataset(d) && pair_float(d->dev); }
 
 // Top-N entries -> ascending SNP indices (order per entry, unranked from the
 // key among the k-combinations of n SNPs) and float MI.

@@ -854,8 +854,17 @@ __device__ __forceinline__ void scan2m_unit(const DevData &D, const ScanParams &
             if (TABLE) {
                 if (valid) {
                     uint4 *o = (uint4 *)(pair_out + pair_index(pa[i], c, D.n) * 8);
-                    o[0] = make_uint4(f[i][0][0], f[i][0][1], f[i][0][2], f[i][0][3]);
-                    o[1] = make_uint4(f[i][1][0], f[i][1][1], f[i][1][2], f[i][1][3]);
+                    if (pair_float(D)) {
+                        float *fo = (float *)o;
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+                            fo[x] = (float)f[i][0][x];
+                            fo[4 + x] = (float)(f[i][0][x] + f[i][1][x]);
+                        }
+                    } else {
+                        o[0] = make_uint4(f[i][0][0], f[i][0][1], f[i][0][2], f[i][0][3]);
+                        o[1] = make_uint4(f[i][1][0], f[i][1][1], f[i][1][2], f[i][1][3]);
+                    }
                 }
                 continue;
             }
@@ -902,6 +911,20 @@ k_scan2m(const DevData D, const ScanParams P, TopState *st, uint32_t *pair_out)
     hist_end<HIST>(lds_hist, P.hist);
 }
 
+// A pair table entry as integer counts: cases f(x, y), then controls.
+__device__ __forceinline__ void pair_counts(const uint32_t *p, bool as_float, uint32_t (&f)[8])
+{
+    const uint4 u = ((const uint4 *)p)[0], v = ((const uint4 *)p)[1];
+    f[0] = u.x, f[1] = u.y, f[2] = u.z, f[3] = u.w, f[4] = v.x, f[5] = v.y, f[6] = v.z, f[7] = v.w;
+    if (as_float) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            f[x] = (uint32_t)__uint_as_float(f[x]);
+            f[4 + x] = (uint32_t)__uint_as_float(f[4 + x]) - f[x];
+        }
+    }
+}
+
 // Order 3.  A wavefront counts PW prefixes (a, b) against the 64 SNPs of a
 // tile.  Every cell word is one v_bitop3_b32 (a_x & b_y & c_z) and one
 // accumulating v_bcnt_u32_b32.  All rows arrive by buffer loads, which
@@ -936,6 +959,7 @@ __device__ __forceinline__ void scan3m_unit(const DevData &D, const ScanParams &
     const uint64_t tau_combo = st->tau_combo;
     const int np = D.n_pad, n = D.n;
     const uint32_t *pair = P.pair;
+    const bool pf = pair_float(D);
     const int t_end = max(t_lo, (bmin + 1) >> 6);
     for (int t = min(t_hi, (np >> 6) - 1); t >= t_end; --t) {  // last tile first (shared in L2)
         const int c = (t << 6) | lane;
@@ -1016,15 +1040,11 @@ __device__ __forceinline__ void scan3m_unit(const DevData &D, const ScanParams &
             const bool valid = in_range && c > pb[i];
             uint32_t fac[8] = {0, 0, 0, 0, 0, 0, 0, 0}, fbc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
             if (valid) {
-                const uint4 *pac = (const uint4 *)(pair + pair_index(pa[i], c, n) * 8);
-                const uint4 *pbc = (const uint4 *)(pair + pair_index(pb[i], c, n) * 8);
-                const uint4 u0 = pac[0], u1 = pac[1], v0 = pbc[0], v1 = pbc[1];
-                fac[0] = u0.x, fac[1] = u0.y, fac[2] = u0.z, fac[3] = u0.w;
-                fac[4] = u1.x, fac[5] = u1.y, fac[6] = u1.z, fac[7] = u1.w;
-                fbc[0] = v0.x, fbc[1] = v0.y, fbc[2] = v0.z, fbc[3] = v0.w;
-                fbc[4] = v1.x, fbc[5] = v1.y, fbc[6] = v1.z, fbc[7] = v1.w;
+                pair_counts(pair + pair_index(pa[i], c, n) * 8, pf, fac);
+                pair_counts(pair + pair_index(pb[i], c, n) * 8, pf, fbc);
             }
-            const uint32_t *pab = pair + pair_index(pa[i], pb[i], n) * 8;
+            uint32_t pab[8];
+            pair_counts(pair + pair_index(pa[i], pb[i], n) * 8, pf, pab);
             const uint32_t *sa = D.singles + (size_t)pa[i] * 6;
             const uint32_t *sb = D.singles + (size_t)pb[i] * 6;
             uint32_t m0[27], m1[27];
@@ -1685,26 +1705,42 @@ k_mfma2x(const DevData D, const ScanParams P, TopState *st, const Fp4Image F4, i
 constexpr int kM3Group = 16 * 64;
 constexpr int kM3Stage = 13 * kM3Group;
 constexpr int kM3Ring = 4;   // default stages resident: the one read + up to 3 loading
+// LDS of a 64 x 32 workgroup: the ring, then the epilogue's lists of 4 waves
+// (512 entries of 36 bytes each: every instance of the tile)
+constexpr int kM3Lds = 4 * 512 * 36;
+static_assert(kM3Lds >= kM3Ring * kM3Stage && kM3Lds / 4 >= 4 * 16 * 64 * 4, "lists hold the ring");
 __device__ __forceinline__ int m3_swz(int r) { return (r >> 1) & 3; }
 
-// pair_index for 0 <= x < y < n: one 32 x 32 -> 64-bit product, no signed
-// division.
-__device__ __forceinline__ uint64_t pair_index_u(uint32_t x, uint32_t y, uint32_t n)
+// Rank of the pair (x, y) among the pairs in row-major order, for any x, y <
+// n + 64: outside the triangle the value lies within 2,200 of [0, C(n, 2))
+// (x (2 n - x - 1) / 2 >= -2,016 for x < n + 64, and y - x - 1 >= -64), which
+// kPairSlack covers.  Signed: on fewer than 64 SNPs, x can exceed 2 n.
+__device__ __forceinline__ int64_t pair_rank(int32_t x, int32_t y, int32_t n)
 {
-    return ((uint64_t)x * (2u * n - x - 1u) >> 1) + (y - x - 1u);
+    return ((int64_t)x * (2 * n - x - 1) >> 1) + (y - x - 1);
 }
 
 // Values of the order-3 matrix-core epilogue that depend only on the first
-// SNP a and the lane's last SNP c: c's singles, the pair (a, c) and the rank
-// of the prefix (a, a + 1).
+// SNP a and the lane's last SNP c.  Counts are pairs in FP32 (exact): of the
+// cases ([0]) and of both classes ([1]) -- the table's second cells follow by
+// the same inclusion-exclusion, and the bound needs no sum per cell.
 struct M3Lane {
     int c;
     bool c_ok;
-    // as FP32 (exact): singles of a and c (class, genotype 0 / 1), the pair
-    // (a, c) (class, x, z), the class totals
-    float sa[2][2], sc[2][2], fac[8], tot[2];
-    int64_t rank_a;
+    float sa[2][2], sc[2][2], fac[2][4], tot[2];   // singles of a, c; the pair (a, c); the totals
+    const float4 *ab;   // entry of the pair (a, 0): + 2 b
+    int64_t rank_a;     // rank of the prefix (a, a + 1)
 };
+
+__device__ __forceinline__ void single_pair(const DevData &D, uint32_t s, float (&f)[2][2])
+{
+    const uint32_t *sp = D.singles + (size_t)s * 6;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+        f[0][g] = (float)sp[g];
+        f[1][g] = (float)(sp[g] + sp[3 + g]);
+    }
+}
 
 __device__ __forceinline__ M3Lane m3_lane(const DevData &D, const ScanParams &P, int a, int c)
 {
@@ -1712,90 +1748,96 @@ __device__ __forceinline__ M3Lane m3_lane(const DevData &D, const ScanParams &P,
     const int n = D.n;
     L.c = c;
     L.c_ok = c < n && c > a;
-    const uint32_t *sa = D.singles + (size_t)a * 6;
-    // an out-of-range c reads c = a + 1's rows (its triples are dropped)
-    const uint32_t c1 = L.c_ok ? c : a + 1;
-    const uint32_t *sp = D.singles + (size_t)c1 * 6;
-    const uint4 *pac = (const uint4 *)(P.pair + pair_index_u(a, c1, n) * 8);
-    const uint4 u0 = pac[0], u1 = pac[1];
-#pragma unroll
-    for (int cls = 0; cls < 2; ++cls) {
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            L.sa[cls][g] = (float)sa[cls * 3 + g];
-            L.sc[cls][g] = (float)sp[cls * 3 + g];
-        }
-        L.tot[cls] = (float)D.total[cls];
-    }
-    const uint32_t f[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-#pragma unroll
-    for (int e = 0; e < 8; ++e) L.fac[e] = (float)f[e];
-    L.rank_a = (int64_t)a * (2 * (int64_t)n - a - 1) / 2;   // rank of the prefix (a, a+1)
+    L.rank_a = (int64_t)a * (2 * (int64_t)n - a - 1) / 2;
+    L.ab = (const float4 *)P.pair + 2 * (L.rank_a - a - 1);
+    single_pair(D, a, L.sa);
+    single_pair(D, c, L.sc);   // c < n_pad: rows past the last SNP are zero
+    const float4 u0 = L.ab[2 * (int64_t)c], u1 = L.ab[2 * (int64_t)c + 1];
+    L.fac[0][0] = u0.x, L.fac[0][1] = u0.y, L.fac[0][2] = u0.z, L.fac[0][3] = u0.w;
+    L.fac[1][0] = u1.x, L.fac[1][1] = u1.y, L.fac[1][2] = u1.z, L.fac[1][3] = u1.w;
+    L.tot[0] = (float)D.total[0];
+    L.tot[1] = (float)(D.total[0] + D.total[1]);
     return L;
 }
 
-// Triple (a, b, L.c): the 8 matrix-core counts cnt(cls, x, y, z), x, y, z in
-// {0, 1}, with the pair table, the singles and the class totals give the 27
-// cells m0 / m1 of each class (inclusion-exclusion in FP32: the counts are
-// exact integers below 2^24, and so is every step); returns whether the
-// triple is one of the scan's.  m3_triple: then the shared epilogue.
+// The triple (a, b, L.c): the 8 matrix-core counts cnt(k, x, y, z), x, y, z in
+// {0, 1}, k = 0 cases, 1 both classes, with the pair table (`bc`: the entry of
+// (b, L.c)), the singles and the totals give the 27 cells m0 (cases) and m1
+// (both classes), by inclusion-exclusion in FP32: the counts are exact
+// integers below 2^24, and so is every step.
 template <class C>
-__device__ __forceinline__ bool m3_cells(const DevData &D, const ScanParams &P, const M3Lane &L, int a, int b, C &&cnt,
+__device__ __forceinline__ void m3_cells(const DevData &D, const M3Lane &L, uint32_t b, const float4 *bc, C &&cnt,
                                          float (&m0)[27], float (&m1)[27])
 {
-    const int n = D.n, c = L.c;
-    const bool in_range = L.c_ok && b > a && c > b;   // a < b < c < n
-    bool valid = in_range;
-    if (P.step != 1 || P.offset != 0) {   // a share of the prefixes (wave-uniform)
-        const int64_t rel = L.rank_a + (b - a - 1) - P.offset;
-        valid = valid && rel >= 0 && (P.step == 1 || rel % P.step == 0);
-    }
-    // a triple outside the range reads the rows of (a, a + 1, a + 2) instead
-    // (every tile has a < n - 2) and is dropped by `valid`: no select per value
-    const uint32_t b1 = in_range ? b : a + 1, c1 = in_range ? c : a + 2;
-    uint32_t fab[8], fbc[8], sb[6];
+    float fab[2][4], fbc[2][4], sb[2][2];
     {
-        const uint4 *pab = (const uint4 *)(P.pair + pair_index_u(a, b1, n) * 8);
-        const uint4 *pbc = (const uint4 *)(P.pair + pair_index_u(b1, c1, n) * 8);
-        const uint4 p0 = pab[0], p1 = pab[1], q0 = pbc[0], q1 = pbc[1];
-        fab[0] = p0.x, fab[1] = p0.y, fab[2] = p0.z, fab[3] = p0.w;
-        fab[4] = p1.x, fab[5] = p1.y, fab[6] = p1.z, fab[7] = p1.w;
-        fbc[0] = q0.x, fbc[1] = q0.y, fbc[2] = q0.z, fbc[3] = q0.w;
-        fbc[4] = q1.x, fbc[5] = q1.y, fbc[6] = q1.z, fbc[7] = q1.w;
-        const uint32_t *sp = D.singles + (size_t)b1 * 6;
-#pragma unroll
-        for (int e = 0; e < 6; ++e) sb[e] = sp[e];
+        const float4 p0 = L.ab[2 * (uint64_t)b], p1 = L.ab[2 * (uint64_t)b + 1], q0 = bc[0], q1 = bc[1];
+        fab[0][0] = p0.x, fab[0][1] = p0.y, fab[0][2] = p0.z, fab[0][3] = p0.w;
+        fab[1][0] = p1.x, fab[1][1] = p1.y, fab[1][2] = p1.z, fab[1][3] = p1.w;
+        fbc[0][0] = q0.x, fbc[0][1] = q0.y, fbc[0][2] = q0.z, fbc[0][3] = q0.w;
+        fbc[1][0] = q1.x, fbc[1][1] = q1.y, fbc[1][2] = q1.z, fbc[1][3] = q1.w;
+        single_pair(D, b, sb);
     }
 #pragma unroll
-    for (int cls = 0; cls < 2; ++cls) {
-        float *mm = cls ? m1 : m0;
+    for (int k = 0; k < 2; ++k) {
+        float *mm = k ? m1 : m0;
         // mm[x*9 + y*3 + z], x, y, z in {0, 1, 2 = any}
 #pragma unroll
         for (int x = 0; x < 2; ++x)
 #pragma unroll
             for (int y = 0; y < 2; ++y) {
 #pragma unroll
-                for (int z = 0; z < 2; ++z) mm[x * 9 + y * 3 + z] = cnt(cls, x, y, z);
-                mm[x * 9 + y * 3 + 2] = (float)fab[cls * 4 + x * 2 + y];
+                for (int z = 0; z < 2; ++z) mm[x * 9 + y * 3 + z] = cnt(k, x, y, z);
+                mm[x * 9 + y * 3 + 2] = fab[k][x * 2 + y];
             }
 #pragma unroll
         for (int x = 0; x < 2; ++x)
 #pragma unroll
-            for (int z = 0; z < 2; ++z) mm[x * 9 + 6 + z] = L.fac[cls * 4 + x * 2 + z];
+            for (int z = 0; z < 2; ++z) mm[x * 9 + 6 + z] = L.fac[k][x * 2 + z];
 #pragma unroll
         for (int y = 0; y < 2; ++y)
 #pragma unroll
-            for (int z = 0; z < 2; ++z) mm[18 + y * 3 + z] = (float)fbc[cls * 4 + y * 2 + z];
-        mm[0 * 9 + 8] = L.sa[cls][0];
-        mm[1 * 9 + 8] = L.sa[cls][1];
-        mm[18 + 0 * 3 + 2] = (float)sb[cls * 3 + 0];
-        mm[18 + 1 * 3 + 2] = (float)sb[cls * 3 + 1];
-        mm[18 + 6 + 0] = L.sc[cls][0];
-        mm[18 + 6 + 1] = L.sc[cls][1];
-        mm[26] = L.tot[cls];
+            for (int z = 0; z < 2; ++z) mm[18 + y * 3 + z] = fbc[k][y * 2 + z];
+        mm[0 * 9 + 8] = L.sa[k][0];
+        mm[1 * 9 + 8] = L.sa[k][1];
+        mm[18 + 0 * 3 + 2] = sb[k][0];
+        mm[18 + 1 * 3 + 2] = sb[k][1];
+        mm[18 + 6 + 0] = L.sc[k][0];
+        mm[18 + 6 + 1] = L.sc[k][1];
+        mm[26] = L.tot[k];
         mobius3(mm);
     }
-    return valid;
+}
+
+// The bound and the screen of such a table.
+__device__ __forceinline__ bool m3_bound_ok(const float (&m0)[27], const float (&m1)[27], float tau,
+                                            const ScanParams &P)
+{
+    return !P.bounded || bound_passes(mi_bound_fn<27>(
+                                          [&](int x, float &fc, float &fx) __attribute__((always_inline)) {
+                                              fc = m0[x];
+                                              fx = m1[x];
+                                          },
+                                          P.frac_c, P.chi_scale),
+                                      tau, P.delta);
+}
+
+__device__ __forceinline__ bool m3_screen_ok(const float (&m0)[27], const float (&m1)[27], float tau,
+                                             const ScanParams &P)
+{
+    const float sum = screen_sum_fn<27>([&](int x, float &fc, float &ft) __attribute__((always_inline)) {
+        fc = m0[x];
+        ft = m1[x] - m0[x];
+    });
+    return fmaf(sum, P.inv_n * 0.69314718f, P.hy) >= tau - P.delta;
+}
+
+// Whether (a, b, c) with a < b < c < n belongs to the scan's share.
+__device__ __forceinline__ bool m3_in_share(const ScanParams &P, const M3Lane &L, int a, int b)
+{
+    if (P.step == 1 && P.offset == 0) return true;   // wave-uniform
+    const int64_t rel = L.rank_a + (b - a - 1) - P.offset;
+    return rel >= 0 && (P.step == 1 || rel % P.step == 0);
 }
 
 __device__ __forceinline__ uint64_t m3_key(const ScanParams &P, int n, int a, int b, int c)
@@ -1804,19 +1846,120 @@ __device__ __forceinline__ uint64_t m3_key(const ScanParams &P, int n, int a, in
     return prefix_key(P.binom, n, pre, 2) + (uint64_t)c;
 }
 
-template <class C>
-__device__ __forceinline__ void m3_triple(const DevData &D, const ScanParams &P, TopState *st, const M3Lane &L, int a,
-                                          int b, float tau, uint64_t tau_combo, C &&cnt)
+// Exact MI and push of the lanes that need it (all lanes call).
+__device__ __forceinline__ void m3_exact_push(bool need, const float (&m0)[27], const float (&m1)[27],
+                                              const ScanParams &P, TopState *st, int n, int a, int b, int c,
+                                              float tau, uint64_t tau_combo)
 {
-    float m0[27], m1[27];
-    const bool valid = m3_cells(D, P, L, a, b, cnt, m0, m1);
-    score_and_push<27>(valid, m0, m1, [&] { return m3_key(P, D.n, a, b, L.c); }, tau, tau_combo, P, st);
+    exact_push<27>(
+        need,
+        [&](int x, uint32_t &n0, uint32_t &n1) __attribute__((always_inline)) {
+            n0 = (uint32_t)m0[x];
+            n1 = (uint32_t)(m1[x] - m0[x]);
+        },
+        [&] { return m3_key(P, n, a, b, c); }, tau, tau_combo, P, st);
+}
+
+// The epilogues' list of marked instances: per entry the 8 corner counts
+// (word (x * 2 + y) * 2 + z: cases | controls << 16) and where they come from.
+struct M3List {
+    uint4 *words;    // [2][cap]
+    uint32_t *id;    // instance k | lane << 4
+    int cap, count;
+};
+
+// Appends the passing lanes' instance k; `spill` takes a lane's that found the
+// list full.
+template <class S>
+__device__ __forceinline__ void m3_mark(M3List &l, bool pass, int k, int lane, const uint32_t (&wd)[8], uint64_t mask,
+                                        S &&spill)
+{
+    const int at = l.count + (int)__popcll(mask & ((1ull << lane) - 1ull));
+    if (pass) {
+        if (at < l.cap) {
+            l.words[at] = make_uint4(wd[0], wd[1], wd[2], wd[3]);
+            l.words[l.cap + at] = make_uint4(wd[4], wd[5], wd[6], wd[7]);
+            l.id[at] = (uint32_t)(k | lane << 4);
+        } else {
+            spill();
+        }
+    }
+    l.count += (int)__popcll(mask);
+}
+
+// Second pass: 64 of the list's entries per round, one per lane -- screen,
+// exact MI, push -- then what `more(have, id, wd)` still returns.  Instance k of
+// lane `from` is b = b0 + 16 (k / 4) + 4 (from / 16) + k % 4, c = c0 + from % 16.
+template <class F>
+__device__ __forceinline__ void m3_second_pass(const DevData &D, const ScanParams &P, TopState *st, const M3List &l,
+                                               int a, int b0, int c0, float tau, uint64_t tau_combo, F &&more)
+{
+    const int lane = threadIdx.x & 63, listed = std::min(l.count, l.cap);
+    asm volatile("" ::: "memory");   // read by other lanes than wrote it (one wave: in order)
+    for (int first = 0;; first += 64) {
+        bool have = false;
+        uint32_t id = 0, wd[8];
+        if (first < listed) {
+            const int at = first + lane;
+            have = at < listed;
+            if (have) {
+                const uint4 u = l.words[at], v = l.words[l.cap + at];
+                id = l.id[at];
+                wd[0] = u.x, wd[1] = u.y, wd[2] = u.z, wd[3] = u.w, wd[4] = v.x, wd[5] = v.y, wd[6] = v.z, wd[7] = v.w;
+            }
+        } else if (!more(have, id, wd)) {
+            break;
+        }
+        bool need = false;
+        int b = 0, c = 0;
+        float m0[27], m1[27];
+        if (have) {
+            const int k = id & 15, from = id >> 4;
+            b = b0 + 16 * (k >> 2) + 4 * (from >> 4) + (k & 3);
+            c = c0 + (from & 15);
+            const M3Lane M = m3_lane(D, P, a, c);
+            m3_cells(
+                D, M, b, (const float4 *)P.pair + 2 * pair_rank(b, c, D.n),
+                [&](int kk, int x, int y, int z) __attribute__((always_inline)) {
+                    const uint32_t v = wd[(x * 2 + y) * 2 + z];
+                    return (float)(kk ? (v & 0xffffu) + (v >> 16) : v & 0xffffu);
+                },
+                m0, m1);
+            need = m3_screen_ok(m0, m1, tau, P);
+        }
+        m3_exact_push(need, m0, m1, P, st, D.n, a, b, c, tau, tau_combo);
+    }
+}
+
+// Bit k: the lane's instance k < N (b = b0 + 16 (k / 4) + 4 (lane / 16) + k % 4,
+// column L.c) is a triple of the scan.
+template <int N>
+__device__ __forceinline__ uint32_t m3_valid(const ScanParams &P, const M3Lane &L, int a, int b0)
+{
+    const int q4 = 4 * ((threadIdx.x & 63) >> 4);
+    uint32_t ok = 0;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const int b = b0 + 16 * (k >> 2) + q4 + (k & 3);
+        ok |= (uint32_t)(L.c_ok && b > a && L.c > b) << k;
+    }
+    if (P.step != 1 || P.offset != 0) {
+        // a share (wave-uniform): not unrolled, 16 copies of the 64-bit
+        // remainder made whole scans 4 % slower by their mere size
+#pragma unroll 1
+        for (uint32_t left = ok; left; left &= left - 1) {
+            const int k = __builtin_ctz(left), b = b0 + 16 * (k >> 2) + q4 + (k & 3);
+            if (!m3_in_share(P, L, a, b)) ok &= ~(1u << k);
+        }
+    }
+    return ok;
 }
 
 // One workgroup's work item: first SNP a, tile u (see k_mfma3); returns at
 // once for items outside the triangle.  Every wave of the workgroup calls it
 // with the same arguments.  R: stages of the LDS ring (R - 1 in flight).
-template <int R>
+// BIG: classes of 2^16 samples or more (2: find out at run time).
+template <int R, int BIG>
 __device__ __forceinline__ void mfma3_tile(const DevData &D, const ScanParams &P, TopState *st, const Fp4Image &F,
                                            int a, int64_t u, int T, int8_t (*lds)[kM3Stage])
 {
@@ -1975,27 +2118,95 @@ __device__ __forceinline__ void mfma3_tile(const DevData &D, const ScanParams &P
     const float tau = st->tau;
     const uint64_t tau_combo = st->tau_combo;
     const M3Lane L = m3_lane(D, P, a, c0 + wc * 16 + rr);
-    // eight instances (bb, j), so that every accumulator index is a constant
-    static_for<8>([&](auto BJ) __attribute__((always_inline)) {
-        constexpr int bb = decltype(BJ)::value >> 2, j = decltype(BJ)::value & 3;
-        m3_triple(D, P, st, L, a, b0 + wb * 32 + bb * 16 + 4 * (lane >> 4) + j, tau, tau_combo,
-                  [&](int cls, int x, int y, int z) __attribute__((always_inline)) {
-                      return acc[cls][x][y][bb][z][j];
-                  });
-    });
+    const uint32_t ok = m3_valid<8>(P, L, a, b0 + wb * 32);
+    const int q4 = 4 * (lane >> 4), bw = b0 + wb * 32;
+    // the wave's quarter of the workgroup's LDS (kM3Lds bytes): nothing reads
+    // the ring any more
+    int8_t *const mine = (int8_t *)lds + w * (kM3Lds / 4);
+    const bool big = BIG == 1 || (BIG == 2 && (D.cases >= (1u << 16) || D.ctrls >= (1u << 16)));
+    if (BIG != 1 && !big) {
+        // two passes: the bound of the eight instances (bb, j), every
+        // accumulator index a constant; then the marked ones
+        M3List l;
+        l.cap = 512;   // 8 instances x 64 lanes
+        l.count = 0;
+        l.words = (uint4 *)mine;
+        l.id = (uint32_t *)(mine + 32 * 512);
+        static_for<2>([&](auto BB) __attribute__((always_inline)) {
+            constexpr int bb = decltype(BB)::value;
+            int64_t bc = pair_rank(bw + 16 * bb + q4, L.c, D.n);
+            static_for<4>([&](auto J) __attribute__((always_inline)) {
+                constexpr int j = decltype(J)::value, k = 4 * bb + j;
+                const int b = bw + 16 * bb + q4 + j;
+                float m0[27], m1[27];
+                m3_cells(
+                    D, L, b, (const float4 *)P.pair + 2 * bc,
+                    [&](int kk, int x, int y, int z) __attribute__((always_inline)) {
+                        return kk ? acc[0][x][y][bb][z][j] + acc[1][x][y][bb][z][j] : acc[0][x][y][bb][z][j];
+                    },
+                    m0, m1);
+                bc += D.n - b - 2;
+                const bool pass = m3_bound_ok(m0, m1, tau, P) && (ok >> k & 1);
+                const uint64_t mask = __ballot(pass);
+                if (mask) {
+                    uint32_t wd[8];
+#pragma unroll
+                    for (int x = 0; x < 2; ++x)
+#pragma unroll
+                        for (int y = 0; y < 2; ++y)
+#pragma unroll
+                            for (int z = 0; z < 2; ++z)
+                                wd[(x * 2 + y) * 2 + z] =
+                                    (uint32_t)acc[0][x][y][bb][z][j] | (uint32_t)acc[1][x][y][bb][z][j] << 16;
+                    m3_mark(l, pass, k, lane, wd, mask, [] {});
+                }
+            });
+        });
+        m3_second_pass(D, P, st, l, a, bw, c0 + wc * 16, tau, tau_combo, [](bool &, uint32_t &, uint32_t (&)[8]) { return false; });
+        return;
+    }
+    if constexpr (BIG != 0) {
+        // counts above 16 bits: a b block's counts go to LDS, and a loop takes
+        // its four instances (one copy of the scoring code per block)
+        float *const cnt = (float *)mine + lane;   // [4 instances][16 counts][64 lanes]
+        static_for<2>([&](auto BB) __attribute__((always_inline)) {
+            constexpr int bb = decltype(BB)::value;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    cnt[(j * 16 + e) * 64] = acc[0][e >> 2][e >> 1 & 1][bb][e & 1][j];
+                    cnt[(j * 16 + 8 + e) * 64] = acc[1][e >> 2][e >> 1 & 1][bb][e & 1][j];
+                }
+#pragma unroll 1
+            for (int j = 0; j < 4; ++j) {
+                const int b = bw + 16 * bb + q4 + j;
+                float m0[27], m1[27];
+                m3_cells(
+                    D, L, b, (const float4 *)P.pair + 2 * pair_rank(b, L.c, D.n),
+                    [&](int kk, int x, int y, int z) __attribute__((always_inline)) {
+                        const int e = j * 16 + (x * 2 + y) * 2 + z;
+                        return kk ? cnt[e * 64] + cnt[(e + 8) * 64] : cnt[e * 64];
+                    },
+                    m0, m1);
+                const bool need = (ok >> (4 * bb + j) & 1) && m3_bound_ok(m0, m1, tau, P) && m3_screen_ok(m0, m1, tau, P);
+                m3_exact_push(need, m0, m1, P, st, D.n, a, b, L.c, tau, tau_combo);
+            }
+        });
+    }
 }
 
-template <int R>
+template <int R, int BIG>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2)))   // 256 registers, no spills
 k_mfma3(const DevData D, const ScanParams P, TopState *st, const Fp4Image F, int a0, int na, int T)
 {
-    __shared__ __attribute__((aligned(1024))) int8_t lds[R][kM3Stage];
+    __shared__ __attribute__((aligned(1024))) int8_t lds[kM3Lds];
     // block order: workgroup L runs on XCD L % 8; XCD k takes the tiles
     // u = 8 i + k, i = 0, 1, ..., and for each tile all na first SNPs in a
     // row, so that the workgroups resident on one XCD share their b and c
     // rows in its L2 (only the a rows differ)
     const int64_t L = blockIdx.x, s = L >> 3;
-    mfma3_tile<R>(D, P, st, F, a0 + (int)(s % na), (s / na) * 8 + (L & 7), T, lds);
+    mfma3_tile<R, BIG>(D, P, st, F, a0 + (int)(s % na), (s / na) * 8 + (L & 7), T, (int8_t(*)[kM3Stage])lds);
 }
 
 // Wide tile: one workgroup takes first SNP a and a whole 64 x 64 tile of
@@ -2223,14 +2434,23 @@ __device__ __forceinline__ void mfma3w_tile(const DevData &D, const ScanParams &
     const float tau = st->tau;
     const uint64_t tau_combo = st->tau_combo;
     const M3Lane L = m3_lane(D, P, a, c0 + 16 * w + rr);
-    // first pass: the bound of each of the 16 instances (bb, j); a lane's
-    // instances that pass are marked in `pend` (bit 4 bb + j), their counts
-    // (f(x, y, z) of class 0 | class 1 << 16, word (x * 2 + y) * 2 + z) kept
-    // in `marked` in the same order.  Second pass: each round scores one
-    // marked instance per lane, so the screening MI (54 logarithms) runs
-    // about as often as the most marked lane has marks, not once per
-    // instance in which any lane of the wave passes the bound (most
-    // instances, at a top-100 threshold)
+    const uint32_t ok = m3_valid<16>(P, L, a, b0);
+    const int q4 = 4 * (lane >> 4);
+    // First pass: the bound of each of the 16 instances.  Those that pass go
+    // with their counts (word (x * 2 + y) * 2 + z: cases | controls << 16) to a
+    // list in the wave's quarter of the ring, which nothing reads any more; an
+    // instance that finds the list full waits in private memory (`pend`,
+    // `marked`).  Second pass: 64 of the list per round, one per lane, so the
+    // screening MI (54 logarithms) runs about once per tile (with a round per
+    // mark of the most marked lane it ran 2 to 4 times).
+    constexpr int kListBytes = R * kM3wStage / 4, kList = kListBytes / 36 / 8 * 8;
+    static_assert(kListBytes % 16 == 0 && 36 * kList <= kListBytes, "list in a quarter of the ring");
+    int8_t *const mine = (int8_t *)lds + w * kListBytes;
+    M3List l;
+    l.cap = kList;
+    l.count = 0;
+    l.words = (uint4 *)mine;
+    l.id = (uint32_t *)(mine + 32 * kList);
     uint32_t pend = 0;
     int nmarked = 0;
     static_for<4>([&](auto BB) __attribute__((always_inline)) {
@@ -2238,57 +2458,57 @@ __device__ __forceinline__ void mfma3w_tile(const DevData &D, const ScanParams &
         v4i lo[4];
 #pragma unroll
         for (int xy = 0; xy < 4; ++xy) lo[xy] = 4 * bb + xy < kM3wKeep ? keep[4 * bb + xy] : stash[4 * bb + xy];
+        // the entry of (b, c) moves by n - b - 2 pairs from b to b + 1
+        int64_t bc = pair_rank(b0 + 16 * bb + q4, L.c, D.n);
         static_for<4>([&](auto J) __attribute__((always_inline)) {
-            constexpr int j = decltype(J)::value;
+            constexpr int j = decltype(J)::value, k = 4 * bb + j;
+            const int b = b0 + 16 * bb + q4 + j;
             float m0[27], m1[27];
-            const bool valid = m3_cells(
-                D, P, L, a, b0 + 16 * bb + 4 * (lane >> 4) + j,
-                [&](int cls, int x, int y, int z) __attribute__((always_inline)) {
-                    return cls ? acc[x][y][bb][z][j]
-                               : (float)((uint32_t)lo[x * 2 + y][z * 2 + (j >> 1)] >> (16 * (j & 1)) & 0xffffu);
+            auto low = [&](int x, int y, int z) __attribute__((always_inline)) {
+                return (uint32_t)lo[x * 2 + y][z * 2 + (j >> 1)] >> (16 * (j & 1)) & 0xffffu;
+            };
+            m3_cells(
+                D, L, b, (const float4 *)P.pair + 2 * bc,
+                [&](int kk, int x, int y, int z) __attribute__((always_inline)) {
+                    return kk ? m0[x * 9 + y * 3 + z] + acc[x][y][bb][z][j] : (float)low(x, y, z);
                 },
                 m0, m1);
-            if (valid && bound_ok<27>(m0, m1, tau, P)) {
-                pend |= 1u << (4 * bb + j);
-                int wd[8];
+            bc += D.n - b - 2;
+            const bool pass = m3_bound_ok(m0, m1, tau, P) && (ok >> k & 1);
+            const uint64_t mask = __ballot(pass);
+            if (mask) {
+                uint32_t wd[8];
 #pragma unroll
                 for (int x = 0; x < 2; ++x)
 #pragma unroll
                     for (int y = 0; y < 2; ++y)
 #pragma unroll
                         for (int z = 0; z < 2; ++z)
-                            wd[(x * 2 + y) * 2 + z] =
-                                (int)((uint32_t)lo[x * 2 + y][z * 2 + (j >> 1)] >> (16 * (j & 1)) & 0xffffu |
-                                      (uint32_t)acc[x][y][bb][z][j] << 16);
-                marked[2 * nmarked] = (v4i){wd[0], wd[1], wd[2], wd[3]};
-                marked[2 * nmarked + 1] = (v4i){wd[4], wd[5], wd[6], wd[7]};
-                ++nmarked;
+                            wd[(x * 2 + y) * 2 + z] = low(x, y, z) | (uint32_t)acc[x][y][bb][z][j] << 16;
+                m3_mark(l, pass, k, lane, wd, mask, [&]() __attribute__((always_inline)) {
+                    pend |= 1u << k;
+                    marked[2 * nmarked] = (v4i){(int)wd[0], (int)wd[1], (int)wd[2], (int)wd[3]};
+                    marked[2 * nmarked + 1] = (v4i){(int)wd[4], (int)wd[5], (int)wd[6], (int)wd[7]};
+                    ++nmarked;
+                });
             }
         });
     });
     int taken = 0;
-    while (__ballot(pend != 0)) {
-        bool need = false;
-        int b = 0;
-        float m0[27], m1[27];
-        if (pend) {
-            const int i = __builtin_ctz(pend), bb = i >> 2, j = i & 3;
-            pend &= pend - 1;
-            b = b0 + 16 * bb + 4 * (lane >> 4) + j;
-            const v4i w0 = marked[2 * taken], w1 = marked[2 * taken + 1];
-            ++taken;
-            m3_cells(
-                D, P, L, a, b,
-                [&](int cls, int x, int y, int z) __attribute__((always_inline)) {
-                    const int e = (x * 2 + y) * 2 + z;
-                    const uint32_t v = (uint32_t)(e < 4 ? w0[e] : w1[e - 4]);
-                    return (float)(cls ? v >> 16 : v & 0xffffu);
-                },
-                m0, m1);
-            need = mi_screen<27>(m0, m1, P.hy, P.inv_n) >= tau - P.delta;
-        }
-        exact_push_arrays<27>(need, m0, m1, [&] { return m3_key(P, D.n, a, b, L.c); }, tau, tau_combo, P, st);
-    }
+    m3_second_pass(D, P, st, l, a, b0, c0 + 16 * w, tau, tau_combo,
+                   [&](bool &have, uint32_t &id, uint32_t (&wd)[8]) __attribute__((always_inline)) {
+                       if (!__ballot(pend != 0)) return false;
+                       have = pend != 0;
+                       if (have) {
+                           id = (uint32_t)(__builtin_ctz(pend) | lane << 4);
+                           pend &= pend - 1;
+                           const v4i u = marked[2 * taken], v = marked[2 * taken + 1];
+                           ++taken;
+#pragma unroll
+                           for (int e = 0; e < 4; ++e) wd[e] = (uint32_t)u[e], wd[4 + e] = (uint32_t)v[e];
+                       }
+                       return true;
+                   });
 }
 
 template <int R>
@@ -2725,8 +2945,7 @@ k_batch_mfma(const BatchJob *__restrict__ jobs, const BatchSeg *__restrict__ seg
     constexpr size_t kWide = (size_t)kM2wRing * kM2wStage > (size_t)kM3Ring * kM3wStage
                                  ? (size_t)kM2wRing * kM2wStage
                                  : (size_t)kM3Ring * kM3wStage;
-    constexpr size_t kNarrow = sizeof(Mfma2Lds<true>) > (size_t)kM3Ring * kM3Stage ? sizeof(Mfma2Lds<true>)
-                                                                                 : (size_t)kM3Ring * kM3Stage;
+    constexpr size_t kNarrow = sizeof(Mfma2Lds<true>) > (size_t)kM3Lds ? sizeof(Mfma2Lds<true>) : (size_t)kM3Lds;
     constexpr size_t kBytes = kWide > kNarrow ? kWide : kNarrow;
     __shared__ __attribute__((aligned(1024))) int8_t lds[kBytes];   // the order-2 or the order-3 tiles
     __shared__ uint32_t unit_sh;
@@ -2758,7 +2977,7 @@ k_batch_mfma(const BatchJob *__restrict__ jobs, const BatchSeg *__restrict__ seg
                 mfma3w_tile<kM3Ring>(D, P, st, F, (int)(j0 + l % na), (int64_t)(l / na) * 8 + x, J.T,
                                      (int8_t(*)[kM3wStage])lds);
             else
-                mfma3_tile<kM3Ring>(D, P, st, F, (int)(j0 + l % na), (int64_t)(l / na) * 8 + x, J.T,
+                mfma3_tile<kM3Ring, 2>(D, P, st, F, (int)(j0 + l % na), (int64_t)(l / na) * 8 + x, J.T,
                                     (int8_t(*)[kM3Stage])lds);
         } else if (J.wide) {
             const int64_t su = j0 + (int64_t)(l / 32) * 8 + x;
@@ -3255,8 +3474,11 @@ hipError_t launch_mfma3(const DevData &D, const ScanParams &P, TopState *st, con
         return hipSuccess;
     }
     const dim3 grid((unsigned)(tiles8 * na * 8)), block(kBlock);
-    if (ring == 3) hipLaunchKernelGGL((k_mfma3<3>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
-    else if (ring == kM3Ring) hipLaunchKernelGGL((k_mfma3<kM3Ring>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
+    const bool big = D.cases >= (1u << 16) || D.ctrls >= (1u << 16);
+    if (ring == 3 && big) hipLaunchKernelGGL((k_mfma3<3, 1>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
+    else if (ring == 3) hipLaunchKernelGGL((k_mfma3<3, 0>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
+    else if (ring == kM3Ring && big) hipLaunchKernelGGL((k_mfma3<kM3Ring, 1>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
+    else if (ring == kM3Ring) hipLaunchKernelGGL((k_mfma3<kM3Ring, 0>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
     else if (ring == 5) hipLaunchKernelGGL((k_mfma3w<3>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
     else if (ring == 6) hipLaunchKernelGGL((k_mfma3w<4>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
     else return hipErrorInvalidValue;

@@ -53,3 +53,26 @@ def test_tuple_scans(order, snps, cases, ctrls, step, offset, missing, outputs, 
         oc, om, _ = O.search(od, order, outputs, step=step, offset=offset, threads=1, mi_mode=2)
         assert got[0].tolist() == oc.tolist() and np.array_equal(got[1], om)
     d.close()
+
+
+@pytest.mark.parametrize("snps,cases,ctrls,outputs,variants", [
+    (70, 66000, 100, 200, (3, 4)),      # a class above 16-bit counts: scored from LDS, block by block
+    (66, 900, 65600, 4000, (4,)),
+    (130, 500, 520, 4096, (3, 4, 5, 6)),   # no threshold at first: every triple is marked, full lists
+    (67, 65000, 300, 50, (4, 6)),       # the largest 16-bit counts
+])
+def test_order3_epilogues(snps, cases, ctrls, outputs, variants):
+    print(f"case: order 3 epilogues {snps}x{cases}+{ctrls}", flush=True)
+    g = genotypes(snps, cases + ctrls, 50 + snps, 0)
+    is_ctrl = (np.arange(cases + ctrls) >= cases).astype(np.uint8)
+    d = fa.Dataset.from_genotypes(g, is_ctrl)
+    dist = fa.Distribution(snps, 2)
+    want = fa.GpuSearch(algorithm=MARGINAL).run_arrays(d, 3, dist, outputs)
+    for v in variants:
+        for sample in (True, False):
+            s = fa.GpuSearch(algorithm=fa.ALGO_MFMA, variant=v, sample_threshold=sample)
+            got = s.run_arrays(d, 3, dist, outputs)
+            assert got[0].tolist() == want[0].tolist() and np.array_equal(got[1], want[1]), (v, sample)
+    (batched, _) = fa.search_batch([(d, 3, dist, outputs)])
+    assert batched[0][0].tolist() == want[0].tolist() and np.array_equal(batched[0][1], want[1])
+    d.close()
