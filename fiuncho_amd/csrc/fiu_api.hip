@@ -733,12 +733,24 @@ ThresholdSample plan_sample(int order, int n, int64_t step, int64_t offset, uint
     ThresholdSample S;
     const double combos = (double)n_pref * (double)(n - order + 1) / (double)order;
     const double expect = (double)outputs * combos / (double)cap;
-    const double want = std::min(std::min(std::max({combos / 128.0, 32768.0, 8.0 * expect}),
+    // The tiles of 16 b rows that fill the device once take little longer than
+    // a few of them, so that many are sampled, up to one combination in 8: with
+    // 98,000 pairs of 5,003 x 9,001 the scan took 255 to 400 us as the sample
+    // had more or fewer pairs of the SNPs with an effect, with 262,144 255
+    // (sampling 29 us); 524,288 cost 100 us more on 300 x 3,000 triples
+    const double floor = tup ? std::max(32768.0, std::min(combos / 8.0, 262144.0)) : 32768.0;
+    const double want = std::min(std::min(std::max({combos / 128.0, floor, 8.0 * expect}),
                                           std::max(8388608.0, 2.0 * expect)),
                                  (double)target);
     S.step = std::max<int64_t>(1, (int64_t)(combos / std::max(want, 1.0)));
     S.tup = tup;
     S.on = tup;
+    // Fewer than 512 whole tiles (4,096 combinations; 1,024 at order 4) leave
+    // the device idle while each workgroup scores 16 combinations per lane,
+    // 19 us of them whatever the samples: tiles of 16 b rows instead, four
+    // times as many workgroups with 4 each (pairs of 1,000 x 4,000 33 -> 21 us,
+    // triples of 151 x 1,203 38 -> 18)
+    S.small = combos / (double)S.step < (order == 4 ? 524288.0 : 2097152.0);
     if (tup) return S;
     // Without the tuple kernels the popcount scan samples the share (step x
     // S.step) of the prefixes, at 5-12x the matrix cores' cost per
@@ -762,12 +774,13 @@ void launch_sample(const ThresholdSample &S, const fiu_dataset *d, const ScanPar
         // one unit in `stride`, and of its tiles one in `tile_stride` (about
         // 32 tiles of an order-3 head, so that many heads are seen)
         TupleArgs B = tuple_args(d, order, all_cells);
-        const int64_t n = (int64_t)d->snps, units = tuple_units(order, all_cells, (uint64_t)n, n_pref);
+        const int64_t n = (int64_t)d->snps, units = tuple_units(order, all_cells, (uint64_t)n, n_pref, S.small);
         const int64_t head_tiles = (n + 63) / 64 * ((n + 63) / 64) / 2;
         const int64_t tiles = order == 2   ? S.step
                               : order == 3 ? std::min(S.step, std::max<int64_t>(2, head_tiles / 32))
                                            : 1;
         B.tile_stride = (int32_t)std::min<int64_t>(tiles, 1 << 20);
+        B.small = S.small;
         B.stride = std::max<int64_t>(1, std::min(S.step / tiles, units));
         H.j0 = B.stride / 2;
         H.j1 = units;
@@ -792,9 +805,9 @@ void launch_sample(const ThresholdSample &S, const fiu_dataset *d, const ScanPar
     check(launch_tau_from_hist(hist, outputs, P.delta, st, s), "threshold launch");
 }
 
-int64_t tuple_units(int order, bool all_cells, uint64_t n, int64_t n_pref)
+int64_t tuple_units(int order, bool all_cells, uint64_t n, int64_t n_pref, bool small)
 {
-    const int bt = tuple_b_block(2, all_cells);
+    const int bt = tuple_b_block(2, all_cells, small);
     return order == 2 ? (n_pref + bt - 1) / bt : (int64_t)binom_sat(n, (uint64_t)order - 2);
 }
 
@@ -913,11 +926,12 @@ class Workspace {
     virtual uint32_t *big_cells(fiu_dataset *d, int order) = 0;
     // timing event i, or null (the search is not timed)
     virtual hipEvent_t event(fiu_dataset *d, size_t i) = 0;
-    // the search state, after a synchronisation of s; where it can, the
-    // workspace reads the top list's first `outputs` entries in the same
-    // synchronisation, for results()
-    virtual void read_state(fiu_dataset *d, const TopState *state, const Cand *top, uint32_t outputs, TopState &hs,
-                            hipStream_t s)
+    // pinned memory into which the last merge writes the state and the top
+    // list (up to kMaxOutputs), or null
+    virtual void *mirror(fiu_dataset *, uint32_t) { return nullptr; }
+    // the search state, after a synchronisation of s; `mirrored`: it and the
+    // list are in the mirror
+    virtual void read_state(fiu_dataset *, const TopState *state, bool, TopState &hs, hipStream_t s)
     {
         check(hipMemcpyAsync(&hs, state, sizeof(hs), hipMemcpyDeviceToHost, s), "state read");
         check(hipStreamSynchronize(s), "search sync");
@@ -969,27 +983,24 @@ class DatasetWorkspace final : public Workspace {
         }
         return d->events[i];
     }
-    // up to kMaxOutputs results: the state and the list in one copy each
-    // into the dataset's pinned readback block, one synchronisation
-    void read_state(fiu_dataset *d, const TopState *state, const Cand *top, uint32_t outputs, TopState &hs,
-                    hipStream_t s) override
+    void *mirror(fiu_dataset *d, uint32_t outputs) override
     {
-        listed_ = nullptr;
-        if (outputs > (uint32_t)kMaxOutputs) return Workspace::read_state(d, state, top, outputs, hs, s);
+        if (outputs > (uint32_t)kMaxOutputs) return nullptr;
         if (!d->readback) {
             void *p = nullptr;
             check(hipHostMalloc(&p, sizeof(TopState) + kMaxOutputs * sizeof(Cand), hipHostMallocDefault),
                   "hipHostMalloc");
             d->readback = p;
         }
-        char *rb = (char *)d->readback;
-        check(hipMemcpyAsync(rb, state, sizeof(TopState), hipMemcpyDeviceToHost, s), "state read");
-        if (outputs)
-            check(hipMemcpyAsync(rb + sizeof(TopState), top, outputs * sizeof(Cand), hipMemcpyDeviceToHost, s),
-                  "top read");
+        return d->readback;
+    }
+    void read_state(fiu_dataset *d, const TopState *state, bool mirrored, TopState &hs, hipStream_t s) override
+    {
+        listed_ = nullptr;
+        if (!mirrored) return Workspace::read_state(d, state, mirrored, hs, s);
         check(hipStreamSynchronize(s), "search sync");
-        std::memcpy(&hs, rb, sizeof(hs));
-        listed_ = (const Cand *)(rb + sizeof(TopState));
+        std::memcpy(&hs, d->readback, sizeof(hs));
+        listed_ = (const Cand *)((const char *)d->readback + sizeof(TopState));
     }
     void results(const Cand *top, uint32_t count, int order, int n, const uint64_t *, int32_t *out_combos,
                  float *out_mi, hipStream_t s) override
@@ -1214,6 +1225,10 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
 
     size_t ev = 0;
     bool timed = true;
+    // the chunk whose merge ends the first pass over them
+    uint64_t last = plan.count;
+    while (last > 0 && plan.at(last - 1).j1 <= plan.at(last - 1).j0) --last;
+    void *const mirror = big_merge || last == 0 ? nullptr : ws.mirror(d, outputs);
     auto run_chunk = [&](uint64_t ci, bool time_it) {
         const Chunk c = plan.at(ci);
         if (c.j1 <= c.j0) return;   // an empty first-SNP chunk
@@ -1253,7 +1268,14 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
                                    (uint32_t)pow2_at_least((uint64_t)h.n_top + count), (uint32_t)ci, redo, s),
                   "merge launch");
         } else {
-            check(launch_merge(state, top, cand, outputs, cap, (uint32_t)ci, redo, s), "merge launch");
+            // first pass: a merge waits for an eighth of the list's length (a
+            // threshold any staler costs the scan more than the merges: 2 ms
+            // of 57 on 50,000 x 32,000 where they waited for twice the
+            // length); re-scans merge and write the list each time
+            const bool more = time_it && ci + 1 < last;
+            const uint32_t wait = more ? std::min(std::max(outputs / 8, 32u), cap / 2) : 0;
+            check(launch_merge(state, top, cand, outputs, cap, (uint32_t)ci, redo, wait, more ? nullptr : mirror, s),
+                  "merge launch");
         }
         ++st.launches;
     };
@@ -1263,7 +1285,7 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     // the (higher) final threshold until none overflows
     TopState hs;
     for (;;) {
-        ws.read_state(d, state, top, outputs, hs, s);
+        ws.read_state(d, state, mirror != nullptr, hs, s);
         if (hs.redo_count == 0) break;
         const uint32_t n_redo = hs.redo_count;
         hs.redo_count = 0;

@@ -288,7 +288,7 @@ constexpr int32_t kTupleFill = 16384;
 // n_pref prefixes; its units (heads, or at order 2 blocks of b's); its
 // arguments once ensure_tuple_tables / ensure_tuple_image succeeded.
 bool tuple_scan(const fiu_dataset *d, int order, int64_t step, int64_t n_pref);
-int64_t tuple_units(int order, bool all_cells, uint64_t n, int64_t n_pref);
+int64_t tuple_units(int order, bool all_cells, uint64_t n, int64_t n_pref, bool small = false);
 TupleArgs tuple_args(const fiu_dataset *d, int order, bool all_cells);
 
 // The pass that seeds a search's threshold: which combinations it screens,
@@ -296,6 +296,7 @@ TupleArgs tuple_args(const fiu_dataset *d, int order, bool all_cells);
 // around a head (tables or image ready), else by the popcount kernels.
 struct ThresholdSample {
     bool on = false, tup = false, layered = false;
+    bool small = false;   // tup: tiles of 16 b rows
     int64_t step = 1, prefixes = 0;
 };
 ThresholdSample plan_sample(int order, int n, int64_t step, int64_t offset, uint64_t total_prefixes, int64_t n_pref,

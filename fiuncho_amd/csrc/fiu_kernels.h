@@ -42,7 +42,7 @@ hipError_t launch_mfma3(const DevData &D, const ScanParams &P, TopState *st, con
 hipError_t launch_mfma2(const DevData &D, const ScanParams &P, TopState *st, int64_t s0, int64_t s1, int T,
                         const uint4 *fp4, int tile, hipStream_t s);
 hipError_t launch_merge(TopState *st, Cand *top, const Cand *cand, uint32_t N, uint32_t cap, uint32_t chunk_id,
-                        uint32_t *redo, hipStream_t s);
+                        uint32_t *redo, uint32_t wait, void *host, hipStream_t s);
 // Top-N merge for N above kMaxOutputs, in global memory: the list's n_top
 // entries and `count` candidates (sizes read by the host) sorted in `work`
 // (L entries, a power of two >= n_top + count), the first N unique kept.
@@ -89,11 +89,12 @@ struct TupleArgs {
     int64_t units;           // set by the launcher
     int32_t rounds, nb, nc, aligned;   // set by the launcher
     int32_t fill;            // workgroups that fill the device
+    bool small;              // sampling: in tiles of 16 b rows
 };
 // Scores (or samples, P.hist) units [P.j0, P.j1): heads (order >= 3) or blocks
 // of tuple_b_block b's (order 2) of the share (P.step, P.offset).  all_cells:
 // orders 2 and 3, any dataset; else orders 2 to 4, uniform datasets.
-int tuple_b_block(int order, bool all_cells);
+int tuple_b_block(int order, bool all_cells, bool small = false);
 hipError_t launch_tuples(int order, bool all_cells, const DevData &D, const ScanParams &P, TopState *st,
                          const TupleArgs &A, hipStream_t s);
 // t[1] of the tables (2 n words), and the fp4 image of all three rows

@@ -1208,19 +1208,37 @@ template <bool FP4> using Mfma2Lds = typename Mfma2LdsT<FP4>::type;
 // cycles per wave per CU, as a linear read).
 __device__ __forceinline__ int m2_swz(int r) { return (r >> 2) & 3; }
 
-// One workgroup's work item: tile `slot` (of 64) of super-block su; returns at
-// once for tiles outside the triangle.  Every wave of the workgroup calls it
-// with the same arguments.
+// Tile `slot` (of 64) of super-block su.
+__device__ __forceinline__ void super_tile(int64_t su, int slot, int T, int &ta, int &tb)
+{
+    int sa, sc;
+    tri_tile(su, (T + kMfmaSuper - 1) / kMfmaSuper, sa, sc);
+    ta = sa * kMfmaSuper + (slot >> 3);
+    tb = sc * kMfmaSuper + (slot & 7);
+}
+
+// Position l in the order of a whole scan: bands of 8 tile rows, in a band
+// column by column (its first columns hold positions below the diagonal, 28
+// per band).  64 positions in a row share 8 + 8 panels, as a super-block does.
+__host__ __device__ inline int64_t band_start(int r, int T) { return 8 * ((int64_t)T * r - 4 * (int64_t)r * (r - 1)); }
+__device__ __forceinline__ void band_tile(int64_t l, int T, int &ta, int &tb)
+{
+    int r = 0;
+    while (8 * (r + 1) < T && band_start(r + 1, T) <= l) ++r;
+    const int64_t at = l - band_start(r, T);
+    ta = 8 * r + (int)(at & 7);
+    tb = 8 * r + (int)std::min<int64_t>(at >> 3, T);
+}
+
+// One workgroup's work item: tile (ta, tb); returns at once for tiles outside
+// the triangle.  Every wave of the workgroup calls it with the same
+// arguments.
 template <bool FP4>
 __device__ __forceinline__ void mfma2_tile(const DevData &D, const ScanParams &P, TopState *st, const Fp4Image &F4,
-                                           int64_t su, int slot, int T, Mfma2Lds<FP4> &lds)
+                                           int ta, int tb, int T, Mfma2Lds<FP4> &lds)
 {
     typedef MfmaFmt<FP4> F;
     typedef typename std::conditional<FP4, v16f, v16i>::type Acc;
-    const int S = (T + kMfmaSuper - 1) / kMfmaSuper;
-    int sa, sc;
-    tri_tile(su, S, sa, sc);
-    const int ta = sa * kMfmaSuper + (slot >> 3), tb = sc * kMfmaSuper + (slot & 7);
     if (ta > tb || tb >= T) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wa = w >> 1, wb = w & 1;
@@ -1352,53 +1370,169 @@ __device__ __forceinline__ void mfma2_tile(const DevData &D, const ScanParams &P
     // a = a0 + wa*32 + 8r + 4(lane/32) + q, r, q < 4
     const float tau = st->tau;
     const uint64_t tau_combo = st->tau_combo;
-    const int b = b0 + wb * 32 + (lane & 31);
+    const int b = b0 + wb * 32 + (lane & 31), aw = a0 + wa * 32 + 4 * (lane >> 5);
     const bool b_ok = b < D.n;
     uint32_t sb[2][2] = {{0, 0}, {0, 0}};
     if (b_ok) {
         const uint32_t *sp = D.singles + (size_t)b * 6;
         sb[0][0] = sp[0], sb[0][1] = sp[1], sb[1][0] = sp[3], sb[1][1] = sp[4];
     }
+    // bit 4 r + q: a pair of the scan
+    uint32_t ok = 0;
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int i = r * 4 + q;
-            const int a = a0 + wa * 32 + 8 * r + 4 * (lane >> 5) + q;
-            const int64_t rel = (int64_t)a - P.offset;
-            const bool valid = b_ok && a < b && rel >= 0 && (P.step == 1 || rel % P.step == 0);
-            const uint32_t *sa = D.singles + (size_t)a * 6;
-            // counts as FP32 (fp4 products) or uint32_t (int8 products): both
-            // exact, and the inclusion-exclusion stays exact in either
-            typedef typename std::conditional<FP4, float, uint32_t>::type Cnt;
-            Cnt m0[9], m1[9];
-#pragma unroll
-            for (int cls = 0; cls < 2; ++cls) {
-                Cnt *m = cls ? m1 : m0;
-                m[0] = (Cnt)acc[cls][0][0][i];
-                m[1] = (Cnt)acc[cls][0][1][i];
-                m[3] = (Cnt)acc[cls][1][0][i];
-                m[4] = (Cnt)acc[cls][1][1][i];
-                m[2] = (Cnt)sa[cls * 3 + 0];
-                m[5] = (Cnt)sa[cls * 3 + 1];
-                m[6] = (Cnt)sb[cls][0];
-                m[7] = (Cnt)sb[cls][1];
-                m[8] = (Cnt)D.total[cls];
-                mobius2(m);
-            }
-            score_and_push<9>(valid, m0, m1, [&] { return prefix_key(P.binom, D.n, &a, 1) + (uint64_t)b; }, tau,
-                              tau_combo, P, st);
+    for (int i = 0; i < 16; ++i) {
+        const int a = aw + 8 * (i >> 2) + (i & 3);
+        ok |= (uint32_t)(b_ok && a < b) << i;
+    }
+    if (P.step != 1 || P.offset != 0) {   // a share (wave-uniform)
+#pragma unroll 1
+        for (uint32_t left = ok; left; left &= left - 1) {
+            const int i = __builtin_ctz(left);
+            const int64_t rel = (int64_t)(aw + 8 * (i >> 2) + (i & 3)) - P.offset;
+            if (rel < 0 || (P.step != 1 && rel % P.step != 0)) ok &= ~(1u << i);
         }
+    }
+    if constexpr (FP4) {
+        if (D.cases < (1u << 16) && D.ctrls < (1u << 16)) {
+            // Two passes: the bound of the lane's 16 pairs, those that pass
+            // with their counts (word g * 2 + h: cases | controls << 16) in
+            // the wave's quarter of the ring, which nothing reads any more;
+            // then one marked pair per lane and round.  (5,003 x 9,001:
+            // 286 us with the screen and the exact MI inline in all 16, 262
+            // so, 400 with a loop over counts that all went through LDS: two
+            // waves per SIMD do not hide the loop's latencies.)
+            uint4 *const mine = (uint4 *)&lds[0][0][0][0] + w * (16 * 64) + lane;
+            float sbf[2][2], tot[2];   // of the cases, of both classes
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                sbf[0][h] = (float)sb[0][h];
+                sbf[1][h] = (float)(sb[0][h] + sb[1][h]);
+            }
+            tot[0] = (float)D.total[0];
+            tot[1] = (float)(D.total[0] + D.total[1]);
+            // the cells of the cases (m0) and of both classes (m1)
+            auto cells = [&](int a, auto &&cnt, float (&m0)[9], float (&m1)[9]) __attribute__((always_inline)) {
+                const uint32_t *sa = D.singles + (size_t)a * 6;
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    float *m = k ? m1 : m0;
+                    m[0] = cnt(k, 0, 0);
+                    m[1] = cnt(k, 0, 1);
+                    m[3] = cnt(k, 1, 0);
+                    m[4] = cnt(k, 1, 1);
+                    m[2] = (float)(k ? sa[0] + sa[3] : sa[0]);
+                    m[5] = (float)(k ? sa[1] + sa[4] : sa[1]);
+                    m[6] = sbf[k][0];
+                    m[7] = sbf[k][1];
+                    m[8] = tot[k];
+                    mobius2(m);
+                }
+            };
+            uint32_t pend = 0;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                float m0[9], m1[9];
+                cells(
+                    aw + 8 * (i >> 2) + (i & 3),
+                    [&](int k, int g, int h) __attribute__((always_inline)) {
+                        return k ? acc[0][g][h][i] + acc[1][g][h][i] : acc[0][g][h][i];
+                    },
+                    m0, m1);
+                const float bound = mi_bound_fn<9>(
+                    [&](int x, float &fc, float &fx) __attribute__((always_inline)) {
+                        fc = m0[x];
+                        fx = m1[x];
+                    },
+                    P.frac_c, P.chi_scale);
+                if ((ok >> i & 1) && (!P.bounded || bound_passes(bound, tau, P.delta))) {
+                    pend |= 1u << i;
+                    uint32_t wd[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        wd[e] = (uint32_t)acc[0][e >> 1][e & 1][i] | (uint32_t)acc[1][e >> 1][e & 1][i] << 16;
+                    mine[i * 64] = make_uint4(wd[0], wd[1], wd[2], wd[3]);
+                }
+            }
+            while (__ballot(pend != 0)) {
+                bool need = false;
+                int a = 0;
+                float m0[9], m1[9];
+                if (pend) {
+                    const int i = __builtin_ctz(pend);
+                    pend &= pend - 1;
+                    a = aw + 8 * (i >> 2) + (i & 3);
+                    const uint4 u = mine[i * 64];
+                    cells(
+                        a,
+                        [&](int k, int g, int h) __attribute__((always_inline)) {
+                            const uint32_t v = g ? (h ? u.w : u.z) : h ? u.y : u.x;
+                            return (float)(k ? (v & 0xffffu) + (v >> 16) : v & 0xffffu);
+                        },
+                        m0, m1);
+                    const float sum = screen_sum_fn<9>([&](int x, float &fc, float &ft) __attribute__((always_inline)) {
+                        fc = m0[x];
+                        ft = m1[x] - m0[x];
+                    });
+                    need = fmaf(sum, P.inv_n * 0.69314718f, P.hy) >= tau - P.delta;
+                }
+                exact_push<9>(
+                    need,
+                    [&](int x, uint32_t &n0, uint32_t &n1) __attribute__((always_inline)) {
+                        n0 = (uint32_t)m0[x];
+                        n1 = (uint32_t)(m1[x] - m0[x]);
+                    },
+                    [&] { return prefix_key(P.binom, D.n, &a, 1) + (uint64_t)b; }, tau, tau_combo, P, st);
+            }
+            return;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int a = aw + 8 * (i >> 2) + (i & 3);
+        const uint32_t *sa = D.singles + (size_t)a * 6;
+        // counts as FP32 (fp4 products) or uint32_t (int8 products): both
+        // exact, and the inclusion-exclusion stays exact in either
+        typedef typename std::conditional<FP4, float, uint32_t>::type Cnt;
+        Cnt m0[9], m1[9];
+#pragma unroll
+        for (int cls = 0; cls < 2; ++cls) {
+            Cnt *m = cls ? m1 : m0;
+            m[0] = (Cnt)acc[cls][0][0][i];
+            m[1] = (Cnt)acc[cls][0][1][i];
+            m[3] = (Cnt)acc[cls][1][0][i];
+            m[4] = (Cnt)acc[cls][1][1][i];
+            m[2] = (Cnt)sa[cls * 3 + 0];
+            m[5] = (Cnt)sa[cls * 3 + 1];
+            m[6] = (Cnt)sb[cls][0];
+            m[7] = (Cnt)sb[cls][1];
+            m[8] = (Cnt)D.total[cls];
+            mobius2(m);
+        }
+        score_and_push<9>(ok >> i & 1, m0, m1, [&] { return prefix_key(P.binom, D.n, &a, 1) + (uint64_t)b; }, tau,
+                          tau_combo, P, st);
+    }
 }
 
+// Super-blocks [s0, s1), or (s0 < 0) the whole triangle in s1 positions: XCD x
+// takes an eighth of the bands' order, where whole super-blocks leave XCDs idle
+// (1,000 SNPs have 3, 5,000 have 55).
 template <bool FP4>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_mfma2(const DevData D, const ScanParams P, TopState *st, const Fp4Image F4, int64_t s0, int64_t s1, int T)
 {
     __shared__ __attribute__((aligned(16))) Mfma2Lds<FP4> lds;
-    const int64_t k = blockIdx.x >> 3, su = s0 + (k >> 6) * 8 + (blockIdx.x & 7);
-    if (su >= s1) return;
-    mfma2_tile<FP4>(D, P, st, F4, su, (int)(k & 63), T, lds);
+    const int64_t k = blockIdx.x >> 3;
+    int ta, tb;
+    if (s0 < 0) {
+        const int64_t l = (blockIdx.x & 7) * ((s1 + 7) >> 3) + k;
+        if (l >= s1) return;
+        band_tile(l, T, ta, tb);
+    } else {
+        const int64_t su = s0 + (k >> 6) * 8 + (blockIdx.x & 7);
+        if (su >= s1) return;
+        super_tile(su, (int)(k & 63), T, ta, tb);
+    }
+    mfma2_tile<FP4>(D, P, st, F4, ta, tb, T, lds);
 }
 
 // Wide order-2 tiles: one workgroup of AT * 4 waves takes AT * 64 a x 128 b
@@ -2134,6 +2268,7 @@ __device__ __forceinline__ void mfma3_tile(const DevData &D, const ScanParams &P
         l.id = (uint32_t *)(mine + 32 * 512);
         static_for<2>([&](auto BB) __attribute__((always_inline)) {
             constexpr int bb = decltype(BB)::value;
+            if (!__ballot(ok >> 4 * bb & 15)) return;   // no triple of the scan
             int64_t bc = pair_rank(bw + 16 * bb + q4, L.c, D.n);
             static_for<4>([&](auto J) __attribute__((always_inline)) {
                 constexpr int j = decltype(J)::value, k = 4 * bb + j;
@@ -2196,6 +2331,20 @@ __device__ __forceinline__ void mfma3_tile(const DevData &D, const ScanParams &P
     }
 }
 
+// Residue (mod 8) of the tiles that XCD x takes of first SNP a.  The tiles of
+// the first SNPs of one 64-SNP tile are dealt on where those of the tile before
+// ended: always starting at XCD 0 gives it the odd tile of every first SNP
+// (151 SNPs: 1.5x the mean).  While the image (n_pad x samples bytes) fits an
+// XCD's 4 MB of L2, the deal moves on with every first SNP instead.
+// `per`: work items per 64 x 64 tile.
+__device__ __forceinline__ int m3_turn(int x, int a, int T, int per, const DevData &D)
+{
+    if ((uint64_t)D.n_pad * (D.total[0] + D.total[1]) <= (4u << 20)) return (x + a) & 7;
+    const uint32_t m = (uint32_t)(T - ((a + 1) >> 6)), t = (uint32_t)T;
+    const uint64_t before = ((uint64_t)t * (t + 1) * (t + 2) - (uint64_t)m * (m + 1) * (m + 2)) / 6;
+    return (x - (int)(before * (uint64_t)per & 7)) & 7;
+}
+
 template <int R, int BIG>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2)))   // 256 registers, no spills
 k_mfma3(const DevData D, const ScanParams P, TopState *st, const Fp4Image F, int a0, int na, int T)
@@ -2206,7 +2355,8 @@ k_mfma3(const DevData D, const ScanParams P, TopState *st, const Fp4Image F, int
     // row, so that the workgroups resident on one XCD share their b and c
     // rows in its L2 (only the a rows differ)
     const int64_t L = blockIdx.x, s = L >> 3;
-    mfma3_tile<R, BIG>(D, P, st, F, a0 + (int)(s % na), (s / na) * 8 + (L & 7), T, (int8_t(*)[kM3Stage])lds);
+    const int a = a0 + (int)(s % na);
+    mfma3_tile<R, BIG>(D, P, st, F, a, (s / na) * 8 + m3_turn((int)(L & 7), a, T, 2, D), T, (int8_t(*)[kM3Stage])lds);
 }
 
 // Wide tile: one workgroup takes first SNP a and a whole 64 x 64 tile of
@@ -2455,6 +2605,7 @@ __device__ __forceinline__ void mfma3w_tile(const DevData &D, const ScanParams &
     int nmarked = 0;
     static_for<4>([&](auto BB) __attribute__((always_inline)) {
         constexpr int bb = decltype(BB)::value;
+        if (!__ballot(ok >> 4 * bb & 15)) return;   // no triple of the scan
         v4i lo[4];
 #pragma unroll
         for (int xy = 0; xy < 4; ++xy) lo[xy] = 4 * bb + xy < kM3wKeep ? keep[4 * bb + xy] : stash[4 * bb + xy];
@@ -2518,7 +2669,8 @@ k_mfma3w(const DevData D, const ScanParams P, TopState *st, const Fp4Image F, in
     __shared__ __attribute__((aligned(1024))) int8_t lds[R][kM3wStage];
     // block order as in k_mfma3 (XCD L % 8 takes tiles u = 8 i + L % 8)
     const int64_t L = blockIdx.x, s = L >> 3;
-    mfma3w_tile<R>(D, P, st, F, a0 + (int)(s % na), (s / na) * 8 + (L & 7), T, lds);
+    const int a = a0 + (int)(s % na);
+    mfma3w_tile<R>(D, P, st, F, a, (s / na) * 8 + m3_turn((int)(L & 7), a, T, 1, D), T, lds);
 }
 
 
@@ -2849,16 +3001,27 @@ k_big_finish(const Cand *work, uint32_t L, Cand *top, uint32_t N, TopState *st, 
     }
 }
 
+// `wait`: candidates that may wait for the next launch's merge (0 after the last
+// launch): below that many this one ends at once, 5 us instead of the 38 that
+// 76 merges of a top-1,000 each took (50,000 x 32,000).  `host`: pinned memory
+// that takes the state and the list (the search's two copies took 15 us).
 __global__ void __launch_bounds__(1024)
 k_merge(TopState *st, Cand *top, const Cand *cand, uint32_t N, uint32_t cap, uint32_t chunk_id,
-        uint32_t *redo)
+        uint32_t *redo, uint32_t wait, char *host)
 {
     __shared__ Cand buf[kMergeSlots];
     __shared__ uint32_t psum[1024];
+    if (wait && !st->overflow && st->cand_count < wait) return;
     merge_topn(st, top, cand, N, cap, buf, psum);
     if (threadIdx.x == 0 && st->overflow) {
         redo[st->redo_count++] = chunk_id;
         st->overflow = 0;
+    }
+    if (host) {
+        __syncthreads();
+        const uint32_t n_top = st->n_top;
+        if (threadIdx.x == 0) *(TopState *)host = *st;
+        for (uint32_t i = threadIdx.x; i < n_top; i += 1024) ((Cand *)(host + sizeof(TopState)))[i] = top[i];
     }
 }
 
@@ -2984,7 +3147,9 @@ k_batch_mfma(const BatchJob *__restrict__ jobs, const BatchSeg *__restrict__ seg
             if (su < j1) mfma2w_tile<kBatchM2wKeep>(D, P, st, F, su, (int)(l % 32), J.T, (int8_t(*)[kM2wStage])lds);
         } else {
             const int64_t su = j0 + (int64_t)(l / 64) * 8 + x;
-            if (su < j1) mfma2_tile<true>(D, P, st, F, su, (int)(l % 64), J.T, *(Mfma2Lds<true> *)lds);
+            int ta, tb;
+            super_tile(su, (int)(l % 64), J.T, ta, tb);
+            if (su < j1) mfma2_tile<true>(D, P, st, F, ta, tb, J.T, *(Mfma2Lds<true> *)lds);
         }
     }
 }
@@ -3433,7 +3598,14 @@ hipError_t launch_mfma2(const DevData &D, const ScanParams &P, TopState *st, int
     F.class_off[1] = fp4_image_units(D, 0);
     if (tile == 2) hipLaunchKernelGGL(k_mfma2x, grid, block, 0, s, D, P, st, F, s0, s1, T);
     else if (tile == 1) hipLaunchKernelGGL(k_mfma2w, grid, block, 0, s, D, P, st, F, s0, s1, T);
-    else if (fp4) hipLaunchKernelGGL((k_mfma2<true>), grid, block, 0, s, D, P, st, F, s0, s1, T);
+    // whole scans of up to 64 super-blocks in the bands' order (scan us,
+    // super-blocks / bands: 1,000 x 4,000 39.5 / 37, 3,000 x 20,000 219 / 189,
+    // 5,003 x 9,001 256 / 256, 8,000 x 5,000 465 / 493)
+    else if (fp4 && s0 == 0 && s1 == mfma2_superblocks(T) && s1 <= 64) {
+        const int rows = (T + 7) / 8;
+        const int64_t last = band_start(rows - 1, T) + 8 * (T - 8 * (rows - 1)), per_xcd = (last + 7) / 8;
+        hipLaunchKernelGGL((k_mfma2<true>), dim3((unsigned)(8 * per_xcd)), block, 0, s, D, P, st, F, -1, last, T);
+    } else if (fp4) hipLaunchKernelGGL((k_mfma2<true>), grid, block, 0, s, D, P, st, F, s0, s1, T);
     else hipLaunchKernelGGL((k_mfma2<false>), grid, block, 0, s, D, P, st, F, s0, s1, T);
     return hipGetLastError();
 }
@@ -3501,9 +3673,9 @@ hipError_t launch_pair_table(const DevData &D, const ScanParams &P, uint32_t *pa
 }
 
 hipError_t launch_merge(TopState *st, Cand *top, const Cand *cand, uint32_t N, uint32_t cap, uint32_t chunk_id,
-                        uint32_t *redo, hipStream_t s)
+                        uint32_t *redo, uint32_t wait, void *host, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_merge, dim3(1), dim3(1024), 0, s, st, top, cand, N, cap, chunk_id, redo);
+    hipLaunchKernelGGL(k_merge, dim3(1), dim3(1024), 0, s, st, top, cand, N, cap, chunk_id, redo, wait, (char *)host);
     return hipGetLastError();
 }
 

@@ -41,8 +41,8 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint32_t voff, i
 // (vmcnt N; lgkm and exp counters not waited on).
 template <int N> __device__ __forceinline__ void wait_vmcnt()
 {
-    static_assert(N >= 0 && N < 16, "vmcnt immediate");
-    __builtin_amdgcn_s_waitcnt(0x0f70 | N);
+    static_assert(N >= 0 && N < 64, "vmcnt immediate");   // bits 3:0 and 15:14
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | N >> 4 << 14);
 }
 
 // wait_vmcnt<L * s>() for a runtime, wave-uniform s (clamped to 0 .. S).

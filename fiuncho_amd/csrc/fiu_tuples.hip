@@ -28,15 +28,18 @@ namespace {
 
 constexpr int ipow(int b, int e) { return e == 0 ? 1 : b * ipow(b, e - 1); }
 
-enum TupleMode { kScore = 0, kSample = 1, kTable = 2 };
+// kSampleSmall: the sampling pass in tiles of 16 b rows
+enum TupleMode { kScore = 0, kSample = 1, kTable = 2, kSampleSmall = 3 };
+constexpr bool samples(int mode) { return mode == kSample || mode == kSampleSmall; }
 
 // Shape of one kernel: W waves, NB blocks of 16 b rows against 16 W c columns,
 // wave w taking columns c0 + 16 w ..; NB is the most whose accumulators (4
-// registers per product and block) stay at 128 or below, so that two waves
-// per SIMD fit.  Two waves per workgroup where the column range of a head is
+// registers per product and block) stay at 144 or below, so that two waves
+// per SIMD fit (order 2 with uncalled genotypes, 9 products: NB = 4 560 us on
+// 4,001 x 8,999, NB = 2 655, whose 18 KB per 72 products outran the loads).  Two waves per workgroup where the column range of a head is
 // short (order 4 runs on a few hundred SNPs) or the staged c rows outweigh
 // the shared b rows (all cells); four where the b rows do.
-template <int K, bool ALL> struct Tup {
+template <int K, bool ALL, int MODE = kScore> struct Tup {
     static constexpr int G = ALL ? 3 : 2;            // genotype rows per SNP
     static constexpr int H = K - 2;                  // head SNPs
     static constexpr int M = ipow(G, H);             // head cells
@@ -44,20 +47,22 @@ template <int K, bool ALL> struct Tup {
     static constexpr int W = K == 4 || (K == 3 && ALL) ? 2 : 4;
     static constexpr int threads = 64 * W;
     static constexpr int CT = 16 * W;                // c columns per workgroup
-    static constexpr int NB = dots <= 8 ? 4 : dots == 9 ? 2 : dots == 16 ? 2 : 1;
+    static constexpr int NB = MODE == kSampleSmall ? 1 : dots <= 9 ? 4 : dots == 16 ? 2 : 1;
     static constexpr int BT = 16 * NB;               // b rows per workgroup
     static constexpr int b_rows = G * BT;            // LDS rows (64 bytes) per stage
     static constexpr int c_rows = G * CT;
     static constexpr int a_rows = G * H;             // per wave: every wave has its own copy
     static constexpr int stage = (b_rows + c_rows + W * a_rows) * 64;
-    static constexpr int ring = 4;                   // stages in LDS, ring - 1 in flight
+    // stages in LDS, ring - 1 in flight: 4, or 3 where two workgroups per CU
+    // would not fit
+    static constexpr int ring = 2 * 4 * stage <= 160 * 1024 ? 4 : 3;
     static constexpr int b_units = b_rows * 4 / W;   // 16-byte units of the b rows a wave loads
     static constexpr int b_loads = (b_units + 63) / 64;
     static constexpr int loads = b_loads + G + (H > 0 ? 1 : 0);   // per wave and stage
     static constexpr int inst = 4 * NB;              // combinations per lane
     static constexpr int cells = ipow(3, K);
     static constexpr int pairs = (dots + 1) / 2;     // words of one class's packed counts
-    static_assert(loads * (ring - 2) < 16, "vmcnt immediate");
+    static_assert(loads * (ring - 2) < 64, "vmcnt immediate");
 };
 
 __device__ __forceinline__ int swz16(int r) { return (r >> 1) & 3; }
@@ -319,9 +324,9 @@ __device__ __forceinline__ float packed_screen(const uint32_t (&m)[CELLS], const
 template <int K, bool ALL, int MODE>
 __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P, TopState *st, const TupleArgs &A,
                                            const Head<K - 2> &hd, int bmin, int c0,
-                                           int8_t (*lds)[Tup<K, ALL>::stage], uint32_t *lds_hist)
+                                           int8_t (*lds)[Tup<K, ALL, MODE>::stage], uint32_t *lds_hist)
 {
-    using Z = Tup<K, ALL>;
+    using Z = Tup<K, ALL, MODE>;
     constexpr int G = Z::G, H = Z::H, NB = Z::NB, R = Z::ring;
     const int n = D.n, np = D.n_pad;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -554,7 +559,7 @@ __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P
         } else {
             uint32_t m[Z::cells];
             cells_of(cur, m);
-            if constexpr (MODE == kSample) {
+            if constexpr (samples(MODE)) {
                 const float ms = packed_screen<Z::cells>(m, P);
                 if (valid) atomicAdd(&lds_hist[hist_bin(ms)], 1u);
             } else if (valid && bound_passes(packed_bound<Z::cells>(m, P), tau, P.delta)) {
@@ -606,12 +611,16 @@ __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P
 // on 2,500 x 16,000, step 8, the scan fetched 129 GB beyond L2 with free
 // tiles and 4.3 with aligned ones, 39 -> 26 ms.
 template <int K, bool ALL, int MODE>
-__global__ void __launch_bounds__((Tup<K, ALL>::threads)) __attribute__((amdgpu_waves_per_eu(MODE == kSample ? 1 : 2, 2)))
+__global__ void __launch_bounds__((Tup<K, ALL, MODE>::threads)) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_tuples(const DevData D, const ScanParams P, TopState *st, const TupleArgs A)
 {
-    using Z = Tup<K, ALL>;
-    __shared__ __attribute__((aligned(1024))) int8_t lds[Z::ring][Z::stage];
-    __shared__ uint32_t lds_hist[MODE == kSample ? kHistBins : 1];
+    using Z = Tup<K, ALL, MODE>;
+    // one array: beside a second one the compiler waits for every pending
+    // direct-to-LDS load ahead of each stage's reads (a sampling pass of
+    // 5,003 x 9,001: 76 us so, 29 with the histogram behind the ring)
+    __shared__ __attribute__((aligned(1024))) int8_t lds_all[Z::ring * Z::stage + (samples(MODE) ? 4 * kHistBins : 0)];
+    int8_t(*const lds)[Z::stage] = (int8_t(*)[Z::stage])lds_all;
+    uint32_t *const lds_hist = (uint32_t *)(lds_all + (samples(MODE) ? Z::ring * Z::stage : 0));
     const int64_t L = blockIdx.x, s = L >> 3;
     if constexpr (K == 3 && MODE == kScore) {
         if (A.aligned) {
@@ -630,28 +639,42 @@ k_tuples(const DevData D, const ScanParams P, TopState *st, const TupleArgs A)
             return;
         }
     }
-    const int64_t i = s % A.units, first = s / A.units * 8 + ((L + (i >> 6)) & 7);
+    // (a sample has few tiles per unit: the XCDs take turns sooner)
+    constexpr int turn = !samples(MODE) ? 6 : K == 2 ? 3 : 0;
+    const int64_t i = s % A.units, first = s / A.units * 8 + ((L + (i >> turn)) & 7);
     const int64_t u = P.j0 + i * A.stride;
     const Head<Z::H> hd = head_at<K>(P, D.n, K == 2 ? 0 : (uint64_t)u);
-    hist_begin<MODE == kSample>(lds_hist);
-    int64_t tile = first;
-    uint32_t pick = MODE == kSample ? (uint32_t)(u % A.tile_stride) * 5u + (uint32_t)first : 0;
+    // sampling: the unit's tiles at multiples of tile_stride, from its own first
+    const int64_t ts = samples(MODE) ? A.tile_stride : 1;
+    int64_t tile = first * ts;
     int64_t bmin = hd.b_first;
     if constexpr (K == 2) bmin += u * Z::BT * P.step;
+    // an order-2 sample takes whole column tiles of the table, the same ones
+    // for eight units in a row, which one XCD runs: their c rows stay in its L2
+    // (50,000 x 32,000: 1.4 -> 0.8 ms)
+    const int64_t skip = K == 2 && samples(MODE) ? (bmin + 1) / Z::CT : 0;
+    if constexpr (samples(MODE)) {
+        const int64_t at = (K == 2 ? u / 8 : u) % ts * 5 + skip;
+        tile += (ts - at % ts) % ts;
+    }
+    bool any = false;   // a workgroup without a tile leaves the histogram alone
     while (bmin < D.n - 1) {
-        const int ct = (int)(D.n - 1 - bmin + Z::CT - 1) / Z::CT;   // column tiles past bmin
+        // column tiles past bmin
+        const int64_t from = K == 2 && samples(MODE) ? skip * Z::CT : bmin + 1;
+        const int ct = (int)(D.n - from + Z::CT - 1) / Z::CT;
         if (tile < ct) {
-            if (MODE != kSample || pick % (uint32_t)A.tile_stride == 0)
-                tuple_tile<K, ALL, MODE>(D, P, st, A, hd, (int)bmin, (int)bmin + 1 + Z::CT * (int)tile, lds, lds_hist);
-            tile += 8 * (int64_t)A.rounds;
-            pick += 8 * (uint32_t)A.rounds;
+            if (!any) hist_begin<samples(MODE)>(lds_hist);
+            any = true;
+            tuple_tile<K, ALL, MODE>(D, P, st, A, hd, (int)bmin, (int)from + Z::CT * (int)tile, lds, lds_hist);
+            tile += 8 * (int64_t)A.rounds * ts;
         } else {
             if constexpr (K == 2) break;
             tile -= ct;
             bmin += (int64_t)Z::BT * P.step;
         }
     }
-    hist_end<MODE == kSample>(lds_hist, P.hist);
+    if (!any) return;
+    hist_end<samples(MODE)>(lds_hist, P.hist);
 }
 
 // fp4 image of genotype rows 0 .. G - 1, as the two-row image of the pair
@@ -685,7 +708,7 @@ __global__ void k_tuple_singles(DevData D, uint32_t *out)
 template <int K, bool ALL, int MODE>
 hipError_t launch_tuples_as(const DevData &D, ScanParams P, TopState *st, TupleArgs A, hipStream_t s)
 {
-    using Z = Tup<K, ALL>;
+    using Z = Tup<K, ALL, MODE>;
     // a dispatch holds at most 2^32 - 1 work-items
     constexpr int64_t max_blocks = (int64_t)(0xffffffffu / (uint32_t)Z::threads);
     int64_t units = (P.j1 - P.j0 + A.stride - 1) / A.stride;
@@ -699,10 +722,11 @@ hipError_t launch_tuples_as(const DevData &D, ScanParams P, TopState *st, TupleA
         // one workgroup per unit and tile; units padded to whole classes
         A.rounds = (int32_t)((most + 7) / 8);
     } else {
-        // a unit's tiles dealt in rounds of 8: no more rounds than fill the
-        // device
+        // a unit's (sampled) tiles dealt in rounds of 8: no more rounds than
+        // fill the device
         const int64_t want = std::max<int64_t>(1, (int64_t)A.fill / std::max<int64_t>(1, 8 * units));
-        A.rounds = (int32_t)std::min<int64_t>((most + 7) / 8, want);
+        const int64_t taken = samples(MODE) ? (most + A.tile_stride - 1) / A.tile_stride : most;
+        A.rounds = (int32_t)std::min<int64_t>((taken + 7) / 8, want);
     }
     const int64_t per_launch = std::max<int64_t>(1, max_blocks / (8 * (int64_t)A.rounds) / 2);
     for (int64_t i = 0; i < units; i += per_launch) {
@@ -729,14 +753,16 @@ hipError_t launch_tuples_k(const DevData &D, const ScanParams &P, TopState *st, 
 {
     if constexpr (!ALL && K <= 3)
         if (A.out) return launch_tuples_as<K, ALL, kTable>(D, P, st, A, s);
+    if (P.hist && A.small) return launch_tuples_as<K, ALL, kSampleSmall>(D, P, st, A, s);
     if (P.hist) return launch_tuples_as<K, ALL, kSample>(D, P, st, A, s);
     return launch_tuples_as<K, ALL, kScore>(D, P, st, A, s);
 }
 
 }  // namespace
 
-int tuple_b_block(int order, bool all_cells)
+int tuple_b_block(int order, bool all_cells, bool small)
 {
+    if (small) return 16;
     if (all_cells) return order == 2 ? Tup<2, true>::BT : Tup<3, true>::BT;
     return order == 2 ? Tup<2, false>::BT : order == 3 ? Tup<3, false>::BT : Tup<4, false>::BT;
 }
