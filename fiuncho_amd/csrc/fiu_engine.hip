@@ -146,6 +146,7 @@ struct Job {
     // plan
     int kind = kKindDirect2, pw = 1, chunks = 1, tiles = 1;
     bool wide = false;   // matrix-core kinds: the 64 x 64 / 64 x 128 tiles
+    int tile = 0;        // the same kinds in a launch of their own: launch_mfma2's tile, launch_mfma3's ring
     // units of work: prefixes (popcount kinds), first SNPs (order 3 on the
     // matrix cores) or super-blocks (order 2 on the matrix cores)
     int64_t n_pref = 0, next = 0, given = 0, seed = 1;
@@ -381,7 +382,7 @@ void Engine::plan_job(Job *j)
     // slice is then the whole scan, not the doubling slices that raise the
     // threshold from nothing
     const double combos = (double)j->prefixes * (double)(n - M) / (double)(M + 1);
-    const bool sampled = tables && combos >= (double)(1 << 18) && d->cases < (1u << 16) && d->ctrls < (1u << 16);
+    const bool sampled = tables && combos >= (double)(1 << 16) && d->cases < (1u << 16) && d->ctrls < (1u << 16);
     auto sample = [&](bool matrix) {
         if (!sampled) return;
         j->sample = plan_sample(order, n, j->step, j->offset, total_prefixes, j->prefixes, j->outputs, 1u << 16,
@@ -413,7 +414,11 @@ void Engine::plan_job(Job *j)
         const uint64_t samples = (uint64_t)d->cases + d->ctrls;
         bool wide = samples >= 8192 && (uint64_t)n >= (order == 3 ? 2048u : 16384u);
         if (tuned_algo == FIU_ALGO_MFMA && te.batch_unit) wide = te.batch_unit == 2;
-        j->wide = wide && d->cases < (1u << 16) && d->ctrls < (1u << 16);
+        const bool pairs16 = d->cases < (1u << 16) && d->ctrls < (1u << 16);
+        const bool chosen = tuned_algo == FIU_ALGO_MFMA && te.batch_unit;
+        j->wide = wide && pairs16;
+        if (order == 3) j->tile = (chosen ? wide : n >= 768) && pairs16 ? 6 : 4;
+        else j->tile = !pairs16 ? 0 : chosen ? wide : samples < 8192 ? 0 : n >= 16384 ? 2 : n >= 8192 ? 1 : 0;
         j->pw = 1;
         j->n_pref = order == 2 ? mfma2_superblocks(T) : std::max(0, n - 2);
         // cost of one combination in the wave-instruction currency of the
@@ -677,11 +682,18 @@ bool Engine::launch_step()
         R.est_instr += range_cost(j, a, b);
         return true;
     };
-    std::vector<std::tuple<Job *, int64_t, int64_t>> tuples;
+    // launches of their own: the scans around a head, and large ranges of the
+    // matrix-core kinds outside an arena, whose own kernels are faster than the
+    // persistent one (290 KB of code for four tiles, spilled queue state): the
+    // searches of a batch of 16 took 12.1 ms in it, 9.9 each by itself.  Below
+    // kOwnRange (50 to 100 us) the persistent kernel packs ranges better.
+    constexpr double kOwnRange = 4e7;
+    std::vector<std::tuple<Job *, int64_t, int64_t>> own;
     auto add_seg = [&](Job *j, int64_t a, int64_t b) {
-        if (batch_mfma(j->kind)) return add_mseg(j, a, b);
-        if (j->kind == kKindTuples) {
-            tuples.emplace_back(j, a, b);
+        const bool mfma = batch_mfma(j->kind);
+        if (mfma && (j->ds->arena || range_cost(j, a, b) < kOwnRange)) return add_mseg(j, a, b);
+        if (mfma || j->kind == kKindTuples) {
+            own.emplace_back(j, a, b);
             R.ranges.emplace_back(j, a, b);
             R.est_instr += range_cost(j, a, b);
             return true;
@@ -767,15 +779,22 @@ bool Engine::launch_step()
               "step descriptor");
     check(hipEventRecord(ev_start_[parity], stream_), "event");
     uint64_t heads = 0;
-    for (auto &t : tuples) {
+    for (auto &t : own) {
         const Job *j = std::get<0>(t);
+        const DevData &D = j->ds->dev;
+        TopState *st = jobs_h_[j->slot].st;
         ScanParams P = jobs_h_[j->slot].P;
         P.j0 = std::get<1>(t);
         P.j1 = std::get<2>(t);
         heads += (uint64_t)(P.j1 - P.j0);
-        check(launch_tuples(j->order, j->all_cells, j->ds->dev, P, jobs_h_[j->slot].st,
-                            tuple_args(j->ds, j->order, j->all_cells), stream_),
-              "scan launch");
+        if (j->kind == kKindTuples)
+            check(launch_tuples(j->order, j->all_cells, D, P, st, tuple_args(j->ds, j->order, j->all_cells), stream_),
+                  "scan launch");
+        else if (j->kind == kKindMfma2)
+            check(launch_mfma2(D, P, st, P.j0, P.j1, D.n_pad / 64, j->ds->fp4.p, j->tile, stream_), "scan launch");
+        else
+            check(launch_mfma3(D, P, st, j->ds->fp4.p, (int)P.j0, (int)P.j1, D.n_pad / 64, j->tile, stream_),
+                  "scan launch");
     }
     check(hipGraphLaunch(exec_, stream_), "step graph launch");
     check(hipEventRecord(ev_end_[parity], stream_), "event");

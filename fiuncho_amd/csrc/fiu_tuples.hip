@@ -272,29 +272,38 @@ __device__ __forceinline__ float ctrls_of(uint32_t w) { return (float)(w >> 16);
 // the MI among the called, and that MI is below its own chi2/M; a single
 // pass over the cells' sum (packed words add without carry) gives n_c, n_t.
 // The added logarithms err by less than 1e-6, inside bound_passes' margin.
-template <int CELLS>
-__device__ __forceinline__ float packed_bound(const uint32_t (&m)[CELLS], const ScanParams &P)
+struct BoundTerms {
+    float frac, scale, base;
+};
+__device__ __forceinline__ BoundTerms bound_terms(float nc, float nt, const ScanParams &P)
 {
-    float frac = P.frac_c, scale = P.chi_scale, base = 0.0f;
-    if (!P.bounded) {
+    BoundTerms t;
+    const float all = nc + nt, r = __builtin_amdgcn_rcpf(fmaxf(all, 1.0f));
+    t.frac = nc * r;
+    const float lc = __builtin_amdgcn_logf(fmaxf(t.frac, 7.9e-31f));
+    const float lt = __builtin_amdgcn_logf(fmaxf(nt * r, 7.9e-31f));
+    t.base = fmaf(fmaf(nc, lc, nt * lt), P.inv_n * 0.69314718f, P.hy);
+    t.scale = nc > 0.0f && nt > 0.0f ? all * P.inv_n * (all * __builtin_amdgcn_rcpf(nc)) * __builtin_amdgcn_rcpf(nt)
+                                     : 0.0f;
+    return t;
+}
+
+// FIXED: the terms are the same for every table (all cover the samples of `t`).
+template <bool FIXED, int CELLS>
+__device__ __forceinline__ float packed_bound(const uint32_t (&m)[CELLS], const ScanParams &P, BoundTerms t)
+{
+    if constexpr (!FIXED) {
         uint32_t sum = 0;
 #pragma unroll
         for (int x = 0; x < CELLS; ++x) sum += m[x];
-        const float nc = cases_of(sum), nt = ctrls_of(sum), all = nc + nt;
-        const float r = __builtin_amdgcn_rcpf(fmaxf(all, 1.0f));
-        frac = nc * r;
-        const float lc = __builtin_amdgcn_logf(fmaxf(frac, 7.9e-31f));
-        const float lt = __builtin_amdgcn_logf(fmaxf(nt * r, 7.9e-31f));
-        base = fmaf(fmaf(nc, lc, nt * lt), P.inv_n * 0.69314718f, P.hy);
-        scale = nc > 0.0f && nt > 0.0f ? all * P.inv_n * (all * __builtin_amdgcn_rcpf(nc)) * __builtin_amdgcn_rcpf(nt)
-                                       : 0.0f;
+        t = bound_terms(cases_of(sum), ctrls_of(sum), P);
     }
-    return base + mi_bound_fn<CELLS>(
-                      [&](int x, float &fc, float &fx) __attribute__((always_inline)) {
-                          fc = cases_of(m[x]);
-                          fx = fc + ctrls_of(m[x]);
-                      },
-                      frac, scale);
+    return t.base + mi_bound_fn<CELLS>(
+                        [&](int x, float &fc, float &fx) __attribute__((always_inline)) {
+                            fc = cases_of(m[x]);
+                            fx = fc + ctrls_of(m[x]);
+                        },
+                        t.frac, t.scale);
 }
 
 template <int CELLS>
@@ -535,7 +544,29 @@ __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P
     };
     uint32_t pend = 0;
     const int i1 = 4 * hi;
-    Loaded<K, ALL> cur, nxt;
+    Loaded<K, ALL> cur;
+    if constexpr (MODE == kScore) {
+        // U instances at a time, without a branch, so that their chains overlap
+        constexpr int U = K <= 3 ? 2 : 1;
+        const BoundTerms fixed = P.bounded ? BoundTerms{P.frac_c, P.chi_scale, 0.0f}
+                                           : bound_terms(cases_of(total), ctrls_of(total), P);
+#pragma unroll 1
+        for (int i = 4 * lo; i < i1; i += U) {
+            Loaded<K, ALL> x[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) load(i + u, x[u]);
+            uint32_t marks = 0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                uint32_t m[Z::cells];
+                cells_of(x[u], m);
+                const float bound = packed_bound<!ALL>(m, P, fixed);
+                marks |= (uint32_t)(bound_passes(bound, tau, P.delta) & valid_at(b_at(i + u))) << u;
+            }
+            pend |= marks << i;
+        }
+    } else {
+    Loaded<K, ALL> nxt;
     load(4 * lo, cur);
 #pragma unroll 1
     for (int i = 4 * lo; i < i1; ++i) {
@@ -559,14 +590,11 @@ __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P
         } else {
             uint32_t m[Z::cells];
             cells_of(cur, m);
-            if constexpr (samples(MODE)) {
-                const float ms = packed_screen<Z::cells>(m, P);
-                if (valid) atomicAdd(&lds_hist[hist_bin(ms)], 1u);
-            } else if (valid && bound_passes(packed_bound<Z::cells>(m, P), tau, P.delta)) {
-                pend |= 1u << i;
-            }
+            const float ms = packed_screen<Z::cells>(m, P);
+            if (valid) atomicAdd(&lds_hist[hist_bin(ms)], 1u);
         }
         cur = nxt;
+    }
     }
     if constexpr (MODE == kScore) {
         // one marked combination per lane and round: screen, exact MI, push
