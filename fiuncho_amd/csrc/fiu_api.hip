@@ -738,8 +738,12 @@ ThresholdSample plan_sample(int order, int n, int64_t step, int64_t offset, uint
     // 98,000 pairs of 5,003 x 9,001 the scan took 255 to 400 us as the sample
     // had more or fewer pairs of the SNPs with an effect, with 262,144 255
     // (sampling 29 us); 524,288 cost 100 us more on 300 x 3,000 triples
-    const double floor = tup ? std::max(32768.0, std::min(combos / 8.0, 262144.0)) : 32768.0;
-    const double want = std::min(std::min(std::max({combos / 128.0, floor, 8.0 * expect}),
+    const double floor = tup ? std::max(32768.0, std::min(combos / 8.0, 262144.0)) : 16384.0;
+    // The popcount scans take the exact MI of up to 729 cells a lane each, so
+    // they sample more for long lists, one in 16 at most (order 5 on
+    // 68 x 3,113, top-1,000: 57.9 ms with one in 128, 41.6 with one in 16)
+    const double spread = tup ? 128.0 : std::min(128.0, std::max(16.0, 1600.0 / std::max(outputs, 1u)));
+    const double want = std::min(std::min(std::max({combos / spread, floor, 8.0 * expect}),
                                           std::max(8388608.0, 2.0 * expect)),
                                  (double)target);
     S.step = std::max<int64_t>(1, (int64_t)(combos / std::max(want, 1.0)));
