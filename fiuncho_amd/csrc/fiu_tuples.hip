@@ -328,8 +328,8 @@ __device__ __forceinline__ float packed_screen(const uint32_t (&m)[CELLS], const
 // the cycles; the products of its 16 x 16 blocks take 8.8), a share of order
 // 3 on 2,500 x 16,000 18 ms (9.7).  Counts wait as 16-bit pairs and the
 // epilogue loads an instance ahead: the whole order-4 scan 35 -> 21 ms.
-// b rows bmin + step * (0 .. BT - 1), of which those above hd.last and below
-// the column count; columns c0 + (0 .. CT - 1).
+// b rows bmin + step * (0 .. BT - 1), of which those from hd.b_first on and
+// below the column count; columns c0 + (0 .. CT - 1).
 template <int K, bool ALL, int MODE>
 __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P, TopState *st, const TupleArgs &A,
                                            const Head<K - 2> &hd, int bmin, int c0,
@@ -366,14 +366,14 @@ __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P
     const int rr = lane & 15, kc = lane >> 4;
     const int fo = rr * 64 + ((kc ^ swz16(rr)) << 4), ao = kc << 4;
     // the 16-row b blocks [lo, hi) with a combination among the wave's columns:
-    // rows above the head, below the last column (a wave without any stages
-    // and waits with the others)
+    // rows from the head's first b on, below the last column (a wave without
+    // any stages and waits with the others)
     const int c_top = std::min(c0 + 16 * w + 15, n - 1);
     int lo = 0, hi = 0;
 #pragma unroll
     for (int bb = 0; bb < NB; ++bb) {
         const int64_t first = (int64_t)bmin + (int64_t)P.step * (16 * bb);
-        if (first + 15 * (int64_t)P.step <= hd.last) lo = bb + 1;
+        if (first + 15 * (int64_t)P.step < hd.b_first) lo = bb + 1;
         if (first < c_top && c0 + 16 * w < n) hi = bb + 1;
     }
     lo = __builtin_amdgcn_readfirstlane(lo);
@@ -508,7 +508,9 @@ __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P
     const float tau = MODE == kScore ? st->tau : 0.0f;
     const uint64_t tau_combo = MODE == kScore ? st->tau_combo : 0;
     auto b_at = [&](int i) { return (int64_t)bmin + (int64_t)P.step * (16 * (i >> 2) + 4 * kc + (i & 3)); };
-    auto valid_at = [&](int64_t b) { return c_ok && b < c && b > hd.last; };
+    // (an aligned block starts below b_first, and in the head where the share's
+    // offset falls, members of the progression above the head lie before it)
+    auto valid_at = [&](int64_t b) { return c_ok && b < c && b >= hd.b_first; };
     // columns at or below the head (aligned tiles) read a valid one's tables
     const uint32_t c_tab = (uint32_t)std::max(c, hd.last + 2);
     const uint32_t total = D.total[0] | D.total[1] << 16;
