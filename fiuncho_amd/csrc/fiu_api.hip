@@ -148,6 +148,7 @@ void finish_upload(fiu_dataset *d, const uint64_t *words)
     check(hipMemcpyAsync(fl, d->flags.p, sizeof(fl), hipMemcpyDeviceToHost, d->stream), "flags");
     check(hipStreamSynchronize(d->stream), "singles sync");
     D.uniform = (n > 0 && fl[0] == 0) ? 1 : 0;
+    D.packs = !(fl[0] & 2) && fl[3] < (1u << 16);
     D.total[0] = fl[1];
     D.total[1] = fl[2];
 }
@@ -379,6 +380,7 @@ fiu_dataset *stage_dataset(const uint64_t *words, size_t snps, size_t cw, size_t
     D.ctrls = ctrls;
     D.singles = d->singles.p;
     D.uniform = uniform ? 1 : 0;
+    D.packs = uniform && total[0] < (1u << 16) && total[1] < (1u << 16);
     D.total[0] = total[0];
     D.total[1] = total[1];
     if (order == 3 && uniform) {
@@ -835,7 +837,7 @@ bool tuple_scan(const fiu_dataset *d, int order, int64_t step, int64_t n_pref)
 {
     const double n = (double)d->snps, combos = (double)n_pref * (n - order + 1) / order;
     const bool fits = !d->dev.uniform ? order <= 3 : order == 4 || (order <= 3 && step > 1);
-    return fits && d->cases < (1u << 16) && d->ctrls < (1u << 16) && n >= 48 &&
+    return fits && counts16(d->dev) && n >= 48 &&
            combos * ((double)d->cases + (double)d->ctrls) >= 2e9;
 }
 
@@ -1131,7 +1133,7 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     // 26.3 / 25.4, 2,000 x 8,000 44.3 / 38.4)
     int ring = algo == FIU_ALGO_MFMA && order == 3 && variant ? variant
                                                               : (n >= 768 ? 6 : 4);
-    if (ring >= 5 && (d->cases >= (1u << 16) || d->ctrls >= (1u << 16) || !ws.private_memory())) ring = 4;
+    if (ring >= 5 && (!counts16(d->dev) || !ws.private_memory())) ring = 4;
     // matrix-core scans walk super-blocks of 8 x 8 tiles of 64 x 64 pairs;
     // fp4 operands accumulate in fp32, exact while every count is below 2^24;
     // they come from the dataset's fp4 image (int8 when it is not there)
@@ -1149,8 +1151,7 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     // 1.44 / 1.67 / 1.94)
     const bool m2_auto = variant == 0 && samples >= 8192;
     const int m2_pick = variant == 4 || (m2_auto && n >= 16384) ? 2 : variant == 3 || (m2_auto && n >= 8192) ? 1 : 0;
-    const int m2_tile = order == 2 && d->cases < (1u << 16) && d->ctrls < (1u << 16) && ws.private_memory()
-                            ? m2_pick : 0;
+    const int m2_tile = order == 2 && counts16(d->dev) && ws.private_memory() ? m2_pick : 0;
 
     // chunk plan: even chunks of about `target` combinations (at most
     // max_chunks of them); before the first, a sampling pass histograms the
@@ -1192,8 +1193,8 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     }
     if (plan.count > max_chunks) fail(FIU_ERR_UNSUPPORTED, "too many launches for this entry point");
     const bool sample = plan.count > 0 && !(cfg && (cfg->flags & FIU_FLAG_NO_THRESHOLD_SAMPLE));
-    const bool tup_sample = sample && (tup || (algo == FIU_ALGO_MFMA && d->cases < (1u << 16) &&
-                                               d->ctrls < (1u << 16) && mfma_fp4 && ws.tuples(d, order - 1, false, s)));
+    const bool tup_sample = sample && (tup || (algo == FIU_ALGO_MFMA && counts16(d->dev) && mfma_fp4 &&
+                                               ws.tuples(d, order - 1, false, s)));
     const ThresholdSample TS =
         sample ? plan_sample(order, n, step, offset, total_prefixes, (int64_t)n_pref, outputs, cap, target, tup_sample,
                              algo == FIU_ALGO_MFMA)

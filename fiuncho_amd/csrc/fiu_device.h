@@ -37,8 +37,17 @@ struct DevData {
     const uint32_t *singles; // [n_pad][2][3] popcount of each row
     uint32_t total[2];       // samples covered per class (uniform datasets)
     int32_t uniform;         // 1 if every SNP covers the same samples
-    int32_t pad_;
+    int32_t packs;           // 1 if no sample has two genotypes of a SNP and no class of a
+                             // SNP's rows holds 2^16 bits or more (counts16)
 };
+
+// Whether the counts of any table, and their sums over its cells, fit 16 bits
+// in each class.  The class sizes alone do not say: a row may hold more bits
+// than its class has samples.
+__host__ __device__ inline bool counts16(const DevData &D)
+{
+    return D.packs && D.cases < (1u << 16) && D.ctrls < (1u << 16);
+}
 
 // A top-N candidate: float MI, then the combination as its lexicographic
 // rank among the k-combinations of the dataset's SNPs (prefix_key), so that

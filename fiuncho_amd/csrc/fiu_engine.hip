@@ -382,7 +382,7 @@ void Engine::plan_job(Job *j)
     // slice is then the whole scan, not the doubling slices that raise the
     // threshold from nothing
     const double combos = (double)j->prefixes * (double)(n - M) / (double)(M + 1);
-    const bool sampled = tables && combos >= (double)(1 << 16) && d->cases < (1u << 16) && d->ctrls < (1u << 16);
+    const bool sampled = tables && combos >= (double)(1 << 16) && counts16(d->dev);
     auto sample = [&](bool matrix) {
         if (!sampled) return;
         j->sample = plan_sample(order, n, j->step, j->offset, total_prefixes, j->prefixes, j->outputs, 1u << 16,
@@ -414,7 +414,7 @@ void Engine::plan_job(Job *j)
         const uint64_t samples = (uint64_t)d->cases + d->ctrls;
         bool wide = samples >= 8192 && (uint64_t)n >= (order == 3 ? 2048u : 16384u);
         if (tuned_algo == FIU_ALGO_MFMA && te.batch_unit) wide = te.batch_unit == 2;
-        const bool pairs16 = d->cases < (1u << 16) && d->ctrls < (1u << 16);
+        const bool pairs16 = counts16(d->dev);
         const bool chosen = tuned_algo == FIU_ALGO_MFMA && te.batch_unit;
         j->wide = wide && pairs16;
         if (order == 3) j->tile = (chosen ? wide : n >= 768) && pairs16 ? 6 : 4;
@@ -470,8 +470,7 @@ void prepare_tuples(Job *j, hipStream_t s)
 {
     fiu_dataset *d = j->ds;
     const uint64_t n = d->snps;
-    if (d->arena || j->order > 4 || j->step < 1 || j->offset < 0 || n < (uint64_t)j->order || d->cases >= (1u << 16) ||
-        d->ctrls >= (1u << 16))
+    if (d->arena || j->order > 4 || j->step < 1 || j->offset < 0 || n < (uint64_t)j->order || !counts16(d->dev))
         return;
     const uint64_t all = binom_sat(n, (uint64_t)j->order - 1);
     const uint64_t pref = all > (uint64_t)j->offset ? (all - (uint64_t)j->offset + (uint64_t)j->step - 1) / (uint64_t)j->step : 0;

@@ -275,8 +275,8 @@ inline uint32_t *pair_table(const fiu_dataset *d) { return d->pair.p + kPairSlac
 bool ensure_fp4_image(fiu_dataset *d, hipStream_t s);
 // fp4 image of all three genotype rows; false when it does not fit.
 bool ensure_tuple_image(fiu_dataset *d, hipStream_t s);
-// Tables of 1 .. m SNPs' counts (TupleTables, m <= 3; classes below 2^16
-// samples, every SNP covering the same ones) and the fp4 image they are
+// Tables of 1 .. m SNPs' counts (TupleTables, m <= 3; datasets with counts16,
+// every SNP covering the same samples) and the fp4 image they are
 // counted from; false when they do not fit, or would take more than a quarter
 // of the free device memory.
 bool ensure_tuple_tables(fiu_dataset *d, int m, hipStream_t s);

@@ -76,7 +76,7 @@ hipError_t launch_mi_batch(const uint32_t *tables, uint64_t n, uint64_t ct_size,
 // Combinations around a head of order - 2 SNPs on the matrix cores
 // (fiu_tuples.hip).  Counts of m SNPs in table t[m]: per m-combination, in
 // lexicographic rank order, 2^m words (genotypes 0 and 1, first SNP most
-// significant), cases | controls << 16; every class below 2^16 samples.
+// significant), cases | controls << 16; datasets with counts16.
 struct TupleTables {
     const uint32_t *t[4];
 };

@@ -1393,7 +1393,7 @@ __device__ __forceinline__ void mfma2_tile(const DevData &D, const ScanParams &P
         }
     }
     if constexpr (FP4) {
-        if (D.cases < (1u << 16) && D.ctrls < (1u << 16)) {
+        if (counts16(D)) {
             // Two passes: the bound of the lane's 16 pairs, those that pass
             // with their counts (word g * 2 + h: cases | controls << 16) in
             // the wave's quarter of the ring, which nothing reads any more;
@@ -2092,7 +2092,7 @@ __device__ __forceinline__ uint32_t m3_valid(const ScanParams &P, const M3Lane &
 // One workgroup's work item: first SNP a, tile u (see k_mfma3); returns at
 // once for items outside the triangle.  Every wave of the workgroup calls it
 // with the same arguments.  R: stages of the LDS ring (R - 1 in flight).
-// BIG: classes of 2^16 samples or more (2: find out at run time).
+// BIG: counts above 16 bits (not counts16; 2: find out at run time).
 template <int R, int BIG>
 __device__ __forceinline__ void mfma3_tile(const DevData &D, const ScanParams &P, TopState *st, const Fp4Image &F,
                                            int a, int64_t u, int T, int8_t (*lds)[kM3Stage])
@@ -2257,7 +2257,7 @@ __device__ __forceinline__ void mfma3_tile(const DevData &D, const ScanParams &P
     // the wave's quarter of the workgroup's LDS (kM3Lds bytes): nothing reads
     // the ring any more
     int8_t *const mine = (int8_t *)lds + w * (kM3Lds / 4);
-    const bool big = BIG == 1 || (BIG == 2 && (D.cases >= (1u << 16) || D.ctrls >= (1u << 16)));
+    const bool big = BIG == 1 || (BIG == 2 && !counts16(D));
     if (BIG != 1 && !big) {
         // two passes: the bound of the eight instances (bb, j), every
         // accumulator index a constant; then the marked ones
@@ -3286,13 +3286,15 @@ __global__ void k_transpose(const uint64_t *__restrict__ src, uint4 *__restrict_
 __global__ void k_singles(const uint4 *__restrict__ bits, DevData D, uint32_t *singles, uint32_t *flags)
 {
     // one thread per (SNP, class): popcount of each row, disjointness of the
-    // rows and equality of their union with the union of SNP 0.
+    // rows and equality of their union with the union of SNP 0; flags[0] bit 0
+    // where either fails, bit 1 where the first does, flags[3] the most bits of
+    // a SNP's rows in a class
     const int id = blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= D.n_pad * 2) return;
     const int s = id >> 1, cls = id & 1;
     const uint4 *base = bits + D.class_off[cls];
     const int np = D.n_pad;
-    uint32_t cnt[3] = {0, 0, 0}, bad = 0, ucnt = 0;
+    uint32_t cnt[3] = {0, 0, 0}, twice = 0, other = 0, ucnt = 0;
     for (int q = 0; q < D.quads[cls]; ++q) {
         const uint4 *row = base + (size_t)q * 3 * np;
         const uint4 r0 = row[s], r1 = row[np + s], r2 = row[2 * np + s];
@@ -3304,14 +3306,16 @@ __global__ void k_singles(const uint4 *__restrict__ bits, DevData D, uint32_t *s
             cnt[0] += __builtin_popcount(a);
             cnt[1] += __builtin_popcount(b);
             cnt[2] += __builtin_popcount(c);
-            bad |= (a & b) | (a & c) | (b & c) | ((a | b | c) ^ ref);
+            twice |= (a & b) | (a & c) | (b & c);
+            other |= (a | b | c) ^ ref;
             ucnt += __builtin_popcount(ref);
         }
     }
     singles[(s * 2 + cls) * 3 + 0] = cnt[0];
     singles[(s * 2 + cls) * 3 + 1] = cnt[1];
     singles[(s * 2 + cls) * 3 + 2] = cnt[2];
-    if (s < D.n && bad) atomicOr(&flags[0], 1u);
+    if (s < D.n && (twice | other)) atomicOr(&flags[0], twice ? 3u : 1u);
+    if (s < D.n) atomicMax(&flags[3], cnt[0] + cnt[1] + cnt[2]);
     if (s == 0) flags[1 + cls] = ucnt;
 }
 
@@ -3646,7 +3650,7 @@ hipError_t launch_mfma3(const DevData &D, const ScanParams &P, TopState *st, con
         return hipSuccess;
     }
     const dim3 grid((unsigned)(tiles8 * na * 8)), block(kBlock);
-    const bool big = D.cases >= (1u << 16) || D.ctrls >= (1u << 16);
+    const bool big = !counts16(D);
     if (ring == 3 && big) hipLaunchKernelGGL((k_mfma3<3, 1>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
     else if (ring == 3) hipLaunchKernelGGL((k_mfma3<3, 0>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
     else if (ring == kM3Ring && big) hipLaunchKernelGGL((k_mfma3<kM3Ring, 1>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);

@@ -11,7 +11,7 @@
 // form (any dataset): genotypes 0, 1 and 2, 3^k products and no tables.
 //
 // Counts of a combination travel as one 32-bit word per cell, cases in the
-// low half and controls in the high half (every class below 2^16 samples):
+// low half and controls in the high half (datasets with counts16):
 // the inclusion-exclusion then runs on both classes with one subtraction,
 // since every intermediate value is itself a pair of counts and no half
 // borrows from the other.
