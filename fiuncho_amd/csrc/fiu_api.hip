@@ -516,7 +516,7 @@ bool ensure_pair_table(fiu_dataset *d, hipStream_t s)
         check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
         if (bytes + (64ull << 20) > free_b) return false;
     }
-    d->pair.alloc(pair_words(n));
+    if (!d->pair.try_alloc(pair_words(n))) return false;
     ScanParams P{};
     P.j0 = 0;
     P.j1 = (int64_t)n;
@@ -542,7 +542,7 @@ bool ensure_fp4_image(fiu_dataset *d, hipStream_t s)
         check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
         if (units * 16 + (64ull << 20) > free_b) return false;
     }
-    d->fp4.alloc(units);
+    if (!d->fp4.try_alloc(units)) return false;
     check(launch_fp4_image(d->dev, d->fp4.p, s), "fp4 image launch");
     check(hipStreamSynchronize(s), "fp4 image sync");
     d->fp4_ready = true;
@@ -564,7 +564,7 @@ bool ensure_tuple_image(fiu_dataset *d, hipStream_t s)
     if (d->fp4x_ready) return true;
     const uint64_t units = 12ull * (d->dev.quads[0] + d->dev.quads[1]) * d->dev.n_pad;
     if (!room_for(d, units * 16, false)) return false;
-    d->fp4x.alloc(units);
+    if (!d->fp4x.try_alloc(units)) return false;
     check(launch_tuple_image(d->dev, d->fp4x.p, s), "fp4 image launch");
     check(hipStreamSynchronize(s), "fp4 image sync");
     d->fp4x_ready = true;
@@ -596,6 +596,12 @@ bool ensure_tuple_tables(fiu_dataset *d, int m, hipStream_t s)
     }
     if (bytes == 0) return true;
     if (!room_for(d, bytes, true)) return false;
+    // (free memory may still be gone, or in pieces, by the time it is asked for)
+    for (int j = d->tup_ready + 1; j <= m; ++j)
+        if (!d->tup[j].try_alloc(binom_sat(n, (uint64_t)j) << j)) {
+            for (int i = d->tup_ready + 1; i < j; ++i) d->tup[i].release();
+            return false;
+        }
     TupleArgs A{};
     A.F = tuple_image(d, false);
     A.stride = 1;
@@ -605,7 +611,6 @@ bool ensure_tuple_tables(fiu_dataset *d, int m, hipStream_t s)
     P.step = 1;
     P.binom = binom;
     for (int j = d->tup_ready + 1; j <= m; ++j) {
-        d->tup[j].alloc(binom_sat(n, (uint64_t)j) << j);
         if (j == 1) {
             check(launch_tuple_singles(d->dev, d->tup[1].p, s), "singles table launch");
         } else {

@@ -110,20 +110,28 @@ template <class T> struct DBuf {
         n = 0;
         return q;
     }
-    void alloc(size_t count)
+    // false, and empty, when there is no memory for it
+    bool try_alloc(size_t count)
     {
-        if (count <= n && p) return;
+        if (count <= n && p) return true;
         release();
         const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
         if (arena) {
             p = (T *)arena->alloc(bytes);
-            if (!p) fail(FIU_ERR_NOMEM, "scan server memory budget exhausted (" + std::to_string(bytes) + " bytes)");
         } else if (hipMalloc(&p, bytes) != hipSuccess) {
             p = nullptr;
             (void)hipGetLastError();
-            fail(FIU_ERR_NOMEM, "device allocation of " + std::to_string(bytes) + " bytes failed");
         }
+        if (!p) return false;
         n = count;
+        return true;
+    }
+    void alloc(size_t count)
+    {
+        if (try_alloc(count)) return;
+        const std::string bytes = std::to_string(std::max<size_t>(count, 1) * sizeof(T)) + " bytes";
+        fail(FIU_ERR_NOMEM, arena ? "scan server memory budget exhausted (" + bytes + ")"
+                                  : "device allocation of " + bytes + " failed");
     }
 };
 
