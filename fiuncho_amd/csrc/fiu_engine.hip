@@ -917,7 +917,7 @@ class Server {
   private:
     void ingest_main();
     void sched_main();
-    size_t footprint(const Job *j) const;
+    size_t footprint(const Job *j, bool padding = true) const;
     size_t host_footprint(const Job *j) const;
     bool fits(const Job *j) const;
     void release_staging(Job *j);
@@ -992,12 +992,14 @@ Server::~Server()
     if (ingest_stream_) (void)hipStreamDestroy(ingest_stream_);
 }
 
-size_t Server::footprint(const Job *j) const
+// `padding`: with the pair table's (a request that fits only without it is
+// admitted when the device is free and runs the kernels that need no table)
+size_t Server::footprint(const Job *j, bool padding) const
 {
     if (j->ds) return 0;  // resident dataset: nothing to upload
     size_t b = dataset_bytes(j->snps, j->cw, j->tw) + staging_bytes(j->snps, j->cw, j->tw);
     b += (size_t)(j->order + 1) * (j->snps + 1) * 8 + Arena::kAlign;   // binomial table (rows up to k)
-    if (j->order == 3) b += pair_table_bytes(j->snps) + Arena::kAlign;
+    if (j->order == 3) b += pair_table_bytes(j->snps) - (padding || j->snps < 2 ? 0 : 2 * kPairSlack * 32) + Arena::kAlign;
     // the fp4 image of the matrix-core scans is not counted: it is allocated
     // at upload only when it fits, else the popcount kinds scan the dataset
     return b;
@@ -1048,8 +1050,9 @@ uint64_t Server::submit(const fiu_request *req)
         j->tw = req->ctrls_words;
         j->cases = req->cases;
         j->ctrls = req->ctrls;
-        if (footprint(j.get()) > arena_->capacity())
-            fail(FIU_ERR_REJECTED, "request needs " + std::to_string(footprint(j.get())) +
+        const size_t need = footprint(j.get(), false);
+        if (need > arena_->capacity())
+            fail(FIU_ERR_REJECTED, "request needs " + std::to_string(need) +
                                        " device bytes, above the server's memory budget");
         j->words.assign(req->words, req->words + req->snps * 3 * (req->cases_words + req->ctrls_words));
     }
