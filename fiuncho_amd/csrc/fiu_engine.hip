@@ -389,7 +389,7 @@ void Engine::plan_job(Job *j)
                                 UINT64_MAX, true, matrix);
         j->seed = j->n_pref;
     };
-    if ((tuned_algo == FIU_ALGO_AUTO || order >= 4) && tables && tuple_scan(d, order, j->step, j->prefixes)) {
+    if (tuned_algo == FIU_ALGO_AUTO && tables && tuple_scan(d, order, j->step, j->prefixes)) {
         j->kind = kKindTuples;
         j->pw = 1;
         j->n_pref = tuple_units(order, j->all_cells, (uint64_t)n, j->prefixes);

@@ -10,7 +10,9 @@ table is loaded into the library, where AUTO searches and batched scans of
 that class use it.  ``autotune_batch`` then times ``fiu_search_batch`` over a
 few datasets of each batch class with every unit size of the batched
 popcount kernels, or both batched tiles of the matrix-core kernels (the
-entry's ``batch_unit``), and keeps the fastest.
+entry's ``batch_unit``), and keeps the fastest.  An entry fixes its class's
+algorithm, so a class whose candidates are all slower than the choice without
+an entry (the scans around a head at order 4) gets none.
 
     entries = tune.autotune()          # times the default classes, loads the table
     entries = tune.autotune_batch()    # adds the batched kernels' unit sizes / tiles
@@ -130,6 +132,12 @@ def _time(search, d, order, dist, outputs, repeats):
     return best, res
 
 
+# The choice without an entry is kept where it is this much faster: 3 to 20
+# times at order 4 where it is another kernel, and a run's noise where it is one
+# of the candidates.
+DEFAULT_GAIN = 1.5
+
+
 def autotune(classes: Iterable[ShapeClass] = DEFAULT_CLASSES, outputs: int = 50, repeats: int = 2,
              seed: int = 7, apply: bool = True, log=None) -> List[Entry]:
     """Time every candidate of every class; returns the table (and loads it
@@ -162,6 +170,13 @@ def autotune(classes: Iterable[ShapeClass] = DEFAULT_CLASSES, outputs: int = 50,
                         f"{t * 1e3:.2f} ms")
                 if best is None or t < best[0]:
                     best = (t, algo, var)
+            # orders above 3: the choice without an entry may be none of the
+            # candidates
+            if best is not None and sc.order > 3:
+                s = GpuSearch()
+                s.run_arrays(d, sc.order, dist, outputs)
+                if _time(s, d, sc.order, dist, outputs, repeats)[0] < best[0] / DEFAULT_GAIN:
+                    best = None
             d.close()
             if best is not None:
                 entries.append(Entry(sc.order, sc.snps_lo, sc.snps_hi, sc.samples_lo, sc.samples_hi,
@@ -209,7 +224,7 @@ def autotune_batch(classes: Iterable[BatchClass] = DEFAULT_BATCH_CLASSES, units:
     """Time fiu_search_batch over each class's datasets with every unit size
     (popcount kinds) or both tiles (a class whose entry is on the matrix
     cores); the fastest goes into the class's table entry (added when the
-    table has none for it).  Returns the whole table (loaded when `apply`).
+    table has none for it, unless the batch is faster without one).  Returns the whole table (loaded when `apply`).
     Raises if two candidates disagree on a result."""
     from . import Dataset, Distribution, search_batch, synth_spec
     saved = get_table()
@@ -249,10 +264,20 @@ def autotune_batch(classes: Iterable[BatchClass] = DEFAULT_BATCH_CLASSES, units:
                         f"{t * 1e3:.2f} ms")
                 if best is None or t < best[0]:
                     best = (t, u)
+            keep = True
+            if not same:
+                # without an entry (timed as the units are, its tables built)
+                set_table(rest)
+                t = float("inf")
+                for _ in range(max(repeats, 2)):
+                    t0 = time.perf_counter()
+                    search_batch(scans)
+                    t = min(t, time.perf_counter() - t0)
+                keep = t >= best[0] / DEFAULT_GAIN
             for d in dss:
                 d.close()
             table = rest + [Entry(base.order, base.snps_lo, base.snps_hi, base.samples_lo, base.samples_hi,
-                                  base.algorithm, base.variant, base.ms, best[1])]
+                                  base.algorithm, base.variant, base.ms, best[1])] if keep else rest
     except BaseException:
         set_table(saved)
         raise

@@ -1,0 +1,62 @@
+"""GPU: which kernels a search takes.  A tuning entry and the options that
+name a kernel are honoured also where AUTO has a scan around a head, and such
+a scan is left alone where it would be the slower one.  Kernels that count
+differently also cut their scans differently, so the launches of an explicit
+algorithm, or the units of a batch, tell which one ran."""
+import math
+
+import numpy as np
+import pytest
+
+import fiuncho_amd as fa
+from fiuncho_amd import tune
+
+from .test_zz_no_alloc import run_static
+
+pytestmark = pytest.mark.gpu
+
+AUTO, DIRECT, MARGINAL, MFMA = fa.ALGO_AUTO, fa.ALGO_DIRECT, fa.ALGO_MARGINAL, fa.ALGO_MFMA
+
+
+@pytest.fixture(autouse=True)
+def empty_table():
+    tune.clear()
+    yield
+    tune.clear()
+
+
+def run(d, order, dist, outputs, **conf):
+    s = fa.GpuSearch(**conf)
+    r = s.run_arrays(d, order, dist, outputs)
+    return r, s.last_stats
+
+
+def same(a, b):
+    return a[0].tolist() == b[0].tolist() and np.array_equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("algorithm", [DIRECT, MARGINAL])
+def test_order4_tuning_entry_is_honoured(algorithm):
+    print(f"case: order-4 entry {algorithm}", flush=True)
+    d = fa.Dataset.synth(fa.synth_spec(98, 300, 324, seed=61))
+    dist = fa.Distribution(98, 3)
+    chunk = 3000
+    want, explicit = run(d, 4, dist, 50, algorithm=algorithm, chunk_combos=chunk)
+    auto, plain = run(d, 4, dist, 50, chunk_combos=chunk)
+    assert plain.launches != explicit.launches    # AUTO's scan around a head is another one
+    tune.set_table([tune.Entry(4, 0, 1000, 0, 100000, algorithm)])
+    got, stats = run(d, 4, dist, 50, chunk_combos=chunk)
+    assert stats.algorithm == algorithm and stats.launches == explicit.launches
+    batched, bs = fa.search_batch([(d, 4, dist, 50)])
+    assert bs.units >= math.comb(98, 3)           # prefixes; a scan around a head has C(98, 2) heads
+    for r in (auto, got, batched[0]):
+        assert same(r, want)
+    d.close()
+
+
+def test_batch_tuner_adds_no_entry_slower_than_the_default():
+    print("case: batch tuner, order 4 above the size of the scan around a head", flush=True)
+    table = tune.autotune_batch([tune.BatchClass(4, 0, 1000, 0, 100000, 140, 4000, count=2)], units=(0, 4), repeats=2)
+    assert not [e for e in table if e.order == 4]
+    table = tune.autotune([tune.ShapeClass(4, 0, 1000, 0, 100000, 120, 2000)], outputs=20, repeats=1)
+    assert not [e for e in table if e.order == 4]
