@@ -1107,7 +1107,12 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     // against 110; with 1 % uncalled, order 3 on 601 x 6,007 3.9 ms against
     // 17.5 and order 2 on 4,001 x 8,999 0.87 ms against 3.2
     const bool tup_all = !d->dev.uniform;
-    const bool tup = algo_req == FIU_ALGO_AUTO && tuple_scan(d, order, step, (int64_t)n_pref) &&
+    // (not where the caller names a kernel, by its operand format or by a variant
+    // of the algorithm that would run instead)
+    const int instead = !d->dev.uniform ? FIU_ALGO_DIRECT : order == 2 ? FIU_ALGO_MFMA : FIU_ALGO_MARGINAL;
+    const bool named = (variant != 0 && valid_variant(instead, order, variant)) ||
+                       (instead == FIU_ALGO_MFMA && cfg && (cfg->flags & FIU_FLAG_MFMA_INT8));
+    const bool tup = algo_req == FIU_ALGO_AUTO && !named && tuple_scan(d, order, step, (int64_t)n_pref) &&
                      ws.tuples(d, order - 1, tup_all, s);
     if (algo_req != FIU_ALGO_DIRECT && d->dev.uniform && order >= 4 && order <= kMaxKmOrder)
         algo = FIU_ALGO_MARGINAL;

@@ -60,3 +60,22 @@ def test_batch_tuner_adds_no_entry_slower_than_the_default():
     assert not [e for e in table if e.order == 4]
     table = tune.autotune([tune.ShapeClass(4, 0, 1000, 0, 100000, 120, 2000)], outputs=20, repeats=1)
     assert not [e for e in table if e.order == 4]
+
+
+@pytest.mark.parametrize("order,snps,conf", [
+    (2, 1100, {"mfma_int8": True}),
+    (2, 1100, {"variant": 2}),
+    (3, 220, {"variant": 2}),
+])
+def test_options_that_name_a_kernel_keep_it_on_shares(order, snps, conf):
+    print(f"case: order {order} share with {conf}", flush=True)
+    d = fa.Dataset.synth(fa.synth_spec(snps, 9000, 8000, seed=62))
+    dist = fa.Distribution(snps, order - 1, 3, 1)
+    chunk = 262144 if order == 2 else 5000
+    want, explicit = run(d, order, dist, 50, algorithm=MFMA if order == 2 else MARGINAL, chunk_combos=chunk, **conf)
+    auto, plain = run(d, order, dist, 50, chunk_combos=chunk)
+    assert plain.launches != explicit.launches
+    got, stats = run(d, order, dist, 50, chunk_combos=chunk, **conf)
+    assert stats.launches == explicit.launches and stats.variant == explicit.variant
+    assert same(got, want) and same(auto, want)
+    d.close()
