@@ -13,6 +13,8 @@ from fiuncho_amd import tune
 
 from .test_zz_no_alloc import run_static
 
+from .test_zz_no_alloc import run_static
+
 pytestmark = pytest.mark.gpu
 
 AUTO, DIRECT, MARGINAL, MFMA = fa.ALGO_AUTO, fa.ALGO_DIRECT, fa.ALGO_MARGINAL, fa.ALGO_MFMA
@@ -78,4 +80,14 @@ def test_options_that_name_a_kernel_keep_it_on_shares(order, snps, conf):
     got, stats = run(d, order, dist, 50, chunk_combos=chunk, **conf)
     assert stats.launches == explicit.launches and stats.variant == explicit.variant
     assert same(got, want) and same(auto, want)
+    d.close()
+
+
+def test_static_search_of_a_share_has_the_pair_table_of_an_earlier_search():
+    print("case: static share", flush=True)
+    d = fa.Dataset.synth(fa.synth_spec(200, 4700, 4700, seed=63))
+    dist = fa.Distribution(200, 2, 3, 1)
+    want = fa.GpuSearch().run_arrays(d, 3, dist, 40)
+    got = run_static(d, 3, dist, 40)
+    assert got[2].algorithm == MARGINAL and same(got, want)
     d.close()
