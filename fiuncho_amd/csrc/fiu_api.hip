@@ -833,17 +833,52 @@ TupleArgs tuple_args(const fiu_dataset *d, int order, bool all_cells)
     return A;
 }
 
+// A tile around a head takes nearly the same time however few of its rows are
+// in the share, so a sparse share is the popcount kernels': they take the
+// share's prefixes only, four or one to a wavefront.  The times of both in
+// microseconds, from the sizes (fitted to 70 shares of 300 to 20,000 SNPs x
+// 1,000 to 40,000 samples, steps 2 to 100,000: the faster one was picked in
+// each where they differ by more than 15 %):
+// - around a head, per 16-row block with a member of the share and per column
+//   tile (at order 3 with every SNP called also per 64-row tile; at order 4 22 ns
+//   per head, member or not);
+// - by popcount, what the samples and cells of its combinations take, and the
+//   chain of the longest wavefront, a head's every column tile, quad by quad.
+// Order 3, 5,000 SNPs x 4,000 samples: step 128 18.2 ms around a head, 19.4 by
+// popcount; step 1,024 11.8 and 4.2.  Order 4, 500 x 8,000, step 1,000: 9.0 and
+// 6.4; 240 x 16,000, step 64: 6.4 and 9.9.
+static bool dense_share(const fiu_dataset *d, int order, double step, double n_pref)
+{
+    const double n = (double)d->snps, s = (double)d->cases + (double)d->ctrls;
+    const double width = (n - order + 1) / order, combos = n_pref * width;   // columns per prefix, on average
+    const double chain = n / 64.0 * (s / 128.0);
+    // heads with a member: all but those among the last `step` b's
+    const double heads = order == 3 ? n : n * (n - 1) / 2;
+    const double with = step >= n ? n_pref : order == 3 ? n - step / 2 : heads - step * (n / 2 - step / 6);
+    const double live = std::min(with, n_pref), blocks = n_pref / 16 + live, tiles = n_pref / 64 + live;
+    if (order == 4)
+        return n_pref * (width + 32) * (s + 600) / 5.6e6 + 2 * chain >=
+               0.022 * heads + (width / 32 + 0.5) * blocks * (0.034 + 4.3e-6 * s);
+    if (!d->dev.uniform)
+        return combos * (s + 100) / 1.5e7 + 0.5 * chain >= (width / 32 + 0.5) * blocks * (0.024 + 6.3e-6 * s);
+    return combos * (s + 750) / 4.5e7 + 0.7 * chain >=
+           (width / 64 + 0.5) * (tiles * (0.045 + 5.8e-6 * s) + blocks * (0.012 + 1.4e-6 * s));
+}
+
 // Its tables, launches and half-empty tiles cost a few tenths of a
-// millisecond: measured at order 4 on 60 SNPs x 4,000 samples (2.0e9
-// combinations x samples) 0.88 ms against 1.28, on 40 x 4,000 (3.7e8) 0.73
-// against 0.49; an order-3 share on 300 x 4,000 (4.5e9) 0.51 against 0.53, on
-// 150 x 4,000 (5.5e8) 0.39 against 0.38.
+// millisecond, which small scans do not earn back, least of all shares of
+// order 2: measured around a head and otherwise, a share (4) of order 2 on
+// 1,000 SNPs x 8,000 samples (1.0e9 combinations x samples) 117 us and 96, on
+// 3,000 x 800 (9.0e8) 109 and 119; order 3 with 1 % uncalled on 40 x 16,000
+// (1.6e8) 219 and 215, on 100 x 4,000 (6.5e8) 171 and 245; order 4 on
+// 40 x 4,000 (3.7e8) 309 and 480.  The first search also builds the tables
+// (order 4 on 100 x 4,000: 0.3 ms), hence one line above all of these.
 bool tuple_scan(const fiu_dataset *d, int order, int64_t step, int64_t n_pref)
 {
     const double n = (double)d->snps, combos = (double)n_pref * (n - order + 1) / order;
     const bool fits = !d->dev.uniform ? order <= 3 : order == 4 || (order <= 3 && step > 1);
-    return fits && counts16(d->dev) && n >= 48 &&
-           combos * ((double)d->cases + (double)d->ctrls) >= 2e9;
+    return fits && counts16(d->dev) && n >= 48 && combos * ((double)d->cases + (double)d->ctrls) >= 2e9 &&
+           (step == 1 || order == 2 || dense_share(d, order, (double)step, (double)n_pref));
 }
 
 }  // namespace fiu
