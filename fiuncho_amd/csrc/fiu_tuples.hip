@@ -77,8 +77,7 @@ __device__ __forceinline__ uint32_t pair_index_u32(uint32_t x, uint32_t y, uint3
 // (the share's prefixes (head, b)), below n - 1.
 template <int H> struct Head {
     int s[H > 0 ? H : 1];
-    int last;        // largest head SNP (-1 without a head)
-    int b_first;     // n - 1 or above: no prefix of the share
+    int b_first;     // above the head; n - 1 or above: no prefix of the share
 };
 
 template <int K>
@@ -86,12 +85,11 @@ __device__ __forceinline__ Head<K - 2> head_at(const ScanParams &P, int n, uint6
 {
     constexpr int H = K - 2;
     Head<H> r;
-    r.last = -1;
+    r.b_first = 0;
     if constexpr (H > 0) {
         unrank(h, n, H, P.binom, r.s);
-        r.last = r.s[H - 1];
+        r.b_first = r.s[H - 1] + 1;
     }
-    r.b_first = r.last + 1;
     if (P.step != 1 || P.offset != 0) {
         // rank of the prefix (head, b) = r0 + b
         const uint64_t stride = (uint64_t)n + 1;
@@ -511,8 +509,8 @@ __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P
     // (an aligned block starts below b_first, and in the head where the share's
     // offset falls, members of the progression above the head lie before it)
     auto valid_at = [&](int64_t b) { return c_ok && b < c && b >= hd.b_first; };
-    // columns at or below the head (aligned tiles) read a valid one's tables
-    const uint32_t c_tab = (uint32_t)std::max(c, hd.last + 2);
+    // columns up to the first b (aligned tiles) read a valid one's tables
+    const uint32_t c_tab = (uint32_t)std::max(c, hd.b_first + 1);
     const uint32_t total = D.total[0] | D.total[1] << 16;
     Subsets<K> S;
     if constexpr (!ALL && MODE != kTable) subsets_at<K>(S, A.T, P, n, hd);
@@ -524,8 +522,8 @@ __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P
         if constexpr (!ALL && MODE != kTable) {
             // a combination outside the scan reads a valid one's tables
             const int64_t b = b_at(i);
-            const bool ok = b < c && b > hd.last;
-            load_tables<K>(x.t, S, ok ? (uint32_t)b : (uint32_t)(hd.last + 1), c_tab, (uint32_t)n);
+            const bool ok = b < c && b >= hd.b_first;
+            load_tables<K>(x.t, S, ok ? (uint32_t)b : (uint32_t)hd.b_first, c_tab, (uint32_t)n);
         }
     };
     // both classes' counts of each product, cases | controls << 16
