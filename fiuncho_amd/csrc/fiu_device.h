@@ -198,12 +198,24 @@ struct BatchHeader {
 };
 
 // Marginal pair table: per pair 8 words, for (x, y) in {0, 1}^2 the case counts
-// f(x, y), then the case + control counts, as FP32 (exact below 2^24 samples;
-// the matrix-core epilogue reads them without a conversion); on datasets with
-// 2^24 samples or more integers, case counts then control counts.  kPairSlack
-// entries of padding on both sides: a tile's lanes past the last SNP, or with b
-// above c, read there and are dropped, with no select per address.
-__host__ __device__ inline bool pair_float(const DevData &D) { return (uint64_t)D.cases + D.ctrls < (1u << 24); }
+// f(x, y), then those of both classes (pair_sums) or of the controls, as FP32
+// while that is exact (pair_float; the matrix-core epilogue reads them without
+// a conversion), else as integers.  kPairSlack entries of padding on both sides:
+// a tile's lanes past the last SNP, or with b above c, read there and are
+// dropped, with no select per address.
+__host__ __device__ inline uint32_t class_bits(const DevData &D, int cls)
+{
+    const uint32_t samples = cls ? D.ctrls : D.cases;
+    return samples > D.total[cls] ? samples : D.total[cls];
+}
+__host__ __device__ inline bool pair_float(const DevData &D)
+{
+    return class_bits(D, 0) < (1u << 24) && class_bits(D, 1) < (1u << 24);
+}
+__host__ __device__ inline bool pair_sums(const DevData &D)
+{
+    return (uint64_t)class_bits(D, 0) + class_bits(D, 1) < (1u << 24);
+}
 constexpr uint64_t kPairSlack = 4096;
 __host__ __device__ inline uint64_t pair_words(uint64_t n) { return ((n < 2 ? 0 : n * (n - 1) / 2) + 2 * kPairSlack) * 8; }
 

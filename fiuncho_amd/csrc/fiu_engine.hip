@@ -685,12 +685,14 @@ bool Engine::launch_step()
     // matrix-core kinds outside an arena, whose own kernels are faster than the
     // persistent one (290 KB of code for four tiles, spilled queue state): the
     // searches of a batch of 16 took 12.1 ms in it, 9.9 each by itself.  Below
-    // kOwnRange (50 to 100 us) the persistent kernel packs ranges better.
+    // kOwnRange (50 to 100 us) the persistent kernel packs ranges better.  Order 3
+    // on 2^24 samples or more has its kernel among the single search's only.
     constexpr double kOwnRange = 4e7;
     std::vector<std::tuple<Job *, int64_t, int64_t>> own;
     auto add_seg = [&](Job *j, int64_t a, int64_t b) {
         const bool mfma = batch_mfma(j->kind);
-        if (mfma && (j->ds->arena || range_cost(j, a, b) < kOwnRange)) return add_mseg(j, a, b);
+        const bool alone = j->kind == kKindMfma3 && !pair_sums(j->ds->dev);
+        if (mfma && !alone && (j->ds->arena || range_cost(j, a, b) < kOwnRange)) return add_mseg(j, a, b);
         if (mfma || j->kind == kKindTuples) {
             own.emplace_back(j, a, b);
             R.ranges.emplace_back(j, a, b);

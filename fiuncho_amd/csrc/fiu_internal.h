@@ -318,7 +318,7 @@ inline bool mfma_dataset(const fiu_dataset *d)
 {
     return d->dev.uniform && d->cases < (1u << 24) && d->ctrls < (1u << 24);
 }
-// Order 3 also reads the pair table as FP32 sums of both classes.
+// Order 3 also reads the pair table as FP32.
 inline bool mfma3_dataset(const fiu_dataset *d) { return mfma_dataset(d) && pair_float(d->dev); }
 
 // Top-N entries -> ascending SNP indices (order per entry, unranked from the

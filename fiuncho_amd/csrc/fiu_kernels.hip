@@ -856,10 +856,11 @@ __device__ __forceinline__ void scan2m_unit(const DevData &D, const ScanParams &
                     uint4 *o = (uint4 *)(pair_out + pair_index(pa[i], c, D.n) * 8);
                     if (pair_float(D)) {
                         float *fo = (float *)o;
+                        const bool sums = pair_sums(D);
 #pragma unroll
                         for (int x = 0; x < 4; ++x) {
                             fo[x] = (float)f[i][0][x];
-                            fo[4 + x] = (float)(f[i][0][x] + f[i][1][x]);
+                            fo[4 + x] = (float)(sums ? f[i][0][x] + f[i][1][x] : f[i][1][x]);
                         }
                     } else {
                         o[0] = make_uint4(f[i][0][0], f[i][0][1], f[i][0][2], f[i][0][3]);
@@ -912,7 +913,7 @@ k_scan2m(const DevData D, const ScanParams P, TopState *st, uint32_t *pair_out)
 }
 
 // A pair table entry as integer counts: cases f(x, y), then controls.
-__device__ __forceinline__ void pair_counts(const uint32_t *p, bool as_float, uint32_t (&f)[8])
+__device__ __forceinline__ void pair_counts(const uint32_t *p, bool as_float, bool sums, uint32_t (&f)[8])
 {
     const uint4 u = ((const uint4 *)p)[0], v = ((const uint4 *)p)[1];
     f[0] = u.x, f[1] = u.y, f[2] = u.z, f[3] = u.w, f[4] = v.x, f[5] = v.y, f[6] = v.z, f[7] = v.w;
@@ -920,7 +921,7 @@ __device__ __forceinline__ void pair_counts(const uint32_t *p, bool as_float, ui
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
             f[x] = (uint32_t)__uint_as_float(f[x]);
-            f[4 + x] = (uint32_t)__uint_as_float(f[4 + x]) - f[x];
+            f[4 + x] = (uint32_t)__uint_as_float(f[4 + x]) - (sums ? f[x] : 0u);
         }
     }
 }
@@ -959,7 +960,7 @@ __device__ __forceinline__ void scan3m_unit(const DevData &D, const ScanParams &
     const uint64_t tau_combo = st->tau_combo;
     const int np = D.n_pad, n = D.n;
     const uint32_t *pair = P.pair;
-    const bool pf = pair_float(D);
+    const bool pf = pair_float(D), ps = pair_sums(D);
     const int t_end = max(t_lo, (bmin + 1) >> 6);
     for (int t = min(t_hi, (np >> 6) - 1); t >= t_end; --t) {  // last tile first (shared in L2)
         const int c = (t << 6) | lane;
@@ -1040,11 +1041,11 @@ __device__ __forceinline__ void scan3m_unit(const DevData &D, const ScanParams &
             const bool valid = in_range && c > pb[i];
             uint32_t fac[8] = {0, 0, 0, 0, 0, 0, 0, 0}, fbc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
             if (valid) {
-                pair_counts(pair + pair_index(pa[i], c, n) * 8, pf, fac);
-                pair_counts(pair + pair_index(pb[i], c, n) * 8, pf, fbc);
+                pair_counts(pair + pair_index(pa[i], c, n) * 8, pf, ps, fac);
+                pair_counts(pair + pair_index(pb[i], c, n) * 8, pf, ps, fbc);
             }
             uint32_t pab[8];
-            pair_counts(pair + pair_index(pa[i], pb[i], n) * 8, pf, pab);
+            pair_counts(pair + pair_index(pa[i], pb[i], n) * 8, pf, ps, pab);
             const uint32_t *sa = D.singles + (size_t)pa[i] * 6;
             const uint32_t *sb = D.singles + (size_t)pb[i] * 6;
             uint32_t m0[27], m1[27];
@@ -1857,7 +1858,9 @@ __device__ __forceinline__ int64_t pair_rank(int32_t x, int32_t y, int32_t n)
 // Values of the order-3 matrix-core epilogue that depend only on the first
 // SNP a and the lane's last SNP c.  Counts are pairs in FP32 (exact): of the
 // cases ([0]) and of both classes ([1]) -- the table's second cells follow by
-// the same inclusion-exclusion, and the bound needs no sum per cell.
+// the same inclusion-exclusion, and the bound needs no sum per cell.  SPLIT: where
+// the sums would not be exact (2^24 samples or more, each class below), [1] is of
+// the controls.
 struct M3Lane {
     int c;
     bool c_ok;
@@ -1866,16 +1869,17 @@ struct M3Lane {
     int64_t rank_a;     // rank of the prefix (a, a + 1)
 };
 
-__device__ __forceinline__ void single_pair(const DevData &D, uint32_t s, float (&f)[2][2])
+template <bool SPLIT> __device__ __forceinline__ void single_pair(const DevData &D, uint32_t s, float (&f)[2][2])
 {
     const uint32_t *sp = D.singles + (size_t)s * 6;
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
         f[0][g] = (float)sp[g];
-        f[1][g] = (float)(sp[g] + sp[3 + g]);
+        f[1][g] = (float)(SPLIT ? sp[3 + g] : sp[g] + sp[3 + g]);
     }
 }
 
+template <bool SPLIT = false>
 __device__ __forceinline__ M3Lane m3_lane(const DevData &D, const ScanParams &P, int a, int c)
 {
     M3Lane L;
@@ -1884,22 +1888,22 @@ __device__ __forceinline__ M3Lane m3_lane(const DevData &D, const ScanParams &P,
     L.c_ok = c < n && c > a;
     L.rank_a = (int64_t)a * (2 * (int64_t)n - a - 1) / 2;
     L.ab = (const float4 *)P.pair + 2 * (L.rank_a - a - 1);
-    single_pair(D, a, L.sa);
-    single_pair(D, c, L.sc);   // c < n_pad: rows past the last SNP are zero
+    single_pair<SPLIT>(D, a, L.sa);
+    single_pair<SPLIT>(D, c, L.sc);   // c < n_pad: rows past the last SNP are zero
     const float4 u0 = L.ab[2 * (int64_t)c], u1 = L.ab[2 * (int64_t)c + 1];
     L.fac[0][0] = u0.x, L.fac[0][1] = u0.y, L.fac[0][2] = u0.z, L.fac[0][3] = u0.w;
     L.fac[1][0] = u1.x, L.fac[1][1] = u1.y, L.fac[1][2] = u1.z, L.fac[1][3] = u1.w;
     L.tot[0] = (float)D.total[0];
-    L.tot[1] = (float)(D.total[0] + D.total[1]);
+    L.tot[1] = (float)(SPLIT ? D.total[1] : D.total[0] + D.total[1]);
     return L;
 }
 
 // The triple (a, b, L.c): the 8 matrix-core counts cnt(k, x, y, z), x, y, z in
-// {0, 1}, k = 0 cases, 1 both classes, with the pair table (`bc`: the entry of
-// (b, L.c)), the singles and the totals give the 27 cells m0 (cases) and m1
-// (both classes), by inclusion-exclusion in FP32: the counts are exact
-// integers below 2^24, and so is every step.
-template <class C>
+// {0, 1}, k = 0 cases, 1 both classes (SPLIT: controls), with the pair table
+// (`bc`: the entry of (b, L.c)), the singles and the totals give the 27 cells m0
+// (cases) and m1, by inclusion-exclusion in FP32: the counts are exact integers
+// below 2^24, and so is every step.
+template <bool SPLIT = false, class C>
 __device__ __forceinline__ void m3_cells(const DevData &D, const M3Lane &L, uint32_t b, const float4 *bc, C &&cnt,
                                          float (&m0)[27], float (&m1)[27])
 {
@@ -1910,7 +1914,7 @@ __device__ __forceinline__ void m3_cells(const DevData &D, const M3Lane &L, uint
         fab[1][0] = p1.x, fab[1][1] = p1.y, fab[1][2] = p1.z, fab[1][3] = p1.w;
         fbc[0][0] = q0.x, fbc[0][1] = q0.y, fbc[0][2] = q0.z, fbc[0][3] = q0.w;
         fbc[1][0] = q1.x, fbc[1][1] = q1.y, fbc[1][2] = q1.z, fbc[1][3] = q1.w;
-        single_pair(D, b, sb);
+        single_pair<SPLIT>(D, b, sb);
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -1944,24 +1948,26 @@ __device__ __forceinline__ void m3_cells(const DevData &D, const M3Lane &L, uint
 }
 
 // The bound and the screen of such a table.
+template <bool SPLIT = false>
 __device__ __forceinline__ bool m3_bound_ok(const float (&m0)[27], const float (&m1)[27], float tau,
                                             const ScanParams &P)
 {
     return !P.bounded || bound_passes(mi_bound_fn<27>(
                                           [&](int x, float &fc, float &fx) __attribute__((always_inline)) {
                                               fc = m0[x];
-                                              fx = m1[x];
+                                              fx = SPLIT ? m0[x] + m1[x] : m1[x];
                                           },
                                           P.frac_c, P.chi_scale),
                                       tau, P.delta);
 }
 
+template <bool SPLIT = false>
 __device__ __forceinline__ bool m3_screen_ok(const float (&m0)[27], const float (&m1)[27], float tau,
                                              const ScanParams &P)
 {
     const float sum = screen_sum_fn<27>([&](int x, float &fc, float &ft) __attribute__((always_inline)) {
         fc = m0[x];
-        ft = m1[x] - m0[x];
+        ft = SPLIT ? m1[x] : m1[x] - m0[x];
     });
     return fmaf(sum, P.inv_n * 0.69314718f, P.hy) >= tau - P.delta;
 }
@@ -1981,6 +1987,7 @@ __device__ __forceinline__ uint64_t m3_key(const ScanParams &P, int n, int a, in
 }
 
 // Exact MI and push of the lanes that need it (all lanes call).
+template <bool SPLIT = false>
 __device__ __forceinline__ void m3_exact_push(bool need, const float (&m0)[27], const float (&m1)[27],
                                               const ScanParams &P, TopState *st, int n, int a, int b, int c,
                                               float tau, uint64_t tau_combo)
@@ -1989,7 +1996,7 @@ __device__ __forceinline__ void m3_exact_push(bool need, const float (&m0)[27], 
         need,
         [&](int x, uint32_t &n0, uint32_t &n1) __attribute__((always_inline)) {
             n0 = (uint32_t)m0[x];
-            n1 = (uint32_t)(m1[x] - m0[x]);
+            n1 = (uint32_t)(SPLIT ? m1[x] : m1[x] - m0[x]);
         },
         [&] { return m3_key(P, n, a, b, c); }, tau, tau_combo, P, st);
 }
@@ -2092,7 +2099,8 @@ __device__ __forceinline__ uint32_t m3_valid(const ScanParams &P, const M3Lane &
 // One workgroup's work item: first SNP a, tile u (see k_mfma3); returns at
 // once for items outside the triangle.  Every wave of the workgroup calls it
 // with the same arguments.  R: stages of the LDS ring (R - 1 in flight).
-// BIG: counts above 16 bits (not counts16; 2: find out at run time).
+// BIG: counts above 16 bits (not counts16; 2: find out at run time; 3: also sums
+// of both classes above FP32's exact integers, not pair_sums).
 template <int R, int BIG>
 __device__ __forceinline__ void mfma3_tile(const DevData &D, const ScanParams &P, TopState *st, const Fp4Image &F,
                                            int a, int64_t u, int T, int8_t (*lds)[kM3Stage])
@@ -2251,14 +2259,15 @@ __device__ __forceinline__ void mfma3_tile(const DevData &D, const ScanParams &P
     // bb, rows b = b0 + wb*32 + 16 bb + 4(lane/16) + j, j < 4
     const float tau = st->tau;
     const uint64_t tau_combo = st->tau_combo;
-    const M3Lane L = m3_lane(D, P, a, c0 + wc * 16 + rr);
+    constexpr bool SPLIT = BIG == 3;
+    const M3Lane L = m3_lane<SPLIT>(D, P, a, c0 + wc * 16 + rr);
     const uint32_t ok = m3_valid<8>(P, L, a, b0 + wb * 32);
     const int q4 = 4 * (lane >> 4), bw = b0 + wb * 32;
     // the wave's quarter of the workgroup's LDS (kM3Lds bytes): nothing reads
     // the ring any more
     int8_t *const mine = (int8_t *)lds + w * (kM3Lds / 4);
-    const bool big = BIG == 1 || (BIG == 2 && !counts16(D));
-    if (BIG != 1 && !big) {
+    const bool big = (BIG & 1) || (BIG == 2 && !counts16(D));
+    if (!(BIG & 1) && !big) {
         // two passes: the bound of the eight instances (bb, j), every
         // accumulator index a constant; then the marked ones
         M3List l;
@@ -2317,15 +2326,17 @@ __device__ __forceinline__ void mfma3_tile(const DevData &D, const ScanParams &P
             for (int j = 0; j < 4; ++j) {
                 const int b = bw + 16 * bb + q4 + j;
                 float m0[27], m1[27];
-                m3_cells(
+                m3_cells<SPLIT>(
                     D, L, b, (const float4 *)P.pair + 2 * pair_rank(b, L.c, D.n),
                     [&](int kk, int x, int y, int z) __attribute__((always_inline)) {
                         const int e = j * 16 + (x * 2 + y) * 2 + z;
+                        if (SPLIT) return cnt[(e + 8 * kk) * 64];
                         return kk ? cnt[e * 64] + cnt[(e + 8) * 64] : cnt[e * 64];
                     },
                     m0, m1);
-                const bool need = (ok >> (4 * bb + j) & 1) && m3_bound_ok(m0, m1, tau, P) && m3_screen_ok(m0, m1, tau, P);
-                m3_exact_push(need, m0, m1, P, st, D.n, a, b, L.c, tau, tau_combo);
+                const bool need = (ok >> (4 * bb + j) & 1) && m3_bound_ok<SPLIT>(m0, m1, tau, P) &&
+                                  m3_screen_ok<SPLIT>(m0, m1, tau, P);
+                m3_exact_push<SPLIT>(need, m0, m1, P, st, D.n, a, b, L.c, tau, tau_combo);
             }
         });
     }
@@ -3650,8 +3661,10 @@ hipError_t launch_mfma3(const DevData &D, const ScanParams &P, TopState *st, con
         return hipSuccess;
     }
     const dim3 grid((unsigned)(tiles8 * na * 8)), block(kBlock);
-    const bool big = !counts16(D);
-    if (ring == 3 && big) hipLaunchKernelGGL((k_mfma3<3, 1>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
+    const bool big = !counts16(D), split = !pair_sums(D);
+    if (ring == 3 && split) hipLaunchKernelGGL((k_mfma3<3, 3>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
+    else if (ring == kM3Ring && split) hipLaunchKernelGGL((k_mfma3<kM3Ring, 3>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
+    else if (ring == 3 && big) hipLaunchKernelGGL((k_mfma3<3, 1>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
     else if (ring == 3) hipLaunchKernelGGL((k_mfma3<3, 0>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
     else if (ring == kM3Ring && big) hipLaunchKernelGGL((k_mfma3<kM3Ring, 1>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
     else if (ring == kM3Ring) hipLaunchKernelGGL((k_mfma3<kM3Ring, 0>), grid, block, 0, s, D, P, st, F, a0, (int)na, T);
