@@ -1493,6 +1493,47 @@ class StaticWorkspace final : public Workspace {
     char *base_;
 };
 
+// What fiu_dataset_words needs for one call.
+struct WordsReader {
+    size_t block;   // SNPs per block, about 2 MB of words
+    hipStream_t stream = nullptr;
+    hipEvent_t done[2] = {nullptr, nullptr};
+    uint64_t *buf[2] = {nullptr, nullptr};
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // the thread's own, while it is changed
+
+    WordsReader(size_t snps, size_t per) : block(std::min(snps, std::max<size_t>(1, (size_t)(1u << 18) / per)))
+    {
+        check(hipThreadExchangeStreamCaptureMode(&mode), "capture mode");
+        try {
+            check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
+            for (int b = 0; b < (snps > block ? 2 : 1); ++b) {
+                check(hipEventCreateWithFlags(&done[b], hipEventDisableTiming), "hipEventCreate");
+                if (hipHostMalloc((void **)&buf[b], block * per * 8, hipHostMallocDefault) != hipSuccess) {
+                    buf[b] = nullptr;
+                    (void)hipGetLastError();
+                    fail(FIU_ERR_NOMEM, "host allocation failed");
+                }
+            }
+        } catch (...) {
+            release();
+            throw;
+        }
+    }
+    WordsReader(const WordsReader &) = delete;
+    WordsReader &operator=(const WordsReader &) = delete;
+    ~WordsReader() { release(); }
+    void release()
+    {
+        if (stream) (void)hipStreamSynchronize(stream);
+        for (int b = 0; b < 2; ++b) {
+            if (buf[b]) (void)hipHostFree(buf[b]);
+            if (done[b]) (void)hipEventDestroy(done[b]);
+        }
+        if (stream) (void)hipStreamDestroy(stream);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
 }  // namespace
 
 namespace fiu {
@@ -1638,27 +1679,28 @@ fiu_status fiu_dataset_words(const fiu_dataset *ds, uint64_t *out)
     return guard([&] {
         if (!ds || !out) fail(FIU_ERR_INVALID, "NULL argument");
         // from the device image, a block of SNPs at a time through pinned
-        // memory the kernel writes (no device memory is needed)
+        // memory the kernel writes (no device memory is needed); two blocks, so
+        // that one is copied out while the next is written.  On a stream of the
+        // call's own: the image does not change, so the words wait for no search,
+        // and may be read while some stream of the process records a graph
         const size_t per = 3 * (ds->cw + ds->tw);
         if (!ds->snps || !per) return;
         check(hipSetDevice(ds->device), "hipSetDevice");
-        const size_t block = std::min(ds->snps, std::max<size_t>(1, (size_t)(1u << 20) / per));
-        struct Pinned {
-            uint64_t *p = nullptr;
-            ~Pinned()
-            {
-                if (p) (void)hipHostFree(p);
-            }
-        } buf;
-        if (hipHostMalloc((void **)&buf.p, block * per * 8, hipHostMallocDefault) != hipSuccess) {
-            (void)hipGetLastError();
-            fail(FIU_ERR_NOMEM, "host allocation failed");
-        }
-        for (size_t s0 = 0; s0 < ds->snps; s0 += block) {
-            const size_t count = std::min(block, ds->snps - s0);
-            check(launch_words(ds->dev, s0, count, ds->cw, ds->tw, buf.p, ds->stream), "words");
-            check(hipStreamSynchronize(ds->stream), "words sync");
-            std::memcpy(out + s0 * per, buf.p, count * per * 8);
+        WordsReader rd(ds->snps, per);
+        size_t at[2] = {0, 0}, count[2] = {0, 0}, next = 0;
+        auto fill = [&](int b) {
+            at[b] = next;
+            count[b] = std::min(rd.block, ds->snps - next);
+            next += count[b];
+            if (!count[b]) return;
+            check(launch_words(ds->dev, at[b], count[b], ds->cw, ds->tw, rd.buf[b], rd.stream), "words");
+            check(hipEventRecord(rd.done[b], rd.stream), "words event");
+        };
+        fill(0);
+        for (int b = 0; count[b]; b ^= 1) {
+            fill(b ^ 1);
+            check(hipEventSynchronize(rd.done[b]), "words sync");
+            std::memcpy(out + at[b] * per, rd.buf[b], count[b] * per * 8);
         }
     });
 }
