@@ -209,7 +209,7 @@ class Engine {
     hipStream_t prep_stream() const { return prep_; }
     // Plan constants of a job (kind, prefixes, unit shape); throws on
     // invalid or unsupported requests.
-    static void plan_job(Job *j);
+    void plan_job(Job *j);
 
   private:
     struct StepRec {
@@ -385,8 +385,8 @@ void Engine::plan_job(Job *j)
     const bool sampled = tables && combos >= (double)(1 << 16) && counts16(d->dev);
     auto sample = [&](bool matrix) {
         if (!sampled) return;
-        j->sample = plan_sample(order, n, j->step, j->offset, total_prefixes, j->prefixes, j->outputs, 1u << 16,
-                                UINT64_MAX, true, matrix);
+        j->sample = plan_sample(order, n, j->step, j->offset, total_prefixes, j->prefixes, j->outputs,
+                                cfg_.cand_cap, UINT64_MAX, true, matrix);
         j->seed = j->n_pref;
     };
     if (tuned_algo == FIU_ALGO_AUTO && tables && tuple_scan(d, order, j->step, j->prefixes)) {
@@ -1106,7 +1106,7 @@ void Server::ingest_main()
                     j->binom = d->binom.p;   // this job's own dataset, built for its order
                     j->staged = true;
                     std::vector<uint64_t>().swap(j->words);
-                    Engine::plan_job(j);
+                    eng_->plan_job(j);
                 }
             } else {
                 if (!j->ds) {
@@ -1119,7 +1119,7 @@ void Server::ingest_main()
                 if (j->order == 3 && j->ds->dev.uniform) (void)ensure_pair_table(j->ds, ingest_stream_);
                 prepare_fp4(j, ingest_stream_);
                 prepare_tuples(j, ingest_stream_);
-                Engine::plan_job(j);
+                eng_->plan_job(j);
             }
         } catch (const Failure &e) {
             ok = false;
@@ -1332,7 +1332,7 @@ fiu_status fiu_search_batch(fiu_scan *scans, size_t n, const fiu_batch_config *c
                 if (j->order == 3 && j->ds->dev.uniform) (void)ensure_pair_table(j->ds, eng.prep_stream());
                 prepare_fp4(j, eng.prep_stream());
                 prepare_tuples(j, eng.prep_stream());
-                Engine::plan_job(j);
+                eng.plan_job(j);
             } catch (const Failure &e) {
                 j->scan->status = e.status;
                 ++done;
