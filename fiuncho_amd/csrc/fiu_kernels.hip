@@ -1385,12 +1385,17 @@ __device__ __forceinline__ void mfma2_tile(const DevData &D, const ScanParams &P
         const int a = aw + 8 * (i >> 2) + (i & 3);
         ok |= (uint32_t)(b_ok && a < b) << i;
     }
-    if (P.step != 1 || P.offset != 0) {   // a share (wave-uniform)
+    if (P.offset != 0) {   // wave-uniform, as below
+        const int first = (int)std::min<int64_t>(P.offset, D.n);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) ok &= ~((uint32_t)(aw + 8 * (i >> 2) + (i & 3) < first) << i);
+        if (!__ballot(ok != 0)) return;
+    }
+    if (P.step != 1) {   // a share
 #pragma unroll 1
         for (uint32_t left = ok; left; left &= left - 1) {
             const int i = __builtin_ctz(left);
-            const int64_t rel = (int64_t)(aw + 8 * (i >> 2) + (i & 3)) - P.offset;
-            if (rel < 0 || (P.step != 1 && rel % P.step != 0)) ok &= ~(1u << i);
+            if (((int64_t)(aw + 8 * (i >> 2) + (i & 3)) - P.offset) % P.step != 0) ok &= ~(1u << i);
         }
     }
     if constexpr (FP4) {
