@@ -768,6 +768,7 @@ ThresholdSample plan_sample(int order, int n, int64_t step, int64_t offset, uint
     // combination; where that leaves too few prefixes to fill the device, the
     // distribution's last ones, which have the fewest last SNPs.
     if (matrix) S.step = std::max<int64_t>(S.step, 256);
+    else S.step = std::max<int64_t>(1, (int64_t)std::ceil(combos / std::max(want, 1.0)));   // never nearly all of it
     S.layered = n_pref / S.step >= 1024;
     if (!S.layered)
         S.prefixes = tail_prefixes(n, order - 1, (uint64_t)step, (uint64_t)offset, total_prefixes, n_pref,
