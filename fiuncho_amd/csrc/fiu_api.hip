@@ -848,7 +848,10 @@ TupleArgs tuple_args(const fiu_dataset *d, int order, bool all_cells)
 // Order 3, 5,000 SNPs x 4,000 samples: step 128 18.2 ms around a head, 19.4 by
 // popcount; step 1,024 11.8 and 4.2.  Order 4, 500 x 8,000, step 1,000: 9.0 and
 // 6.4; 240 x 16,000, step 64: 6.4 and 9.9.
-static bool dense_share(const fiu_dataset *d, int order, double step, double n_pref)
+// Without a starting threshold every combination of the first chunk goes to the
+// FP64 MI, which two waves per SIMD hide badly: 800 x 6,000, step 8, 10.3 ms
+// around a head and 8.3 by popcount, 1,500 x 16,000 50 and 65.
+static bool dense_share(const fiu_dataset *d, int order, double step, double n_pref, bool sampled)
 {
     const double n = (double)d->snps, s = (double)d->cases + (double)d->ctrls;
     const double width = (n - order + 1) / order, combos = n_pref * width;   // columns per prefix, on average
@@ -863,7 +866,8 @@ static bool dense_share(const fiu_dataset *d, int order, double step, double n_p
     if (!d->dev.uniform)
         return combos * (s + 100) / 1.5e7 + 0.5 * chain >= (width / 32 + 0.5) * blocks * (0.024 + 6.3e-6 * s);
     return combos * (s + 750) / 4.5e7 + 0.7 * chain >=
-           (width / 64 + 0.5) * (tiles * (0.045 + 5.8e-6 * s) + blocks * (0.012 + 1.4e-6 * s));
+           (width / 64 + 0.5) * (tiles * (0.045 + 5.8e-6 * s) + blocks * (0.012 + 1.4e-6 * s)) +
+               (sampled ? 0.0 : 1000.0 + 8e-5 * combos);
 }
 
 // Its tables, launches and half-empty tiles cost a few tenths of a
@@ -874,12 +878,12 @@ static bool dense_share(const fiu_dataset *d, int order, double step, double n_p
 // (1.6e8) 219 and 215, on 100 x 4,000 (6.5e8) 171 and 245; order 4 on
 // 40 x 4,000 (3.7e8) 309 and 480.  The first search also builds the tables
 // (order 4 on 100 x 4,000: 0.3 ms), hence one line above all of these.
-bool tuple_scan(const fiu_dataset *d, int order, int64_t step, int64_t n_pref)
+bool tuple_scan(const fiu_dataset *d, int order, int64_t step, int64_t n_pref, bool sampled)
 {
     const double n = (double)d->snps, combos = (double)n_pref * (n - order + 1) / order;
     const bool fits = !d->dev.uniform ? order <= 3 : order == 4 || (order <= 3 && step > 1);
     return fits && counts16(d->dev) && n >= 48 && combos * ((double)d->cases + (double)d->ctrls) >= 2e9 &&
-           (step == 1 || order == 2 || dense_share(d, order, (double)step, (double)n_pref));
+           (step == 1 || order == 2 || dense_share(d, order, (double)step, (double)n_pref, sampled));
 }
 
 }  // namespace fiu
@@ -1148,7 +1152,9 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     const int instead = !d->dev.uniform ? FIU_ALGO_DIRECT : order == 2 ? FIU_ALGO_MFMA : FIU_ALGO_MARGINAL;
     const bool named = (variant != 0 && valid_variant(instead, order, variant)) ||
                        (instead == FIU_ALGO_MFMA && cfg && (cfg->flags & FIU_FLAG_MFMA_INT8));
-    const bool tup = algo_req == FIU_ALGO_AUTO && !named && tuple_scan(d, order, step, (int64_t)n_pref) &&
+    const bool tup = algo_req == FIU_ALGO_AUTO && !named &&
+                     tuple_scan(d, order, step, (int64_t)n_pref,
+                                !(cfg && (cfg->flags & FIU_FLAG_NO_THRESHOLD_SAMPLE))) &&
                      ws.tuples(d, order - 1, tup_all, s);
     if (algo_req != FIU_ALGO_DIRECT && d->dev.uniform && order >= 4 && order <= kMaxKmOrder)
         algo = FIU_ALGO_MARGINAL;

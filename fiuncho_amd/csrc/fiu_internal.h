@@ -294,8 +294,9 @@ Fp4Image tuple_image(const fiu_dataset *d, bool all_cells);
 constexpr int32_t kTupleFill = 16384;
 // Whether a scan around a head is the faster one for an AUTO search of these
 // n_pref prefixes; its units (heads, or at order 2 blocks of b's); its
-// arguments once ensure_tuple_tables / ensure_tuple_image succeeded.
-bool tuple_scan(const fiu_dataset *d, int order, int64_t step, int64_t n_pref);
+// arguments once ensure_tuple_tables / ensure_tuple_image succeeded.  `sampled`:
+// the search starts from a sampled threshold.
+bool tuple_scan(const fiu_dataset *d, int order, int64_t step, int64_t n_pref, bool sampled = true);
 int64_t tuple_units(int order, bool all_cells, uint64_t n, int64_t n_pref, bool small = false);
 TupleArgs tuple_args(const fiu_dataset *d, int order, bool all_cells);
 

@@ -120,3 +120,17 @@ def test_sparse_shares_stay_with_the_popcount_scan(order, snps, samples, step, m
     assert (stats.launches != explicit.launches) == head
     assert same(got, want)
     d.close()
+
+
+def test_unsampled_share_stays_with_the_popcount_scan():
+    # 8.3 ms by popcount, 10.3 around a head, whose exact MI it floods
+    print("case: order 3 800x6000 share of 8, no sample", flush=True)
+    d = fa.Dataset.synth(fa.synth_spec(800, 3000, 3000, seed=66))
+    dist = fa.Distribution(800, 2, 8, 3)
+    conf = {"chunk_combos": 25000, "sample_threshold": False}   # 1.9 heads
+    want, explicit = run(d, 3, dist, 50, algorithm=MARGINAL, **conf)
+    got, stats = run(d, 3, dist, 50, **conf)
+    auto, sampled = run(d, 3, dist, 50, chunk_combos=25000)
+    assert stats.launches == explicit.launches != sampled.launches
+    assert same(got, want) and same(auto, want)
+    d.close()
