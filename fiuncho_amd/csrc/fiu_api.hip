@@ -517,14 +517,18 @@ bool ensure_pair_table(fiu_dataset *d, hipStream_t s)
         if (bytes + (64ull << 20) > free_b) return false;
     }
     if (!d->pair.try_alloc(pair_words(n))) return false;
-    ScanParams P{};
-    P.j0 = 0;
-    P.j1 = (int64_t)n;
-    P.step = 1;
-    P.offset = 0;
-    P.total_prefixes = n;
-    P.binom = binom;
-    check(launch_pair_table(d->dev, P, pair_table(d), s), "pair table launch");
+    if (d->tup_ready >= 2) {
+        check(launch_pair_from_counts(d->tup[2].p, n * (n - 1) / 2, pair_table(d), s), "pair table launch");
+    } else {
+        ScanParams P{};
+        P.j0 = 0;
+        P.j1 = (int64_t)n;
+        P.step = 1;
+        P.offset = 0;
+        P.total_prefixes = n;
+        P.binom = binom;
+        check(launch_pair_table(d->dev, P, pair_table(d), s), "pair table launch");
+    }
     check(hipStreamSynchronize(s), "pair table sync");
     d->pair_ready = true;
     return true;

@@ -19,6 +19,8 @@ hipError_t launch_tau_from_hist(const uint32_t *hist, uint32_t N, float delta, T
 // A search's start: state reset, sampling histogram (when set) cleared.
 hipError_t launch_search_begin(TopState *st, uint32_t *hist, hipStream_t s);
 hipError_t launch_pair_table(const DevData &D, const ScanParams &P, uint32_t *pair_out, hipStream_t s);
+// The same from the tables of two SNPs' counts (TupleTables t[2]).
+hipError_t launch_pair_from_counts(const uint32_t *t2, uint64_t pairs, uint32_t *pair_out, hipStream_t s);
 // Order 2 on the matrix cores: the pair triangle of T x T 64-SNP tiles is cut
 // into super-blocks of 8 x 8 tiles; a launch scores super-blocks [s0, s1)
 // into the top-N state, with fp4 (e2m1) operands from the dataset's fp4 image

@@ -83,13 +83,19 @@ def test_options_that_name_a_kernel_keep_it_on_shares(order, snps, conf):
     d.close()
 
 
-def test_static_search_of_a_share_has_the_pair_table_of_an_earlier_search():
-    print("case: static share", flush=True)
-    d = fa.Dataset.synth(fa.synth_spec(200, 4700, 4700, seed=63))
-    dist = fa.Distribution(200, 2, 3, 1)
+@pytest.mark.parametrize("snps,cases,ctrls", [(200, 4700, 4700), (193, 65535, 300)])
+def test_static_search_of_a_share_has_the_pair_table_of_an_earlier_search(snps, cases, ctrls):
+    print(f"case: static share {snps}x{cases}+{ctrls}", flush=True)
+    d = fa.Dataset.synth(fa.synth_spec(snps, cases, ctrls, seed=63))
+    dist = fa.Distribution(snps, 2, 3, 1)
     want = fa.GpuSearch().run_arrays(d, 3, dist, 40)
     got = run_static(d, 3, dist, 40)
     assert got[2].algorithm == MARGINAL and same(got, want)
+    # that table, made of the share's count tables, serves the other kernels
+    whole = fa.Distribution(snps, 2)
+    direct = fa.GpuSearch(algorithm=DIRECT).run_arrays(d, 3, whole, 300)
+    for algorithm in (MARGINAL, MFMA):
+        assert same(fa.GpuSearch(algorithm=algorithm).run_arrays(d, 3, whole, 300), direct)
     d.close()
 
 
