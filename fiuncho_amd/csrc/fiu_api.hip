@@ -147,8 +147,8 @@ void finish_upload(fiu_dataset *d, const uint64_t *words)
     uint32_t fl[4];
     check(hipMemcpyAsync(fl, d->flags.p, sizeof(fl), hipMemcpyDeviceToHost, d->stream), "flags");
     check(hipStreamSynchronize(d->stream), "singles sync");
-    D.uniform = (n > 0 && fl[0] == 0) ? 1 : 0;
-    D.packs = !(fl[0] & 2) && fl[3] < (1u << 16);
+    D.uniform = (n > 0 && !(fl[0] & 1)) ? 1 : 0;
+    D.packs = !(fl[0] & 2);
     D.total[0] = fl[1];
     D.total[1] = fl[2];
 }

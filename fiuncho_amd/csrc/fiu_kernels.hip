@@ -3302,9 +3302,9 @@ __global__ void k_transpose(const uint64_t *__restrict__ src, uint4 *__restrict_
 __global__ void k_singles(const uint4 *__restrict__ bits, DevData D, uint32_t *singles, uint32_t *flags)
 {
     // one thread per (SNP, class): popcount of each row, disjointness of the
-    // rows and equality of their union with the union of SNP 0; flags[0] bit 0
-    // where either fails, bit 1 where the first does, flags[3] the most bits of
-    // a SNP's rows in a class
+    // rows and equality of their union with the union of SNP 0.  flags[0]: bit 0
+    // where either fails, bit 1 where the first does or a SNP's rows of a class
+    // hold 2^16 bits or more
     const int id = blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= D.n_pad * 2) return;
     const int s = id >> 1, cls = id & 1;
@@ -3330,8 +3330,8 @@ __global__ void k_singles(const uint4 *__restrict__ bits, DevData D, uint32_t *s
     singles[(s * 2 + cls) * 3 + 0] = cnt[0];
     singles[(s * 2 + cls) * 3 + 1] = cnt[1];
     singles[(s * 2 + cls) * 3 + 2] = cnt[2];
-    if (s < D.n && (twice | other)) atomicOr(&flags[0], twice ? 3u : 1u);
-    if (s < D.n) atomicMax(&flags[3], cnt[0] + cnt[1] + cnt[2]);
+    const uint32_t flag = (twice | other ? 1u : 0u) | (twice || cnt[0] + cnt[1] + cnt[2] >= (1u << 16) ? 2u : 0u);
+    if (s < D.n && flag) atomicOr(&flags[0], flag);
     if (s == 0) flags[1 + cls] = ucnt;
 }
 
