@@ -1148,8 +1148,8 @@ void search(fiu_dataset *d, Workspace &ws, int order, int32_t step, int32_t offs
     // too) and, every cell counted, orders 2 and 3 on datasets with uncalled
     // genotypes.  Measured against the popcount scans: order 4, 240 x 16,000,
     // 22 ms against 478; share (8, 3) of order 3, 2,500 x 16,000, 26 ms
-    // against 110; with 1 % uncalled, order 3 on 601 x 6,007 3.9 ms against
-    // 17.5 and order 2 on 4,001 x 8,999 0.87 ms against 3.2
+    // against 109; with 1 % uncalled, order 3 on 601 x 6,007 3.5 ms against
+    // 17.3 and order 2 on 4,001 x 8,999 0.67 ms against 3.0
     const bool tup_all = !d->dev.uniform;
     // (not where the caller names a kernel, by its operand format or by a variant
     // of the algorithm that would run instead)

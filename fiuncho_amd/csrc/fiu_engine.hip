@@ -370,7 +370,7 @@ void Engine::plan_job(Job *j)
     const bool has_te = tuned(order, d->snps, (uint64_t)d->cases + d->ctrls, te);
     const int tuned_algo = has_te ? te.algorithm : FIU_ALGO_AUTO;
     const double unit_instr = has_te && te.batch_unit ? 40000.0 * std::ldexp(1.0, (int)te.batch_unit - 3) : 40000.0;
-    // a scan around a head where the single search takes one and prepare_scan
+    // a scan around a head where the single search takes one and prepare_tuples
     // found room for its tables: launches of its own, a whole range each
     // (order 4 on 160 SNPs x 5,000 samples: the popcount kind's persistent
     // launches took 3.5 ms of a 17 ms batch)
@@ -404,13 +404,14 @@ void Engine::plan_job(Job *j)
         (order == 2 || (order == 3 && d->pair_ready && j->step == 1 && mfma3_dataset(d)))) {
         j->kind = order == 2 ? kKindMfma2 : kKindMfma3;
         // the tile: a tuning entry's batch tile (batch_unit 1 = the 64 x 32 /
-        // 64 x 64 tiles, 2 = the wide ones), else the sizes where the single
-        // search takes the wide tiles (their counts wait as 16-bit pairs:
-        // classes below 2^16 samples).  The entry's variant, timed on single
-        // searches, is not used: on the 64-dataset batch, wide tiles for
-        // the order-3 datasets of 512-2,048 SNPs that the single-search
-        // tuner puts on them made the batch 9 % slower (finer units balance
-        // the persistent kernel better)
+        // 64 x 64 tiles, 2 = the wide ones), else by size (wide tiles' counts
+        // wait as 16-bit pairs: counts16).  `wide` is for ranges in the
+        // persistent kernel, which wants finer units than a launch of its own:
+        // on the 64-dataset batch, wide tiles for its order-3 datasets of
+        // 512-2,048 SNPs made it 9 % slower.  `tile` is for those launches and
+        // follows the single search's sizes (order 3 from 768 SNPs, order 2
+        // from 8,192 and 16,384 with 8,192 samples).  The entry's variant,
+        // timed on single searches, is not used
         const uint64_t samples = (uint64_t)d->cases + d->ctrls;
         bool wide = samples >= 8192 && (uint64_t)n >= (order == 3 ? 2048u : 16384u);
         if (tuned_algo == FIU_ALGO_MFMA && te.batch_unit) wide = te.batch_unit == 2;

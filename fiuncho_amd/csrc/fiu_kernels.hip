@@ -236,7 +236,7 @@ k_scan_direct(const DevData D, const ScanParams P, TopState *st)
 // the cell-order value is below 3^k x 2^-52 x sum |p ln p| < 1e-10 nats, so
 // a combination whose value plus 1e-9 rounds below the current threshold
 // would be rejected by its exact value as well.  The others get the exact
-// value in cell order (mi_exact's chain: wave 0 computes the terms of 64
+// value in cell order (mi_exact_part_fn's chain: wave 0 computes the terms of 64
 // cells at a time and every lane runs the chain over them).
 template <int K, bool HIST>
 __global__ void __launch_bounds__(kBlock) k_scan_any(const DevData D, const ScanParams P, TopState *st)

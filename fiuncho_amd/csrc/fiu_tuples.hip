@@ -33,12 +33,13 @@ enum TupleMode { kScore = 0, kSample = 1, kTable = 2, kSampleSmall = 3 };
 constexpr bool samples(int mode) { return mode == kSample || mode == kSampleSmall; }
 
 // Shape of one kernel: W waves, NB blocks of 16 b rows against 16 W c columns,
-// wave w taking columns c0 + 16 w ..; NB is the most whose accumulators (4
-// registers per product and block) stay at 144 or below, so that two waves
-// per SIMD fit (order 2 with uncalled genotypes, 9 products: NB = 4 560 us on
-// 4,001 x 8,999, NB = 2 655, whose 18 KB per 72 products outran the loads).  Two waves per workgroup where the column range of a head is
-// short (order 4 runs on a few hundred SNPs) or the staged c rows outweigh
-// the shared b rows (all cells); four where the b rows do.
+// wave w taking columns c0 + 16 w ..; NB is a power of two, 4 at most, whose
+// accumulators (4 registers per product and block) stay at 144 or below, so
+// that two waves per SIMD fit (order 2 with uncalled genotypes, 9 products:
+// NB = 4 560 us on 4,001 x 8,999, NB = 2 655, whose 18 KB per 72 products outran
+// the loads).  Two waves per workgroup where the column range of a head is short
+// (order 4 runs on a few hundred SNPs) or the staged c rows outweigh the shared
+// b rows (all cells); four where the b rows do.
 template <int K, bool ALL, int MODE = kScore> struct Tup {
     static constexpr int G = ALL ? 3 : 2;            // genotype rows per SNP
     static constexpr int H = K - 2;                  // head SNPs
@@ -561,40 +562,41 @@ __device__ __forceinline__ void tuple_tile(const DevData &D, const ScanParams &P
                 uint32_t m[Z::cells];
                 cells_of(x[u], m);
                 const float bound = packed_bound<!ALL>(m, P, fixed);
-                marks |= (uint32_t)(bound_passes(bound, tau, P.delta) & valid_at(b_at(i + u))) << u;
+                const bool pass = bound_passes(bound, tau, P.delta), valid = valid_at(b_at(i + u));
+                marks |= ((uint32_t)pass & (uint32_t)valid) << u;   // no branch
             }
             pend |= marks << i;
         }
     } else {
-    Loaded<K, ALL> nxt;
-    load(4 * lo, cur);
+        Loaded<K, ALL> nxt;
+        load(4 * lo, cur);
 #pragma unroll 1
-    for (int i = 4 * lo; i < i1; ++i) {
-        load(std::min(i + 1, i1 - 1), nxt);
-        const int64_t bi = b_at(i);
-        const bool valid = valid_at(bi);
-        if constexpr (MODE == kTable) {
-            if (valid) {
-                const uint64_t stride = (uint64_t)n + 1;
-                int64_t r = (int64_t)P.binom[(uint64_t)K * stride + n] - 1;
+        for (int i = 4 * lo; i < i1; ++i) {
+            load(std::min(i + 1, i1 - 1), nxt);
+            const int64_t bi = b_at(i);
+            const bool valid = valid_at(bi);
+            if constexpr (MODE == kTable) {
+                if (valid) {
+                    const uint64_t stride = (uint64_t)n + 1;
+                    int64_t r = (int64_t)P.binom[(uint64_t)K * stride + n] - 1;
 #pragma unroll
-                for (int q = 0; q < H; ++q) r -= (int64_t)P.binom[(uint64_t)(K - q) * stride + (n - 1 - hd.s[q])];
-                const int64_t v = n - 1 - bi;
-                r -= v * (v - 1) / 2 + (n - 1 - c);
-                uint4 *to = (uint4 *)(A.out + (r << K));
-                uint32_t x[Z::dots];
-                words(cur, x);
+                    for (int q = 0; q < H; ++q) r -= (int64_t)P.binom[(uint64_t)(K - q) * stride + (n - 1 - hd.s[q])];
+                    const int64_t v = n - 1 - bi;
+                    r -= v * (v - 1) / 2 + (n - 1 - c);
+                    uint4 *to = (uint4 *)(A.out + (r << K));
+                    uint32_t x[Z::dots];
+                    words(cur, x);
 #pragma unroll
-                for (int e = 0; e < Z::dots; e += 4) to[e / 4] = make_uint4(x[e], x[e + 1], x[e + 2], x[e + 3]);
+                    for (int e = 0; e < Z::dots; e += 4) to[e / 4] = make_uint4(x[e], x[e + 1], x[e + 2], x[e + 3]);
+                }
+            } else {
+                uint32_t m[Z::cells];
+                cells_of(cur, m);
+                const float ms = packed_screen<Z::cells>(m, P);
+                if (valid) atomicAdd(&lds_hist[hist_bin(ms)], 1u);
             }
-        } else {
-            uint32_t m[Z::cells];
-            cells_of(cur, m);
-            const float ms = packed_screen<Z::cells>(m, P);
-            if (valid) atomicAdd(&lds_hist[hist_bin(ms)], 1u);
+            cur = nxt;
         }
-        cur = nxt;
-    }
     }
     if constexpr (MODE == kScore) {
         // one marked combination per lane and round: screen, exact MI, push

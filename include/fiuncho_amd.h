@@ -106,7 +106,9 @@ fiu_status fiu_dataset_info(const fiu_dataset *ds, size_t *snps,
                             size_t *cases_words, size_t *ctrls_words,
                             size_t *device_bytes);
 
-/* Copy the host-layout words back (3*(cases_words+ctrls_words)*snps words). */
+/* Copy the host-layout words back (3*(cases_words+ctrls_words)*snps words)
+ * from the device image, on a stream of the call's own: it waits for no
+ * search, and may be called while a stream of the process records a graph. */
 fiu_status fiu_dataset_words(const fiu_dataset *ds, uint64_t *out);
 
 fiu_status fiu_dataset_destroy(fiu_dataset *ds);
@@ -116,7 +118,16 @@ fiu_status fiu_dataset_destroy(fiu_dataset *ds);
 /* ------------------------------------------------------------------------ */
 
 typedef enum {
-    FIU_ALGO_AUTO = 0,     /* fastest exact path the dataset allows */
+    FIU_ALGO_AUTO = 0,     /* fastest exact path the dataset allows: one of
+                              those below, or, from about 2e9 combinations x
+                              samples on, a scan around a head of order - 2
+                              SNPs on the matrix cores (order 4; shares of
+                              orders 2 and 3 that are dense enough; orders 2
+                              and 3 where SNPs cover different samples).  Such
+                              a scan counts the cells of FIU_ALGO_MARGINAL
+                              (order 2: FIU_ALGO_MFMA) or, with different
+                              samples, of FIU_ALGO_DIRECT, and reports that
+                              one */
     FIU_ALGO_DIRECT = 1,   /* AND+popcount of all 3^k cells (the reference's);
                               every order, any dataset (the only algorithm
                               at orders 7-12) */
@@ -150,7 +161,9 @@ typedef struct {
     uint32_t flags;          /* FIU_FLAG_* */
     void *stream;            /* hipStream_t to run on, NULL = library stream */
     int32_t variant;         /* kernel variant of the algorithm, 0 = the
-                                tuned or default one (fiu_tune_entry) */
+                                tuned or default one (fiu_tune_entry).  With
+                                AUTO: of the algorithm it runs; a share then
+                                keeps that algorithm's kernel */
     int32_t reserved;
 } fiu_config;
 
@@ -163,7 +176,9 @@ typedef struct {
     uint64_t redo_chunks;    /* chunks re-scanned after a candidate overflow */
     double scan_ms;          /* device time of the scan launches (HIP events) */
     double total_ms;         /* wall time of the call */
-    int32_t algorithm;       /* algorithm actually used */
+    int32_t algorithm;       /* algorithm used: which cells were counted (a
+                                scan around a head reports as fiu_algorithm
+                                says) */
     int32_t variant;         /* its kernel variant (fiu_tune_entry) */
 } fiu_search_stats;
 
@@ -178,7 +193,12 @@ typedef struct {
  * out_combos receives order ints per result (ascending SNP indices), out_mi
  * the MI as float, *out_count the number of results (<= outputs).
  * Replaces: Search::run (Search.h:40-43) / ThreadedSearch::run
- * (ThreadedSearch.h:207-246).  `cfg` and `stats` may be NULL. */
+ * (ThreadedSearch.h:207-246).  `cfg` and `stats` may be NULL.
+ * Searches keep what they derive from a dataset with it, until it is
+ * destroyed: the fp4 images, the order-3 pair table (32 bytes a pair) and the
+ * counts of 1 to order - 1 SNPs (2^m words per m-combination: 16 bytes a pair,
+ * 32 a triple; never more than a quarter of the device memory free at the
+ * time).  Where one finds no room the search runs the kernels without it. */
 fiu_status fiu_search(const fiu_dataset *ds, uint16_t order,
                       int32_t dist_step, int32_t dist_offset,
                       uint32_t outputs, const fiu_config *cfg,
@@ -188,8 +208,9 @@ fiu_status fiu_search(const fiu_dataset *ds, uint16_t order,
 /* Search that allocates nothing.
  * No counterpart in the reference: for callers that cannot allocate device
  * memory -- code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc.  Same arguments, results, errors and algorithm choice as
- * fiu_search; the search runs in one fixed block of device memory per GPU
+ * forbid hipMalloc.  Same arguments, results and errors as fiu_search, and the
+ * same algorithm choice but for the scans around a head, in whose place the
+ * kernels of the algorithm they report run; the search runs in one fixed block of device memory per GPU
  * (fiu_search_static_bytes(), under 9 MiB), which the library holds until
  * the process ends, and calls no hipMalloc / hipFree (and no host heap
  * allocation).  Limits, refused with FIU_ERR_UNSUPPORTED: candidate_cap <=
@@ -293,24 +314,27 @@ fiu_status fiu_write_results(const char *path, const int32_t *combos,
  *                      only, 8;
  *   FIU_ALGO_MFMA, order 3: tile and LDS staging depth: 3, 4 = 64 x 32
  *                      (b, c) per workgroup with 3 or 4 stages, 5, 6 =
- *                      64 x 64 with 3 or 4 stages (default: 6 from 2,048
- *                      SNPs and 8,192 samples on, else 4; 5 and 6 fall back
- *                      to 4 when a class holds 2^16 samples or more);
+ *                      64 x 64 with 3 or 4 stages (default: 6 from 768
+ *                      SNPs on, else 4; 5 and 6 fall back to 4 when a class
+ *                      holds 2^16 samples or more);
  *   FIU_ALGO_MFMA, order 2: 1 = int8 operands, 2 = fp4 operands, 64 x 64
  *                      pairs per workgroup, 3 = fp4 operands, 64 x 128 pairs
  *                      per workgroup, 4 = fp4 operands, 128 x 128 pairs per
  *                      workgroup (3 and 4: 64 x 64 when a class holds 2^16
- *                      samples or more); default: 4 from 16,384 SNPs and
- *                      8,192 samples on, else 2.
+ *                      samples or more); default, from 8,192 samples on: 4
+ *                      from 16,384 SNPs, 3 from 8,192; else 2.
  * The table is written by an autotuner that times the candidates on the
- * device (fiuncho_amd.tune); it is process-wide and starts empty.  Batched
+ * device (fiuncho_amd.tune); it is process-wide and starts empty.  An entry
+ * fixes its class's algorithm, so that AUTO's scans around a head are not
+ * taken there: an order-4 class is best left without one.  Batched
  * scans use its algorithm and its batch_unit.  For the popcount kinds
  * (orders 2-5 off the matrix cores) batch_unit is the work of one unit of the
  * persistent kernels, 0 = the default (about 40,000 wave instructions: that
  * many 64-SNP tiles of last SNPs per prefix group), k = 1..6 = the default
  * times 2^(k-3) (a quarter to 8 times).  For FIU_ALGO_MFMA entries it is the
- * batched tile: 0 = by size (64 x 64 / 64 x 128 from 2,048 / 16,384 SNPs and
- * 8,192 samples on, as the single search's default), 1 = 64 x 32 (order 3)
+ * batched tile: 0 = by size (in the persistent kernel 64 x 64 / 64 x 128 from
+ * 2,048 / 16,384 SNPs and 8,192 samples on; in launches of their own the
+ * single search's defaults), 1 = 64 x 32 (order 3)
  * / 64 x 64 (order 2), 2 = 64 x 64 / 64 x 128 (classes below 2^16 samples);
  * above 2 is FIU_ERR_INVALID.  The variant does not steer batched scans. */
 typedef struct {
@@ -334,11 +358,12 @@ fiu_status fiu_get_tuning(fiu_tune_entry *entries, size_t cap, size_t *n);
 /* ------------------------------------------------------------------------ */
 /* No counterpart in the reference, which runs one search per process
  * (MPIEngine.h:135-137).  Many searches over different datasets, sizes and
- * orders (2-5) advance together through batched device steps: persistent launches
- * over a slice of every active search (popcount kinds, orders 4-5, matrix-core
- * kinds for order 2 and whole order-3 scans), then one top-N merge per
- * search, replayed from a HIP graph.  Each search returns exactly what
- * fiu_search returns for it alone. */
+ * orders (2-5) advance together through batched device steps: launches of their
+ * own for scans around a head and large matrix-core ranges, persistent launches
+ * over a slice of every other active search (popcount kinds, orders 4-5,
+ * matrix-core kinds for order 2 and whole order-3 scans), then one top-N merge
+ * per search; the persistent launches and merges are replayed from a HIP graph.
+ * Each search returns exactly what fiu_search returns for it alone. */
 
 typedef struct {
     uint32_t struct_size;    /* sizeof(fiu_batch_config) */
@@ -372,7 +397,9 @@ typedef struct {
     uint64_t steps;          /* batched steps launched */
     uint64_t units;          /* work units claimed: wavefront units of the
                                 popcount kinds, workgroup units (tiles) of
-                                the matrix-core kinds */
+                                the matrix-core kinds, and of launches of
+                                their own the heads, first SNPs or
+                                super-blocks */
     uint64_t redo_ranges;    /* prefix ranges scanned again (candidate overflow) */
     double device_ms;        /* device time of the steps (HIP events) */
     double total_ms;         /* wall time of the call */
