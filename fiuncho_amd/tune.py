@@ -205,8 +205,9 @@ class BatchClass:
     algorithm: int = ALGO_MARGINAL
 
 
-# Orders 4 and 5, the batched scans that run on the popcount kinds, and
-# orders 2 and 3 at the sizes where the matrix cores' two tiles compete.
+# Orders 4 and 5, whose popcount kinds have a unit size (order 4 gets an entry
+# only where the scans around a head are not the faster choice), and orders 2 and
+# 3 at the sizes where the matrix cores' two tiles compete.
 DEFAULT_BATCH_CLASSES: List[BatchClass] = [
     BatchClass(4, 0, 512, 0, 8192, 200, 3000),
     BatchClass(4, 0, 512, 8192, INF, 160, 16000),
